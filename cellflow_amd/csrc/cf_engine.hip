@@ -834,16 +834,16 @@ struct Engine {
     ea.start = b.start[cur];
     ea.sims = b.sims;
     ea.wave_sim = b.wave_sim;
-    ea.ecand_d2 = b.ecand_d2;
-    ea.ecand_id = b.ecand_id;
     ea.estage = b.estage;
     ea.estride = edge_maxc_alloc;
     ea.ecount = b.fcount;
-    ea.P = P;
     ea.nwaves = nwaves;
     ea.edge_cap = cap;
+    bool near = true;
+    for (const SimDesc& d : hdesc)
+      near = near && d.edge_rx == 1 && d.edge_ry == 1 && d.edge_rz == 1;
     timed(ev, 0);
-    const hipError_t e0 = launch_edges(ea, st);
+    const hipError_t e0 = launch_edges(ea, near, st);
     arm_kernel_timer(nullptr, nullptr);
     HIPR(e0);
     TileSortArgs ta{};

@@ -184,12 +184,9 @@ struct EdgeArgs {
   const uint32_t* __restrict__ start;
   const SimDesc* __restrict__ sims;
   const uint32_t* __restrict__ wave_sim;
-  float* ecand_d2;      // [cap][P] by slot: scratch of the streaming selection
-  uint32_t* ecand_id;
   uint32_t* estage;     // kept partners: owner index o's rank r at o * estride + r
   uint32_t* ecount;     // kept partners per owner index: non-zero counts only (zero between
                         // passes: the edge tiles clear what they read)
-  long P;
   long estride;
   int nwaves;
   int edge_cap;
@@ -442,7 +439,8 @@ void arm_kernel_timer(hipEvent_t start, hipEvent_t stop);
 // host-side launchers (cf_kernels.hip)
 hipError_t launch_force(const ForceArgs& a, bool edges, int block, int variant, int reach,
                         int lanes, hipStream_t st);
-hipError_t launch_edges(const EdgeArgs& a, hipStream_t st);
+// near: every simulation's edge reach is one cell on every axis.
+hipError_t launch_edges(const EdgeArgs& a, bool near, hipStream_t st);
 hipError_t launch_tile_sort(const TileSortArgs& a, hipStream_t st);
 hipError_t launch_scan(const ScanPlan& p, hipStream_t st);
 hipError_t launch_fill(const SortArgs& a, hipStream_t st);

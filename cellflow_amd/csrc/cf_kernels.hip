@@ -1230,9 +1230,130 @@ __global__ void __launch_bounds__(256) k_force_grp(ForceArgs a) {
 // particles still advance together (split by position instead, a long list before the
 // split and one after it would run one after the other).  Group sums use DPP mirror
 // butterflies.
+//
+// k_force_ord (variant 0 at 16 lanes, the default tuning) is the same kernel in
+// k_force_grp's order of summation, so its results are those of k_force_grp<16> bit for
+// bit: 16 order lanes per particle (candidate c of the flattened rows 0..8 goes to order
+// lane c mod 16), reduced by halving the distance.  With G = 8 each lane stands for order
+// lanes 8 apart and keeps two sums.  A wave with more than kWalkFrom candidates walks the
+// runs from a table in the list's place, 16 lanes per particle: building a list costs
+// about as much as the pairs it saves once runs are long.
+// Bound: instruction issue (the same pairs in about half of k_force_grp's instructions).
+// Measured against k_force_grp<16> (uniform states at 12,500 per unit volume, us per
+// launch): 1k 10.1 -> 5.8, 20k 11.6 -> 7.1, 100k 35 -> 18.4, 100k with edges 46.5 -> 24,
+// the same after 300 steps 48.5 -> 32, 500k 142 -> 71; 1M clustered (238 neighbours) with
+// edges 1171 -> 640, without 485 -> 440; 20k of a preset (516 neighbours) 82 -> 77.
 
 constexpr int kWaveList = 640;  // candidate slots per wave
-constexpr int kListEdges = 24;  // LDS edge candidates per particle (more: streaming selection)
+constexpr int kListEdges = 24;  // LDS edge candidates per particle (more: the wave selects)
+
+// The proximity-graph partners of one owner with more candidates than its LDS list holds,
+// chosen by the whole wave: its lanes walk the owner's slot runs together and append the
+// qualifying candidates to a list of kSelCap entries (d^2, index); when it fills, it is cut
+// to the `cap` smallest indices (the reference keeps the first 2*maxC by index,
+// ParticleSimulation.cu:215), and from then on only smaller ones are appended.  So one pass
+// serves any number of candidates: a selection by one lane through global scratch took
+// milliseconds on states whose owners have hundreds (1M clustered with edges, 20 steps in:
+// the force pass 1649 -> 560 us; the standalone pass 1372 -> 260 us).
+constexpr int kSelCap = 192;  // at least 64 (one round of the lanes) above the largest cap
+static_assert(kSelCap - kWave >= kMaxEdgeCap, "a cut list has room for a round");
+
+struct WaveSel {
+  float2* buf;      // kSelCap entries of LDS: d^2, index bits
+  int n;            // entries held
+  uint32_t below;   // only indices below this can still be among the cap smallest
+};
+
+// Cuts the list to its `cap` smallest indices (it holds more).
+__device__ __forceinline__ void wave_sel_cut(WaveSel& s, int cap, int lane) {
+  constexpr int kPer = kSelCap / kWave;
+  wave_lds_sync();
+  float2 e[kPer];
+  uint32_t ix[kPer];
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const bool in = lane + u * kWave < s.n;
+    e[u] = in ? s.buf[lane + u * kWave] : make_float2(0.0f, 0.0f);
+    ix[u] = in ? __float_as_uint(e[u].y) : 0xFFFFFFFFu;
+  }
+  // the cap-th smallest index, bit by bit: the largest t with fewer than cap indices below it
+  uint32_t t = 0u;
+  for (int b = 31; b >= 0; --b) {
+    const uint32_t c = t | (1u << b);
+    int m = 0;
+#pragma unroll
+    for (int u = 0; u < kPer; ++u) m += __popcll(__ballot(ix[u] < c));
+    if (m < cap) t = c;
+  }
+  wave_lds_sync();
+  int n = 0;
+#pragma unroll
+  for (int u = 0; u < kPer; ++u) {
+    const unsigned long long m = __ballot(ix[u] <= t);
+    if (ix[u] <= t) s.buf[n + __popcll(m & ((1ull << lane) - 1ull))] = e[u];
+    n += __popcll(m);
+  }
+  s.n = n;
+  s.below = t;
+  wave_lds_sync();
+}
+
+// Walks `nruns` runs (first slot, length; CODED: the slot carries an image-shift code above
+// kCodeShift, and a shifted run holds no partner) of the owner `me` with index `myid`.
+// GEN: the grid is too small for shifted runs, so the pair must be its own nearest image.
+template <bool CODED>
+__device__ __forceinline__ void wave_sel_runs(WaveSel& s, const float4* __restrict__ pos,
+                                              const uint32_t* __restrict__ id,
+                                              const uint2* runs, int nruns, const float4& me,
+                                              uint32_t myid, const SimDesc& sd, bool gen, int cap,
+                                              int lane) {
+  for (int r = 0; r < nruns; ++r) {
+    const uint32_t first = __builtin_amdgcn_readfirstlane(runs[r].x);
+    const uint32_t len = __builtin_amdgcn_readfirstlane(runs[r].y);
+    if (CODED && !gen && (first >> kCodeShift) != 0u) continue;
+    const uint32_t q0 = CODED ? first & ((1u << kCodeShift) - 1u) : first;
+    for (uint32_t t0 = 0; t0 < len; t0 += (uint32_t)kWave) {
+      bool hit = false;
+      float d2 = 0.0f;
+      uint32_t jid = 0u;
+      if (t0 + (uint32_t)lane < len) {
+        const float4 pj = pos[q0 + t0 + lane];
+        jid = id[q0 + t0 + lane];
+        const float ux = pj.x - me.x, uy = pj.y - me.y, uz = pj.z - me.z;
+        d2 = fmaf(uz, uz, fmaf(uy, uy, ux * ux));
+        hit = __float_as_uint(pj.w) == __float_as_uint(me.w) && d2 < sd.edge_d2 &&
+              jid > myid && jid < s.below;
+        if (CODED && gen)
+          hit = hit && min_image(ux, sd.Lx) == ux && min_image(uy, sd.Ly) == uy &&
+                min_image(uz, sd.Lz) == uz;
+      }
+      const unsigned long long m = __ballot(hit);
+      if (m == 0ull) continue;
+      if (hit)
+        s.buf[s.n + __popcll(m & ((1ull << lane) - 1ull))] = make_float2(d2, __uint_as_float(jid));
+      s.n += __popcll(m);
+      if (s.n > kSelCap - kWave) wave_sel_cut(s, cap, lane);
+    }
+  }
+}
+
+// Ranks the cap smallest indices by (d^2, index) and writes the first maxc to the owner's
+// record; returns how many.
+__device__ __forceinline__ uint32_t wave_sel_finish(WaveSel& s, int cap, int maxc,
+                                                    uint32_t* __restrict__ rec, int lane) {
+  if (s.n > cap) wave_sel_cut(s, cap, lane);
+  wave_lds_sync();
+  const bool in = lane < s.n;
+  const float2 e = in ? s.buf[lane] : make_float2(0.0f, 0.0f);
+  int rank = 0;
+  for (int k = 0; k < s.n; ++k) {
+    const float2 f = s.buf[k];
+    rank += (f.x < e.x || (f.x == e.x && __float_as_uint(f.y) < __float_as_uint(e.y))) ? 1 : 0;
+  }
+  if (in && rank < maxc) rec[rank] = __float_as_uint(e.y);
+  wave_lds_sync();  // the list is reused for the next owner
+  return (uint32_t)min(s.n, maxc);
+}
 
 // Sum over aligned groups of G lanes (G in 4, 8, 16, 32), every lane gets its group's sum.
 template <int G>
@@ -1273,6 +1394,18 @@ __device__ __forceinline__ uint32_t group_excl_scan(uint32_t v, int g) {
   return x - v;
 }
 
+// Sum over aligned groups of G order lanes (8 or 16) by halving the distance, 8 (G = 16),
+// 4, 2, 1: k_force_grp's order.  Lanes 4-7 of each eight hold order lanes 7-4, so the half
+// mirror pairs order lanes 4 apart.
+template <int G>
+__device__ __forceinline__ float ordered_sum(float x) {
+  static_assert(G == 8 || G == 16, "");
+  if (G == 16) x = dpp_add<0x128>(x);  // row rotate by 8
+  x = dpp_add<0x141>(x);               // half mirror
+  x = dpp_add<0x4E>(x);                // quad_perm [2,3,0,1]
+  return dpp_add<0xB1>(x);             // quad_perm [1,0,3,2]
+}
+
 // ParticleSimulation.cu:136-161 for one particle: density factor, friction-Euler step and
 // wrap; the new state by pre-step slot p, the acceleration (when stored) and the new cell
 // (commit_cell).  cyo, czo: the pre-step cell's row and plane.
@@ -1307,14 +1440,17 @@ __device__ __forceinline__ void integrate_commit(const ForceArgs& a, const SimDe
 // wave 0 with one lane per particle, instead of once per wave with one lane of each group
 // active: each wave leaves its particles' sums in LDS, and after a block barrier wave 0
 // reloads their (cache-resident) state and finishes them.  Same arithmetic, same results.
-template <bool EDGES, int R, int G, bool TILE, bool CONS = false>
-// With the consolidated tail, the 27-cell stencil at G = 8 fits 7 waves per SIMD (72 VGPRs,
-// under 22.8 KB of LDS per block).  Without it the velocity stays live to the end and the
-// kernel needs a few more registers: held to 72 it spills, and a spilling kernel's scratch
-// allocation cuts its occupancy far below 7 waves (a 6x slower launch), so no hint there.
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R == 1 && G == 8 && CONS ? 7 : 1, 8)))
-k_force_list(ForceArgs a) {
+template <bool EDGES, int R, int G, bool TILE, bool CONS, int V = 0, bool HITS = false>
+__device__ __forceinline__ void force_list(const ForceArgs& a) {
   constexpr int kRows = (2 * R + 1) * (2 * R + 1);
+  constexpr int VL = V ? V : G;     // lanes of the summation order
+  constexpr int kSub = VL / G;      // of them each lane stands for (1 or 2)
+  // candidates of a wave from which it walks its runs instead of listing them (V): beyond
+  // one pass of the list at G = 16; at G = 8, where the walk re-reads each particle's state,
+  // beyond two (400k particles at 50,000 per unit volume: 144 us against 166 from 640; 2560
+  // is no different)
+  constexpr uint32_t kWalkFrom = G == 8 ? 1280u : 640u;
+  static_assert(kSub * G == VL && kSub <= 2, "one or two order lanes per lane");
   constexpr int kOwn = kWave / G;
   constexpr int kRpl = (kRows + G - 1) / G;  // stencil rows per lane
   // the pair table by field (kMaxTypes^2 words each), so the lanes of different owners,
@@ -1328,10 +1464,14 @@ k_force_list(ForceArgs a) {
   __shared__ float ptab[4 * kTT];
   // list entries: slot | image-shift code << kCodeShift (slots stay below 2^kCodeShift),
   // the wave's particles one after another
-  __shared__ uint32_t lslot[4][kWaveList];
-  __shared__ float2 el_d[EDGES ? 4 : 1][EDGES ? kOwn : 1][EDGES ? kListEdges : 1];
-  __shared__ uint32_t el_i[EDGES ? 4 : 1][EDGES ? kOwn : 1][EDGES ? kListEdges : 1];
+  __shared__ __align__(16) uint32_t lslot[4][kWaveList];
+  // edge candidates listed per particle; together at least the wave selection's list
+  constexpr int kLE = kSelCap / kOwn > kListEdges ? kSelCap / kOwn : kListEdges;
+  __shared__ float2 el_d[EDGES ? 4 : 1][EDGES ? kOwn : 1][EDGES ? kLE : 1];
+  __shared__ __align__(8) uint32_t el_i[EDGES ? 4 : 1][EDGES ? kOwn : 1][EDGES ? kLE : 1];
   __shared__ uint32_t el_n[4][kOwn];
+  __shared__ uint32_t hl[HITS ? 4 : 1][HITS ? kOwn : 1][HITS ? kPairList : 1];
+  __shared__ uint32_t hn[HITS ? 4 : 1][HITS ? kOwn : 1];
   __shared__ float4 cres[CONS ? 4 * kOwn : 1];    // force sums and count bits (CONS)
   __shared__ uint32_t cedge[CONS ? 4 * kOwn : 1];  // kept edges | active << 30 | edges << 31
   const int lane = threadIdx.x & (kWave - 1);
@@ -1378,6 +1518,7 @@ k_force_list(ForceArgs a) {
   c.fzr = fminf(fmaxf(pi.z * sd.ihz - (float)c.cz, 0.0f), 1.0f);
   own_gaps<R>(c, sd);
   if (EDGES && g == 0) el_n[wv][o] = 0u;
+  if (HITS && g == 0) hn[wv][o] = 0u;
   // the pruning radius straight from the pair table in memory, so the stencil rows (and
   // their cell-start loads) overlap the copy of the table into LDS
   c.cut2 = active ? a.pairs[sd.tab + ti * sd.T].pad : 0.0f;
@@ -1385,24 +1526,32 @@ k_force_list(ForceArgs a) {
   // ---- this lane's runs, their place in the particle's flattened candidate order ----
   uint32_t rs[2 * kRpl], rl[2 * kRpl], rk[2 * kRpl];
   uint32_t mine = 0u;
-  if (R == 1 && G == 8 && !c.gen) {
-    // 9 rows over 8 lanes in one pass: lane g takes row g (lane 4 row 8 in place of the
-    // centre row 4), and every lane works out the centre row, which has no y or z wrap
-    // and no y or z gap (so the row itself folds to its x ends), for lane 0 to keep
-    static_assert(R != 1 || G != 8 || kRpl == 2, "two run pairs per lane");
+  bool fast8 = false;
+  if constexpr (R == 1 && G == 8) {
+    if (!c.gen) {
+      // 9 rows over 8 lanes in one pass, and every lane works out the centre row, which has
+      // no y or z wrap and no y or z gap (so the row itself folds to its x ends), for one
+      // lane to keep: lane g takes row g (lane 4 row 8 in place of the centre row 4) and
+      // lane 0 keeps the centre row; in row order (V), lanes 0-3 take rows 0-3, lanes 4-7
+      // rows 5-8, and lane 3 keeps the centre row
+      static_assert(kRpl == 2, "two run pairs per lane");
+      fast8 = true;
 #pragma unroll
-    for (int k = 0; k < 2 * kRpl; ++k) rs[k] = rl[k] = rk[k] = 0u;
-    if (active) {
-      row_runs_fast<R>(a, sd, c, g == 4 ? 8 : g, rs[0], rl[0], rk[0], rs[1], rl[1], rk[1]);
-      row_runs_fast<R>(a, sd, c, 4, rs[2], rl[2], rk[2], rs[3], rl[3], rk[3]);
-      if (g != 0) rl[2] = rl[3] = 0u;
+      for (int k = 0; k < 2 * kRpl; ++k) rs[k] = rl[k] = rk[k] = 0u;
+      if (active) {
+        row_runs_fast<R>(a, sd, c, V ? g + (g >> 2) : g == 4 ? 8 : g, rs[0], rl[0], rk[0], rs[1],
+                         rl[1], rk[1]);
+        row_runs_fast<R>(a, sd, c, 4, rs[2], rl[2], rk[2], rs[3], rl[3], rk[3]);
+        if (g != (V ? 3 : 0)) rl[2] = rl[3] = 0u;
+      }
+#pragma unroll
+      for (int k = 0; k < 2 * kRpl; ++k) mine += rl[k];
     }
-#pragma unroll
-    for (int k = 0; k < 2 * kRpl; ++k) mine += rl[k];
-  } else {
+  }
+  if (!fast8) {
 #pragma unroll
     for (int i = 0; i < kRpl; ++i) {
-      const int r = g + i * G;
+      const int r = V ? g * kRpl + i : g + i * G;  // V: the lanes' rows in row order
       rs[2 * i] = rl[2 * i] = rk[2 * i] = rs[2 * i + 1] = rl[2 * i + 1] = rk[2 * i + 1] = 0u;
       if (active && r < nrows)
         row_runs<R>(a, sd, c, r, rs[2 * i], rl[2 * i], rk[2 * i], rs[2 * i + 1], rl[2 * i + 1],
@@ -1421,14 +1570,17 @@ k_force_list(ForceArgs a) {
   // is an odd multiple of G: each lane keeps the entries it takes in one pass (g, g+G, ...)
   // and the particles' lanes of one read fall on different banks.
   static_assert(kWaveList % kWave == 0, "list of whole rows");
-  constexpr uint32_t kQuota = (uint32_t)(G * ((kWaveList / kWave - 1) | 1));
+  constexpr uint32_t kQuota =
+      V ? (uint32_t)(VL * ((kWaveList / kOwn / VL - 1) | 1)) : (uint32_t)(G * ((kWaveList / kWave - 1) | 1));
+  static_assert(kQuota * kOwn <= kWaveList && kQuota % VL == 0, "whole passes");
   uint32_t incl = total;
 #pragma unroll
   for (int d = G; d < kWave; d <<= 1) {
     const uint32_t y = __shfl_up(incl, d, kWave);
     if (lane >= d) incl += y;
   }
-  const bool packed = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1) <= (uint32_t)kWaveList;
+  const uint32_t wave_total = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+  const bool packed = wave_total <= (uint32_t)kWaveList;
   const uint32_t obase = packed ? incl - total : (uint32_t)o * kQuota;
   const uint32_t quota = packed ? (uint32_t)kWaveList : kQuota;
   wave_lds_sync();  // pair table ready
@@ -1438,8 +1590,172 @@ k_force_list(ForceArgs a) {
   const bool want_edges = EDGES && a.edges && sd.edge_on;  // the same for the whole wave
   const bool do_edges = want_edges && active;
   float fx = 0.0f, fy = 0.0f, fz = 0.0f;
+  float hx = 0.0f, hy = 0.0f, hz = 0.0f;  // the sums of the lane's other order lane
   int cnt = 0;
-  for (uint32_t b0 = 0; b0 < total; b0 += quota) {
+  // order lane of this lane (and, with two, of this one + G): lanes 4-7 of each eight in
+  // reverse, so that the half mirror of the sums below pairs order lanes 4 apart
+  const int gv = V ? ((g & 4) ? (g & ~7) + 11 - (g & 7) : g) : g;
+  // the particle whose candidates this lane takes (its own; in the dense walk at G = 8 one
+  // of the wave's, 16 lanes each)
+  float px = pi.x, py = pi.y, pz = pi.z;
+  uint32_t pt = ti, pid = idi;
+  int ps = p, po = o;
+  bool pe = do_edges;
+  const float* prow = row;
+  auto swap_sums = [&]() {
+    float t = fx; fx = hx; hx = t;
+    t = fy; fy = hy; hy = t;
+    t = fz; fz = hz; hz = t;
+  };
+  // ParticleSimulation.cu:92-131 for candidate q: cutoff, count, force, edge candidate.
+  // code: image shift of a shifted run (0: none); jq: the candidate's index where HAVE_ID
+  auto pair = [&](auto gen_kind, auto have_id, uint32_t q, uint32_t code, const float4& pj,
+                  uint32_t jq) {
+    constexpr bool GEN = decltype(gen_kind)::value;
+    constexpr bool HAVE_ID = decltype(have_id)::value;
+    float dx = pj.x - px, dy = pj.y - py, dz = pj.z - pz;
+    bool raw;
+    if constexpr (!GEN) {
+      raw = code == 0u;
+      if (!raw) {  // image-shifted run
+        dx += shift_of(code & 3u, sd.Lx);
+        dy += shift_of((code >> 2) & 3u, sd.Ly);
+        dz += shift_of((code >> 4) & 3u, sd.Lz);
+      }
+    } else {  // per-pair minimum image
+      const float ux = dx, uy = dy, uz = dz;
+      dx = min_image(ux, sd.Lx);
+      dy = min_image(uy, sd.Ly);
+      dz = min_image(uz, sd.Lz);
+      raw = (dx == ux) && (dy == uy) && (dz == uz);
+    }
+    const float s2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+    const uint32_t tj = __float_as_uint(pj.w);
+    const float thr = prow[tj];
+    const float sp = s2 + 1e-4f;
+    if (sp < thr) {
+      cnt++;
+      // (rep e^(-k rr^2) - att rr) fv / r with rr = r / effR, r = sqrt(sp), the constants
+      // folded per type pair
+      const float rep_fv = prow[kTT + tj], att_fv_ie = prow[2 * kTT + tj];
+      const float k_ie2 = prow[3 * kTT + tj];
+      const float inv = __builtin_amdgcn_rsqf(sp);
+      const float ex = __builtin_amdgcn_exp2f(k_ie2 * sp);
+      const float w = fmaf(rep_fv, ex, -(att_fv_ie * (sp * inv))) * inv;
+      fx = fmaf(dx, w, fx);
+      fy = fmaf(dy, w, fy);
+      fz = fmaf(dz, w, fz);
+      if (HITS && q != (uint32_t)ps) {
+        const uint32_t at = atomicAdd(&hn[wv][po], 1u);
+        if (at < (uint32_t)kPairList) hl[wv][po][at] = q;
+      }
+    }
+    if (EDGES) {
+      // edges are non-periodic (ParticleSimulation.cu:222-227): unshifted pairs only
+      if (pe && raw && tj == pt && s2 < sd.edge_d2) {
+        const uint32_t jid = HAVE_ID ? jq : a.id[q];
+        if (jid > pid) {
+          const uint32_t kk = atomicAdd(&el_n[wv][po], 1u);
+          if (kk < (uint32_t)kLE) {
+            el_d[wv][po][kk] = make_float2(s2, 0.0f);
+            el_i[wv][po][kk] = jid;
+          }
+        }
+      }
+    }
+  };
+  const bool walk = V != 0 && wave_total > kWalkFrom;
+  if constexpr (V != 0) if (walk) {
+    // dense neighbourhoods: no list (it would cost about as much as the pairs), the lanes
+    // walk the runs themselves from a table in the list's place, entry 2 * row + half
+    static_assert(kOwn * 2 * kRows * 2 <= kWaveList, "the run table fits the list");
+    uint2* wr = reinterpret_cast<uint2*>(&lslot[wv][0]) + o * 2 * kRows;
+    // entry of this lane's run pair i (-1: none); lane 3 also keeps the centre row (fast8)
+    auto entry = [&](int i) {
+      if (fast8) return i == 0 ? 2 * (g + (g >> 2)) : g == 3 ? kRows - 1 : -1;
+      return g * kRpl + i < kRows ? 2 * (g * kRpl + i) : -1;
+    };
+#pragma unroll
+    for (int i = 0; i < kRpl; ++i) {
+      const int e = entry(i);
+      if (e >= 0) {
+        wr[e] = make_uint2(rs[2 * i], rl[2 * i]);
+        wr[e + 1] = make_uint2(rs[2 * i + 1], rl[2 * i + 1]);
+      }
+    }
+    wave_lds_sync();
+    // 16 lanes per particle, one for each order lane: at G = 8 the wave takes its particles
+    // four at a time
+    static_assert(V == 0 || V == 16, "16 order lanes");
+    const uint2* wt = reinterpret_cast<const uint2*>(&lslot[wv][0]);
+    auto runs = [&](auto gen_kind) {
+      const int gw16 = lane & 15;
+      const int v16 = (gw16 & 4) ? (gw16 & 8) + 11 - (gw16 & 7) : gw16;
+#pragma unroll 1
+      for (int b4 = 0; b4 < kOwn; b4 += 4) {
+        if (G != 16) {
+          po = b4 + (lane >> 4);
+          ps = (int)base + po;
+          pe = want_edges;  // an inactive particle has no runs
+          const float4 pw = a.pos[ps];
+          px = pw.x;
+          py = pw.y;
+          pz = pw.z;
+          pt = ps - sd.p0 < sd.n ? __float_as_uint(pw.w) : 0u;
+          pid = a.id[ps];
+          prow = &ptab[pt * sd.T];
+          fx = fy = fz = 0.0f;
+          cnt = 0;
+        }
+        const uint2* we = wt + po * 2 * kRows;
+        uint32_t cum = 0u;
+        for (int r = 0; r < 2 * nrows; ++r) {
+          const uint2 e = we[r];
+          const uint32_t len = e.y;
+          if (len == 0u) continue;
+          const uint32_t q0 = e.x & ((1u << kCodeShift) - 1u), code = e.x >> kCodeShift;
+          uint32_t t = (uint32_t)(v16 - (int)cum) & 15u;
+          if (t < len) {
+            float4 pj = a.pos[q0 + t];
+            while (true) {
+              const uint32_t tn = t + 16u;
+              const float4 pn = a.pos[q0 + min(tn, len - 1u)];
+              pair(gen_kind, std::false_type{}, q0 + t, code, pj, 0u);
+              if (tn >= len) break;
+              t = tn;
+              pj = pn;
+            }
+          }
+          cum += len;
+        }
+        if (G != 16) {
+          fx = ordered_sum<16>(fx);
+          fy = ordered_sum<16>(fy);
+          fz = ordered_sum<16>(fz);
+          cnt = dpp_group_sum_i<16>(cnt);
+          if (1e-4f < prow[pt]) cnt -= 1;  // the particle itself
+          if (gw16 == 0) cres[wv * kOwn + po] = make_float4(fx, fy, fz, __int_as_float(cnt));
+        }
+      }
+    };
+    if (c.gen) runs(std::true_type{});
+    else runs(std::false_type{});
+    // the lane's runs again, for the edge overflow below: they take no registers in between
+    if constexpr (EDGES) {
+#pragma unroll
+      for (int i = 0; i < kRpl; ++i) {
+        const int e = entry(i);
+        const uint2 r0 = e >= 0 ? wr[e] : make_uint2(0u, 0u);
+        const uint2 r1 = e >= 0 ? wr[e + 1] : make_uint2(0u, 0u);
+        rs[2 * i] = r0.x;
+        rl[2 * i] = r0.y;
+        rs[2 * i + 1] = r1.x;
+        rl[2 * i + 1] = r1.y;
+      }
+    }
+    __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");
+  }
+  for (uint32_t b0 = 0; b0 < (walk ? 0u : total); b0 += quota) {
     const uint32_t b1 = b0 + quota;
     uint32_t f0 = first;
 #pragma unroll
@@ -1464,80 +1780,72 @@ k_force_list(ForceArgs a) {
     // one copy of the loop per grid kind (the choice is the same for the whole wave), so
     // the common kind carries no per-pair minimum-image code
     auto pairs = [&](auto gen_kind) {
-      constexpr bool GEN = decltype(gen_kind)::value;
-      for (uint32_t k = (uint32_t)g; k < nb; k += (uint32_t)G) {
-        const uint32_t e = lslot[wv][obase + k];
-        const uint32_t q = e & ((1u << kCodeShift) - 1u), code = e >> kCodeShift;
-        const float4 pj = a.pos[q];
-        // the index travels with the position: an edge candidate then waits for no load
-        const uint32_t jq = want_edges ? a.id[q] : 0u;
-        float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-        bool raw;
-        if constexpr (!GEN) {
-          raw = code == 0u;
-          if (!raw) {  // image-shifted run
-            dx += shift_of(code & 3u, sd.Lx);
-            dy += shift_of((code >> 2) & 3u, sd.Ly);
-            dz += shift_of((code >> 4) & 3u, sd.Lz);
-          }
-        } else {  // per-pair minimum image
-          const float ux = dx, uy = dy, uz = dz;
-          dx = min_image(ux, sd.Lx);
-          dy = min_image(uy, sd.Ly);
-          dz = min_image(uz, sd.Lz);
-          raw = (dx == ux) && (dy == uy) && (dz == uz);
+#pragma unroll 1
+      for (int h = 0; h < kSub; ++h) {
+        for (uint32_t k = (uint32_t)(gv + h * G); k < nb; k += (uint32_t)VL) {
+          const uint32_t e = lslot[wv][obase + k];
+          const uint32_t q = e & ((1u << kCodeShift) - 1u);
+          const float4 pj = a.pos[q];
+          // the index travels with the position: an edge candidate then waits for no load
+          const uint32_t jq = want_edges ? a.id[q] : 0u;
+          pair(gen_kind, std::true_type{}, q, e >> kCodeShift, pj, jq);
         }
-        const float s2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-        const uint32_t tj = __float_as_uint(pj.w);
-        const float thr = row[tj];
-        const float sp = s2 + 1e-4f;
-        if (sp < thr) {
-          cnt++;
-          // ParticleSimulation.cu:104-131 with rr = r / effR, r = sqrt(sp):
-          // (rep e^(-k rr^2) - att rr) fv / r, the constants folded per type pair
-          const float rep_fv = row[kTT + tj], att_fv_ie = row[2 * kTT + tj];
-          const float k_ie2 = row[3 * kTT + tj];
-          const float inv = __builtin_amdgcn_rsqf(sp);
-          const float ex = __builtin_amdgcn_exp2f(k_ie2 * sp);
-          const float w = fmaf(rep_fv, ex, -(att_fv_ie * (sp * inv))) * inv;
-          fx = fmaf(dx, w, fx);
-          fy = fmaf(dy, w, fy);
-          fz = fmaf(dz, w, fz);
-        }
-        if (EDGES) {
-          // edges are non-periodic (ParticleSimulation.cu:222-227): unshifted pairs only
-          if (do_edges && raw && tj == ti && s2 < sd.edge_d2) {
-            const uint32_t jid = jq;
-            if (jid > idi) {
-              const uint32_t kk = atomicAdd(&el_n[wv][o], 1u);
-              if (kk < (uint32_t)kListEdges) {
-                el_d[wv][o][kk] = make_float2(s2, 0.0f);
-                el_i[wv][o][kk] = jid;
-              }
-            }
-          }
-        }
+        if (kSub > 1) swap_sums();
       }
     };
     if (c.gen) pairs(std::true_type{});
     else pairs(std::false_type{});
     __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront");  // list reused by the next chunk
   }
-  fx = dpp_group_sum_f<G>(fx);
-  fy = dpp_group_sum_f<G>(fy);
-  fz = dpp_group_sum_f<G>(fz);
-  cnt = dpp_group_sum_i<G>(cnt);
-  if (active && 1e-4f < row[ti]) cnt -= 1;  // the particle itself
+  if constexpr (V != 0) {
+    static_assert(CONS, "the sums go to LDS");
+    if (G == 16 || !walk) {
+      if constexpr (kSub > 1) {  // order lanes G apart
+        fx += hx;
+        fy += hy;
+        fz += hz;
+      }
+      fx = ordered_sum<G>(fx);
+      fy = ordered_sum<G>(fy);
+      fz = ordered_sum<G>(fz);
+      cnt = dpp_group_sum_i<G>(cnt);
+      if (active && 1e-4f < row[ti]) cnt -= 1;  // the particle itself
+      if (g == 0) cres[wv * kOwn + o] = make_float4(fx, fy, fz, __int_as_float(cnt));
+    }
+  } else {
+    fx = dpp_group_sum_f<G>(fx);
+    fy = dpp_group_sum_f<G>(fy);
+    fz = dpp_group_sum_f<G>(fz);
+    cnt = dpp_group_sum_i<G>(cnt);
+    if (active && 1e-4f < row[ti]) cnt -= 1;  // the particle itself
+  }
+  if constexpr (HITS) {
+    // the wave's lists are complete: each in slot order (rank by counting; slots are
+    // distinct), all of a particle's partners or, beyond kPairList, only their number
+    wave_lds_sync();
+    const uint32_t nh = active ? hn[wv][o] : 0u;
+    const long k = (long)(p - sd.p0);
+    if (nh <= (uint32_t)kPairList)
+      for (uint32_t e = g; e < nh; e += G) {
+        const uint32_t q = hl[wv][o][e];
+        uint32_t rank = 0;
+        for (uint32_t e2 = 0; e2 < nh; ++e2) rank += (hl[wv][o][e2] < q) ? 1u : 0u;
+        a.hits[k * kPairList + rank] = q;
+      }
+    if (active && g == 0) a.nhits[k] = nh;
+  }
   // CONS: the sums go to LDS now, so they take no registers through the edge selection
-  if (CONS && g == 0) cres[wv * kOwn + o] = make_float4(fx, fy, fz, __int_as_float(cnt));
+  if (V == 0 && CONS && g == 0) cres[wv * kOwn + o] = make_float4(fx, fy, fz, __int_as_float(cnt));
 
   uint32_t ekept = 0u;  // kept edges of the particle (lane g == 0), passed on by CONS
   if (EDGES) {
     // the wave's candidate lists are complete
     wave_lds_sync();
     const uint32_t n = do_edges ? el_n[wv][o] : 0u;
-    const bool fits = n <= (uint32_t)kListEdges;
+    const bool fits = n <= (uint32_t)kLE;
     const int cap = a.edge_cap, maxc = sd.edge_maxc;
+    // the owner's record: by index when the tile sort follows, else by slot
+    const uint32_t orec = TILE ? idi : (uint32_t)p;
     if (fits)
       for (uint32_t k = g; k < n; k += G) {
         const uint32_t ik = el_i[wv][o][k];
@@ -1558,151 +1866,39 @@ k_force_list(ForceArgs a) {
           rank += (d2.y != 0.0f && (d2.x < dk.x || (d2.x == dk.x && i2 < ik))) ? 1u : 0u;
         }
         if (rank < (uint32_t)maxc)
-          a.estage[(long)(TILE ? idi : (uint32_t)p) * a.estride + rank] = ik;
+          a.estage[(long)orec * a.estride + rank] = ik;
       }
     // Owners with more candidates than their LDS list holds (n counts them all): the whole
-    // wave takes them one at a time, in the wave's LDS lists (free now: every fitting
-    // owner's selection above is done).  Its 64 lanes walk the owner's flattened candidates
-    // again, append the qualifying ones (d^2 in el_d's words, index in lslot's, up to
-    // kOvfCap), keep the cap smallest indices and rank those by (d^2, index), as above.
-    // More than kOvfCap qualifying: the owner's lane takes the streaming selection below.
-    uint32_t ovf_e = ~0u;  // kept edges of an owner this handled (its lane g == 0)
-    if constexpr (G == 8) {
-      constexpr int kOvfCap = 320;
-      static_assert(kOvfCap <= kWaveList, "indices fit the wave's lslot");
-      static_assert(kOvfCap <= 2 * kOwn * kListEdges, "d^2 fits the wave's el_d");
-      constexpr int kOvfInfo = G * 2 * kRpl * 2;  // after the runs in the wave's el_i
-      static_assert(kOvfInfo + 7 <= kOwn * kListEdges, "runs and owner fit the wave's el_i");
-      float* ov_d = &el_d[wv][0][0].x;
-      uint32_t* ov_i = &lslot[wv][0];
-      uint32_t* ov_r = &el_i[wv][0][0];
+    // wave takes them one at a time, in the wave's LDS lists (free then: every fitting
+    // owner's selection above is done)
+    uint32_t ovf_e = 0u;  // kept edges of an owner this handled (its lane g == 0)
+    {
+      static_assert(kOwn * kLE >= kSelCap, "the selection fits the wave's el_d");
+      static_assert(G * 2 * kRpl * 2 <= kOwn * kLE, "an owner's runs fit the wave's el_i");
+      uint2* ov_r = reinterpret_cast<uint2*>(&el_i[wv][0][0]);
       unsigned long long left = __ballot(do_edges && g == 0 && !fits);
       if (left) wave_lds_sync();  // the fitting owners' reads of el_d, el_i are done
       while (left) {
         const int L = __ffsll((long long)left) - 1;
         left &= left - 1ull;
         const int os = L / G;
-        // the owner's runs, position, type, index, candidate count and record go to LDS
-        // (read where used: they take no registers through the walk)
         if (o == os)
 #pragma unroll
-          for (int k = 0; k < 2 * kRpl; ++k) {
-            ov_r[(g * 2 * kRpl + k) * 2] = rs[k];
-            ov_r[(g * 2 * kRpl + k) * 2 + 1] = rl[k];
-          }
-        if (lane == L) {
-          ov_r[kOvfInfo] = __float_as_uint(pi.x);
-          ov_r[kOvfInfo + 1] = __float_as_uint(pi.y);
-          ov_r[kOvfInfo + 2] = __float_as_uint(pi.z);
-          ov_r[kOvfInfo + 3] = ti;
-          ov_r[kOvfInfo + 4] = idi;
-          ov_r[kOvfInfo + 5] = total;
-          ov_r[kOvfInfo + 6] = TILE ? idi : (uint32_t)p;
-          el_n[wv][os] = 0u;
-        }
+          for (int k = 0; k < 2 * kRpl; ++k) ov_r[g * 2 * kRpl + k] = make_uint2(rs[k], rl[k]);
         wave_lds_sync();
-        const uint32_t otot = ov_r[kOvfInfo + 5];
-        for (uint32_t i0 = 0; i0 < otot; i0 += (uint32_t)kWave) {
-          const uint32_t i = i0 + (uint32_t)lane;
-          if (i >= otot) continue;
-          uint32_t off = i, ent = 0u;
-          for (int r = 0; r < G * 2 * kRpl; ++r) {
-            const uint32_t len = ov_r[2 * r + 1];
-            if (off < len) {
-              ent = ov_r[2 * r] + off;
-              break;
-            }
-            off -= len;
-          }
-          const uint32_t q = ent & ((1u << kCodeShift) - 1u);
-          if (!c.gen && (ent >> kCodeShift) != 0u) continue;  // image-shifted: no partner
-          const float4 pj = a.pos[q];
-          if (__float_as_uint(pj.w) != ov_r[kOvfInfo + 3]) continue;
-          const float ux = pj.x - __uint_as_float(ov_r[kOvfInfo]),
-                      uy = pj.y - __uint_as_float(ov_r[kOvfInfo + 1]),
-                      uz = pj.z - __uint_as_float(ov_r[kOvfInfo + 2]);
-          if (c.gen && !(min_image(ux, sd.Lx) == ux && min_image(uy, sd.Ly) == uy &&
-                         min_image(uz, sd.Lz) == uz))
-            continue;
-          const float s2 = fmaf(uz, uz, fmaf(uy, uy, ux * ux));
-          if (!(s2 < sd.edge_d2)) continue;
-          const uint32_t jid = a.id[q];
-          if (jid <= ov_r[kOvfInfo + 4]) continue;
-          const uint32_t k = atomicAdd(&el_n[wv][os], 1u);
-          if (k < (uint32_t)kOvfCap) {
-            ov_d[k] = s2;
-            ov_i[k] = jid;
-          }
-        }
-        wave_lds_sync();
-        const uint32_t m = el_n[wv][os];
-        if (m <= (uint32_t)kOvfCap) {
-          // the cap smallest indices (marked in bit 31; indices stay below 2^26)
-          uint32_t keep = 0u;
-          for (uint32_t k = lane, b = 0; k < m; k += kWave, ++b) {
-            const uint32_t ik = ov_i[k];
-            uint32_t below = 0;
-            for (uint32_t k2 = 0; k2 < m; ++k2) below += (ov_i[k2] < ik) ? 1u : 0u;
-            keep |= (below < (uint32_t)cap ? 1u : 0u) << b;
-          }
-          wave_lds_sync();
-          for (uint32_t k = lane, b = 0; k < m; k += kWave, ++b)
-            if ((keep >> b) & 1u) ov_i[k] |= 0x80000000u;
-          wave_lds_sync();
-          for (uint32_t k = lane; k < m; k += kWave) {
-            const uint32_t ik = ov_i[k];
-            if (!(ik & 0x80000000u)) continue;
-            const float dk = ov_d[k];
-            uint32_t rank = 0;
-            for (uint32_t k2 = 0; k2 < m; ++k2) {
-              const uint32_t i2 = ov_i[k2];
-              const float d2 = ov_d[k2];
-              rank += ((i2 & 0x80000000u) && (d2 < dk || (d2 == dk && i2 < ik))) ? 1u : 0u;
-            }
-            if (rank < (uint32_t)maxc)
-              a.estage[(long)ov_r[kOvfInfo + 6] * a.estride + rank] = ik & 0x7FFFFFFFu;
-          }
-          if (lane == L) ovf_e = (uint32_t)min(min((int)m, cap), maxc);
-        }
-        wave_lds_sync();  // the LDS lists are reused for the next owner
+        // the owner's state again, at a uniform address: it takes no registers until here
+        const int so = __builtin_amdgcn_readfirstlane((int)base + os);
+        const float4 me = a.pos[so];
+        const uint32_t myid = a.id[so];
+        WaveSel sel{&el_d[wv][0][0], 0, 0xFFFFFFFFu};
+        wave_sel_runs<true>(sel, a.pos, a.id, ov_r, G * 2 * kRpl, me, myid, sd, c.gen, cap, lane);
+        const uint32_t e = wave_sel_finish(
+            sel, cap, maxc, a.estage + (long)(TILE ? myid : (uint32_t)so) * a.estride, lane);
+        if (lane == L) ovf_e = e;
       }
     }
     if (do_edges && g == 0) {
-      uint32_t e;
-      if (fits) {
-        e = (uint32_t)min(min((int)n, cap), maxc);
-      } else if (ovf_e != ~0u) {
-        e = ovf_e;
-      } else {
-        // more candidates than the wave's LDS lists hold: exact streaming selection by one
-        // lane, over the stencil rows again
-        EdgeAcc ea;
-        ea.q = 0;
-        ea.maxid = 0;
-        ea.maxk = 0;
-        for (int r = 0; r < nrows; ++r) {
-          uint32_t st[2], ln[2], cd[2];
-          row_runs<R>(a, sd, c, r, st[0], ln[0], cd[0], st[1], ln[1], cd[1]);
-          for (int h = 0; h < 2; ++h) {
-            if (!c.gen && cd[h] != 0u) continue;  // image-shifted runs hold no edge partner
-            for (uint32_t t = 0; t < ln[h]; ++t) {
-              const uint32_t q = st[h] + t;
-              const float4 pj = a.pos[q];
-              if (__float_as_uint(pj.w) != ti) continue;
-              const float ux = pj.x - pi.x, uy = pj.y - pi.y, uz = pj.z - pi.z;
-              if (c.gen && !(min_image(ux, sd.Lx) == ux && min_image(uy, sd.Ly) == uy &&
-                             min_image(uz, sd.Lz) == uz))
-                continue;
-              const float s2 = fmaf(uz, uz, fmaf(uy, uy, ux * ux));
-              if (!(s2 < sd.edge_d2)) continue;
-              const uint32_t jid = a.id[q];
-              if (jid > idi) edge_push(ea, s2, jid, cap, a.ecand_d2, a.ecand_id, a.P, p);
-            }
-          }
-        }
-        e = (uint32_t)edge_finish(ea, cap, maxc, a.ecand_d2, a.ecand_id, a.estage, a.P, p,
-                                  TILE ? idi : (uint32_t)p, a.estride);
-      }
+      const uint32_t e = fits ? (uint32_t)min(min((int)n, cap), maxc) : ovf_e;
       ekept = e;
       if (!CONS && e != 0u) a.ecount[idi] = e;  // zero already (the sorts clear it)
     }
@@ -1725,13 +1921,36 @@ k_force_list(ForceArgs a) {
       const uint32_t e = fl & 0x3FFFFFFFu;
       if (e != 0u) a.ecount[pl_id] = e;  // zero already (the sorts clear it)
     }
-    integrate_commit<TILE>(a, sd, pl, pl_pos, pl_vel, pl_id, r.x, r.y, r.z,
-                           __float_as_int(r.w), bin_axis(pl_pos.y, sd.ihy, sd.ny),
-                           bin_axis(pl_pos.z, sd.ihz, sd.nz));
+    SimDesc td = sd;
+    // the grid sizes' float copies made here again, not kept (in vector registers) from the
+    // start of the kernel
+    if constexpr (V != 0) asm volatile("" : "+s"(td.nx), "+s"(td.ny), "+s"(td.nz));
+    integrate_commit<TILE>(a, td, pl, pl_pos, pl_vel, pl_id, r.x, r.y, r.z,
+                           __float_as_int(r.w), bin_axis(pl_pos.y, td.ihy, td.ny),
+                           bin_axis(pl_pos.z, td.ihz, td.nz));
     return;
   }
   if (!active || g != 0) return;
   integrate_commit<TILE>(a, sd, p, pi, vi, idi, fx, fy, fz, cnt, c.cy, c.cz);
+}
+
+// The force kernels of variants 3 (CONS false) and 4.
+// With the consolidated tail, the 27-cell stencil at G = 8 fits 7 waves per SIMD (72 VGPRs,
+// under 22.8 KB of LDS per block).  Without it the velocity stays live to the end and the
+// kernel needs a few more registers: held to 72 it spills, and a spilling kernel's scratch
+// allocation cuts its occupancy far below 7 waves (a 6x slower launch), so no hint there.
+template <bool EDGES, int R, int G, bool TILE, bool CONS = false>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(R == 1 && G == 8 && CONS ? 7 : 1, 8)))
+k_force_list(ForceArgs a) {
+  force_list<EDGES, R, G, TILE, CONS>(a);
+}
+
+// Variant 0 at 16 lanes per particle (the default tuning), see above.  HITS (the gradient
+// rollout, no edges): also lists each particle's in-range partners (ForceArgs::hits).
+template <bool EDGES, int R, int G, bool TILE, bool HITS = false>
+__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(EDGES && R == 1 && G == 8 ? 7 : 1, 8)))
+k_force_ord(ForceArgs a) {
+  force_list<EDGES, R, G, TILE, true, 16, HITS>(a);
 }
 
 // ------------------------------------------------------------------------------------
@@ -1744,9 +1963,11 @@ k_force_list(ForceArgs a) {
 // 0.052 cell.  Qualifying candidates (same type :219, larger index :215, d^2 < D^2 :227) go
 // to the owner's LDS list; the two-phase selection then keeps the 2*maxC smallest indices
 // and ranks them by (d^2, index) (:228-246).  An owner with more than kListEdges candidates
-// takes the exact streaming selection of one lane.  Kept partners are staged by owner index
-// (estage[index * estride + rank]), the non-zero per-owner counts go to `ecount`, and
-// k_tile_sort's edge tiles write the canonical list.
+// is chosen for by its whole wave (WaveSel).  Rows longer than kEdgeShare slots are shared by
+// the owner's lanes.  Kept partners are staged by owner index (estage[index * estride +
+// rank]), the non-zero per-owner counts go to `ecount`, and k_tile_sort's edge tiles write the
+// canonical list.  Bound: latency in sparse states (100k: 15.5 us), issue in dense ones (20k
+// of a preset, 516 neighbours: 55 -> 33 us; 1M clustered 1353 -> 290 us).
 
 constexpr int kEdgeLanes = 8;
 
@@ -1817,17 +2038,18 @@ __device__ __forceinline__ bool edge_row_fast(const SimDesc& sd, const EdgeOwner
 }
 
 // Runs a lane's stencil rows r = r0, r0 + G, ... (kEdgeRowBatch of them at a time, their
-// cell-start loads issued together) and calls f(q, pj, jid) for each slot q, in row order.
+// cell-start loads issued together) and calls f(pj, jid) for each slot, in row order.
 // The batch's slot runs are walked as one sequence, kEdgeLoadBatch slots at a time, so the
 // loads of several short rows are in flight together; an index is loaded with its
 // position, so a qualifying candidate waits for no further load.
 constexpr int kEdgeRowBatch = 3;
 constexpr int kEdgeLoadBatch = 4;
+constexpr int kEdgeRuns = 9;    // rows of the reach-1 stencil
+constexpr int kEdgeShare = 32;  // slots of one lane's rows above which its owner's lanes share them
 
-// ER > 0: reach ER on every axis (edge_row_fast); ER = 0: any reach (edge_row).
-template <int ER, class F>
+template <class F>
 __device__ __forceinline__ void edge_walk(const EdgeArgs& a, const SimDesc& sd,
-                                          const EdgeOwner<ER>& w, float cut2, int r0, int step,
+                                          const EdgeOwner<0>& w, float cut2, int r0, int step,
                                           int nrows, F&& f) {
   for (int rb = r0; rb < nrows; rb += kEdgeRowBatch * step) {
     int c0[kEdgeRowBatch], c1[kEdgeRowBatch];
@@ -1835,11 +2057,8 @@ __device__ __forceinline__ void edge_walk(const EdgeArgs& a, const SimDesc& sd,
 #pragma unroll
     for (int i = 0; i < kEdgeRowBatch; ++i) {
       const int r = rb + i * step;
-      if constexpr (ER > 0)
-        on[i] = r < nrows && edge_row_fast<ER>(sd, w, cut2, r, c0[i], c1[i]);
-      else
-        on[i] = r < nrows && edge_row(sd, w.cx, w.cy, w.cz, w.fxr, w.fyr, w.fzr, cut2, r,
-                                      c0[i], c1[i]);
+      on[i] = r < nrows && edge_row(sd, w.cx, w.cy, w.cz, w.fxr, w.fyr, w.fzr, cut2, r, c0[i],
+                                    c1[i]);
     }
     int qa[kEdgeRowBatch], len[kEdgeRowBatch];
 #pragma unroll
@@ -1854,7 +2073,6 @@ __device__ __forceinline__ void edge_walk(const EdgeArgs& a, const SimDesc& sd,
       total += len[i];
     }
     for (int x0 = 0; x0 < total; x0 += kEdgeLoadBatch) {
-      int qs[kEdgeLoadBatch];
       float4 pj[kEdgeLoadBatch];
       uint32_t jid[kEdgeLoadBatch];
 #pragma unroll
@@ -1866,23 +2084,23 @@ __device__ __forceinline__ void edge_walk(const EdgeArgs& a, const SimDesc& sd,
           if (x >= run) q = qa[i] + (x - run);
           run += len[i];
         }
-        qs[u] = q;
         const bool in = x < total;
         pj[u] = in ? a.pos[q] : make_float4(0.0f, 0.0f, 0.0f, -1.0f);
         jid[u] = in ? a.id[q] : 0u;
       }
 #pragma unroll
       for (int u = 0; u < kEdgeLoadBatch; ++u)
-        if (x0 + u < total) f(qs[u], pj[u], jid[u]);
+        if (x0 + u < total) f(pj[u], jid[u]);
     }
   }
 }
 
 template <int ER>
-__device__ __forceinline__ void edges_owner(const EdgeArgs& a, const SimDesc& sd, int wv, int o,
-                                            int g, int p, bool active, const float4& pi,
+__device__ __forceinline__ void edges_owner(const EdgeArgs& a, const SimDesc& sd, int o, int g,
+                                            int lane, int base, bool active, const float4& pi,
                                             uint32_t idi, float2 (*el_d)[kListEdges],
-                                            uint32_t (*el_i)[kListEdges], uint32_t* el_n) {
+                                            uint32_t (*el_i)[kListEdges], uint32_t* el_n,
+                                            uint2 (*el_r)[ER == 1 ? kEdgeRuns : 1]) {
   constexpr int G = kEdgeLanes;
   const uint32_t ti = __float_as_uint(pi.w);
   EdgeOwner<ER> w;
@@ -1906,20 +2124,77 @@ __device__ __forceinline__ void edges_owner(const EdgeArgs& a, const SimDesc& sd
   const int nrows = (2 * sd.edge_ry + 1) * (2 * sd.edge_rz + 1);
   if (g == 0) el_n[o] = 0u;
   wave_lds_sync();
-  if (active)
-    edge_walk<ER>(a, sd, w, cut2, g, G, nrows,
-              [&](int, const float4& pj, uint32_t jid) {
-                if (__float_as_uint(pj.w) != ti) return;        // :219
-                const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-                const float s2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-                if (!(s2 < sd.edge_d2)) return;                  // :227
-                if (jid <= idi) return;                          // j > i, :215
-                const uint32_t kk = atomicAdd(&el_n[o], 1u);
-                if (kk < (uint32_t)kListEdges) {
-                  el_d[o][kk] = make_float2(s2, 0.0f);
-                  el_i[o][kk] = jid;
-                }
-              });
+  auto visit = [&](const float4& pj, uint32_t jid) {
+    if (__float_as_uint(pj.w) != ti) return;        // :219
+    const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
+    const float s2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
+    if (!(s2 < sd.edge_d2)) return;                  // :227
+    if (jid <= idi) return;                          // j > i, :215
+    const uint32_t kk = atomicAdd(&el_n[o], 1u);
+    if (kk < (uint32_t)kListEdges) {
+      el_d[o][kk] = make_float2(s2, 0.0f);
+      el_i[o][kk] = jid;
+    }
+  };
+  if constexpr (ER == 1) {
+    // the owner's nine rows: lane g takes row g, lane 0 also row 8
+    int qa[2], len[2];
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      int c0 = 0, c1 = 0;
+      const int r = g + i * G;
+      const bool on = active && r < 9 && edge_row_fast<ER>(sd, w, cut2, r, c0, c1);
+      qa[i] = on ? (int)a.start[c0] : 0;
+      len[i] = on ? (int)a.start[c1 + 1] : 0;
+    }
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      len[i] -= qa[i];
+      if (g + i * G < 9) el_r[o][g + i * G] = make_uint2((uint32_t)qa[i], (uint32_t)len[i]);
+    }
+    const int mine = len[0] + len[1];
+    if (__any(mine > kEdgeShare)) {
+      // long rows: the owner's lanes share each of them (a lane with a row of its own would
+      // walk it alone while the lanes of the rows out of reach idle)
+      wave_lds_sync();
+      for (int r = 0; r < 9; ++r) {
+        const uint2 e = el_r[o][r];
+        for (uint32_t t0 = (uint32_t)g; t0 < e.y; t0 += kEdgeLoadBatch * G) {
+          float4 pj[kEdgeLoadBatch];
+          uint32_t jid[kEdgeLoadBatch];
+#pragma unroll
+          for (int u = 0; u < kEdgeLoadBatch; ++u) {
+            const uint32_t q = e.x + min(t0 + (uint32_t)(u * G), e.y - 1u);
+            pj[u] = a.pos[q];
+            jid[u] = a.id[q];
+          }
+#pragma unroll
+          for (int u = 0; u < kEdgeLoadBatch; ++u)
+            if (t0 + (uint32_t)(u * G) < e.y) visit(pj[u], jid[u]);
+        }
+      }
+    } else {
+      // short rows: each lane walks its own, kEdgeLoadBatch slots in flight, an index with
+      // its position so that a qualifying candidate waits for no further load
+      for (int x0 = 0; x0 < mine; x0 += kEdgeLoadBatch) {
+        float4 pj[kEdgeLoadBatch];
+        uint32_t jid[kEdgeLoadBatch];
+#pragma unroll
+        for (int u = 0; u < kEdgeLoadBatch; ++u) {
+          const int x = x0 + u;
+          const int q = x < len[0] ? qa[0] + x : qa[1] + (x - len[0]);
+          const bool in = x < mine;
+          pj[u] = in ? a.pos[q] : make_float4(0.0f, 0.0f, 0.0f, -1.0f);
+          jid[u] = in ? a.id[q] : 0u;
+        }
+#pragma unroll
+        for (int u = 0; u < kEdgeLoadBatch; ++u)
+          if (x0 + u < mine) visit(pj[u], jid[u]);
+      }
+    }
+  } else {
+    if (active) edge_walk(a, sd, w, cut2, g, G, nrows, visit);
+  }
   wave_lds_sync();
   const uint32_t n = active ? el_n[o] : 0u;
   const bool fits = n <= (uint32_t)kListEdges;
@@ -1947,36 +2222,60 @@ __device__ __forceinline__ void edges_owner(const EdgeArgs& a, const SimDesc& sd
       }
       if (rank < (uint32_t)maxc) a.estage[(long)idi * a.estride + rank] = ik;
     }
-  if (!active || g != 0) return;
-  uint32_t e;
-  if (fits) {
-    e = (uint32_t)min(min((int)n, cap), maxc);
-  } else {
-    // more candidates than the LDS list holds: exact streaming selection by this lane
-    EdgeAcc ea;
-    ea.q = 0;
-    ea.maxid = 0;
-    ea.maxk = 0;
-    edge_walk<ER>(a, sd, w, cut2, 0, 1, nrows,
-              [&](int, const float4& pj, uint32_t jid) {
-                if (__float_as_uint(pj.w) != ti) return;
-                const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
-                const float s2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-                if (!(s2 < sd.edge_d2)) return;
-                if (jid > idi) edge_push(ea, s2, jid, cap, a.ecand_d2, a.ecand_id, a.P, p);
-              });
-    e = (uint32_t)edge_finish(ea, cap, maxc, a.ecand_d2, a.ecand_id, a.estage, a.P, p, idi,
-                              a.estride);
+  // the other owners: the whole wave takes them one at a time, in the wave's LDS lists
+  uint32_t ovf_e = 0u;
+  unsigned long long left = __ballot(g == 0 && !fits);
+  if (left) wave_lds_sync();  // the fitting owners' reads of el_d, el_i are done
+  while (left) {
+    const int L = __ffsll((long long)left) - 1;
+    left &= left - 1ull;
+    const int so = __builtin_amdgcn_readfirstlane(base + L / G);
+    const float4 me = a.pos[so];
+    const uint32_t myid = a.id[so];
+    WaveSel sel{&el_d[0][0], 0, 0xFFFFFFFFu};
+    if constexpr (ER == 1) {
+      wave_sel_runs<false>(sel, a.pos, a.id, el_r[L / G], 9, me, myid, sd, false, cap, lane);
+    } else {
+      // 64 rows at a time, one per lane, listed in el_i's place
+      uint2* rows = reinterpret_cast<uint2*>(&el_i[0][0]);
+      for (int r0 = 0; r0 < nrows; r0 += kWave) {
+        const int r = r0 + lane;
+        int c0, c1;
+        const int cx = bin_axis(me.x, sd.ihx, sd.nx), cy = bin_axis(me.y, sd.ihy, sd.ny),
+                  cz = bin_axis(me.z, sd.ihz, sd.nz);
+        uint2 e = make_uint2(0u, 0u);
+        if (r < nrows &&
+            edge_row(sd, cx, cy, cz, fminf(fmaxf(me.x * sd.ihx - (float)cx, 0.0f), 1.0f),
+                     fminf(fmaxf(me.y * sd.ihy - (float)cy, 0.0f), 1.0f),
+                     fminf(fmaxf(me.z * sd.ihz - (float)cz, 0.0f), 1.0f), cut2, r, c0, c1)) {
+          e.x = a.start[c0];
+          e.y = a.start[c1 + 1] - e.x;
+        }
+        wave_lds_sync();
+        rows[lane] = e;
+        wave_lds_sync();
+        wave_sel_runs<false>(sel, a.pos, a.id, rows, min(kWave, nrows - r0), me, myid, sd, false,
+                             cap, lane);
+      }
+    }
+    const uint32_t e = wave_sel_finish(sel, cap, maxc, a.estage + (long)myid * a.estride, lane);
+    if (lane == L) ovf_e = e;
   }
+  if (!active || g != 0) return;
+  const uint32_t e = fits ? (uint32_t)min(min((int)n, cap), maxc) : ovf_e;
   if (e) a.ecount[idi] = e;  // zero already: the edge tiles that read the counts clear them
 }
 
-__global__ void __launch_bounds__(256) k_edges_g(EdgeArgs a) {
+template <int ER>
+__device__ __forceinline__ void edges_body(const EdgeArgs& a) {
   constexpr int G = kEdgeLanes;
   constexpr int kOwn = kWave / G;
+  static_assert(kOwn * kListEdges >= kSelCap, "the wave selection's list fits el_d");
+  static_assert(kOwn * kListEdges >= 2 * kWave, "64 rows fit el_i");
   __shared__ float2 el_d[4][kOwn][kListEdges];
-  __shared__ uint32_t el_i[4][kOwn][kListEdges];
+  __shared__ __align__(8) uint32_t el_i[4][kOwn][kListEdges];
   __shared__ uint32_t el_n[4][kOwn];
+  __shared__ uint2 el_r[4][kOwn][ER == 1 ? kEdgeRuns : 1];
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int gw = xcd_block() * (blockDim.x >> 6) + wv;
@@ -1993,11 +2292,14 @@ __global__ void __launch_bounds__(256) k_edges_g(EdgeArgs a) {
     pi = a.pos[p];
     idi = a.id[p];
   }
-  if (sd.edge_rx == 1 && sd.edge_ry == 1 && sd.edge_rz == 1)
-    edges_owner<1>(a, sd, wv, o, g, p, active, pi, idi, el_d[wv], el_i[wv], el_n[wv]);
-  else
-    edges_owner<0>(a, sd, wv, o, g, p, active, pi, idi, el_d[wv], el_i[wv], el_n[wv]);
+  edges_owner<ER>(a, sd, o, g, lane, (int)base, active, pi, idi, el_d[wv], el_i[wv], el_n[wv],
+                  el_r[wv]);
 }
+
+// Edge distances within one cell on every axis (8 waves per SIMD; the other kernel's row
+// walk takes more registers), and any distance.
+__global__ void __launch_bounds__(256) k_edges_g(EdgeArgs a) { edges_body<1>(a); }
+__global__ void __launch_bounds__(256) k_edges_far(EdgeArgs a) { edges_body<0>(a); }
 
 // ------------------------------------------------------------------------------------
 // k_tile_sort: the (cell, index) sort of one step, and the step's canonical edge list.
@@ -3048,8 +3350,34 @@ static void launch_cons(const ForceArgs& a, bool edges, hipStream_t st) {
   }
 }
 
+template <int R, int G>
+static void launch_ord(const ForceArgs& a, bool edges, hipStream_t st) {
+  const long waves = (long)a.nwaves * G;  // one wave per 64/G particle slots
+  const dim3 g((unsigned)((waves + 3) / 4)), b(256);
+  if (a.hits) {
+    if (a.tile_sort) CF_LAUNCH((k_force_ord<false, R, G, true, true>), g, b, 0, st, a);
+    else CF_LAUNCH((k_force_ord<false, R, G, false, true>), g, b, 0, st, a);
+  } else if (a.tile_sort) {
+    if (edges) CF_LAUNCH((k_force_ord<true, R, G, true>), g, b, 0, st, a);
+    else CF_LAUNCH((k_force_ord<false, R, G, true>), g, b, 0, st, a);
+  } else {
+    if (edges) CF_LAUNCH((k_force_ord<true, R, G, false>), g, b, 0, st, a);
+    else CF_LAUNCH((k_force_ord<false, R, G, false>), g, b, 0, st, a);
+  }
+}
+
 hipError_t launch_force(const ForceArgs& a, bool edges, int block, int variant, int reach,
                         int lanes, hipStream_t st) {
+  // Variant 0 at 16 lanes: k_force_ord while slots fit a list entry, else k_force_grp.  8
+  // lanes per particle issue fewer instructions, 16 give twice the waves: below 28k slots
+  // 8 lanes leave under 3.5 waves per SIMD (20k particles: 7.7 us against 7.1; 37k: 9.3
+  // against 10.3).  The 125-cell stencil's 25 rows need 16 lanes at two rows each.
+  if (variant == 0 && lanes == 16 && a.P <= (1L << kCodeShift)) {
+    if (reach == 2) launch_ord<2, 16>(a, edges, st);
+    else if (a.P < 28672) launch_ord<1, 16>(a, edges, st);
+    else launch_ord<1, 8>(a, edges, st);
+    return hipGetLastError();
+  }
   if (a.hits && (variant != 0 || edges)) return hipErrorInvalidValue;  // lists: variant 0 only
   if (variant == 0) {
     if (reach == 1) {
@@ -3115,9 +3443,11 @@ hipError_t launch_force(const ForceArgs& a, bool edges, int block, int variant, 
   return hipGetLastError();
 }
 
-hipError_t launch_edges(const EdgeArgs& a, hipStream_t st) {
+hipError_t launch_edges(const EdgeArgs& a, bool near, hipStream_t st) {
   // kWave / kEdgeLanes owners per wave, four waves per block
-  CF_LAUNCH(k_edges_g, dim3((a.nwaves * kEdgeLanes + 3) / 4), dim3(256), 0, st, a);
+  const dim3 g((a.nwaves * kEdgeLanes + 3) / 4), b(256);
+  if (near) CF_LAUNCH(k_edges_g, g, b, 0, st, a);
+  else CF_LAUNCH(k_edges_far, g, b, 0, st, a);
   return hipGetLastError();
 }
 
