@@ -229,6 +229,7 @@ struct Engine {
 
   uint32_t* tile_sim = nullptr;
   int ntiles = 0, ntiles_cap = 0, netiles = 0;
+  int nhelp = 0;   // helper blocks of the tile sort
   // set only while the gradient rollout steps: where the force kernel lists the step's
   // in-range partners (ForceArgs::hits)
   uint32_t* fhits = nullptr;
@@ -443,10 +444,11 @@ struct Engine {
       d.edge_rx = re[0];
       d.edge_ry = re[1];
       d.edge_rz = re[2];
-      // cell tiles: tr rows of one plane, about kTileTarget particles at this density
+      // cell tiles: tr rows of one plane, about `target` particles at this density
+      const double target = (double)std::min<long>(kTileMax, std::max<long>(kTileMin, P / kTileBlocks));
       const double occ = (double)std::max(h.n, 1) / (double)d.ncells;
       const int trmax = std::max(1, std::min(d.ny, kTileCells / d.nx));
-      d.tr = (int)std::max(1.0, std::min((double)trmax, std::floor(kTileTarget / (d.nx * occ))));
+      d.tr = (int)std::max(1.0, std::min((double)trmax, std::floor(target / (d.nx * occ))));
       d.nyt = (d.ny + d.tr - 1) / d.tr;
       d.t0 = nt;
       nt += d.nz * d.nyt;
@@ -480,6 +482,8 @@ struct Engine {
       ntiles_cap = nt;
     }
     ntiles = nt;
+    // crowded tiles have at most P / kTilePart parts beyond their first
+    nhelp = (int)std::min<long>(kMaxHelp, P / kTilePart);
     htile_sim.assign(nt, 0u);
     for (size_t s2 = 0; s2 < hdesc.size(); ++s2)
       for (int t = 0; t < hdesc[s2].nz * hdesc[s2].nyt; ++t) htile_sim[hdesc[s2].t0 + t] = (uint32_t)s2;
@@ -762,6 +766,7 @@ struct Engine {
     ta.ftl = ftl;
     ta.flag = b.flag;
     ta.ntiles = ntiles;
+    ta.nhelp = nhelp;
     if (edges) {
       ta.ecount = b.fcount;
       ta.eticket = eticket;

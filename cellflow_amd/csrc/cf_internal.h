@@ -20,9 +20,18 @@ constexpr int kMaxEdgeCap = 64;        // 2 * CF_MAX_CONNECTIONS
 // step, in the tile's window (the tile's rows and one row either side, in the tile's plane
 // and one plane either side, cyclically), unless it is a far mover: those carry kFarBit
 // in their key and are listed apart.
-constexpr int kTileCells = 2048;       // most cells in one tile (tr * nx)
-constexpr int kTileCap = 2048;         // members a tile sorts in LDS at once
-constexpr int kTileTarget = 384;       // expected members of a tile (chooses tr)
+constexpr int kTileCells = 1024;       // most cells in one tile (tr * nx; nx <= 1024)
+constexpr int kTileCap = 1024;         // members a block sorts in LDS at once
+constexpr int kMaxHelp = 512;          // helper blocks that take the parts beyond a tile's first
+constexpr int kTilePart = 512;         // members per block of a tile with more than kTileCap
+// Expected members of a tile (chooses tr): the particles over kTileBlocks, so that one round
+// of blocks covers the chip, within kTileMin (smaller tiles read more window than members)
+// and kTileMax (a tile of more than kTileCap is shared; 768 expected leaves 9 deviations).
+// us per sort at 192 / 256 / 384 / 512 / 768: 37k 5.8 / 6.1 / 6.3 / 6.9 / 7.9; 100k 8.5 / 7.7
+// / 7.8 / 7.7 / 8.5; 200k 18.8 / 15.2 / 10.1 / 9.1 / 10.3; 500k 103 / 41 / 28 / 21 / 15.
+constexpr int kTileBlocks = 390;
+constexpr int kTileMin = 192;
+constexpr int kTileMax = 768;
 constexpr int kEdgeTile = 1024;        // owner ids per edge tile
 // The list force kernels (variants 3 and 4) keep each candidate as slot | image-shift code
 // << kCodeShift in LDS, so they take at most 2^kCodeShift slots.
@@ -260,6 +269,7 @@ struct TileSortArgs {
   long edge_room;                       // entries `edges` holds
   const uint32_t* __restrict__ wave_sim;
   int netiles;
+  int nhelp;        // blocks for the parts of tiles with more than kTileCap members
   long P;
   int one_sim;                          // one simulation: tile_sim is all zero
 };

@@ -102,6 +102,11 @@ __device__ __forceinline__ void wave_lds_sync() {
   __builtin_amdgcn_wave_barrier();
 }
 
+// A value that is the same in every lane, in a scalar register.
+__device__ __forceinline__ uint32_t uniform(uint32_t v) {
+  return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
+
 __device__ __forceinline__ uint32_t wave_inclusive_scan(uint32_t v, int lane) {
 #pragma unroll
   for (int d = 1; d < kWave; d <<= 1) {
@@ -2313,10 +2318,22 @@ __global__ void __launch_bounds__(256) k_edges_far(EdgeArgs a) { edges_body<0>(a
 // in.  An edge tile writes its owners' edges at the sum of the counts of the edge tiles
 // before it (a decoupled look-back) plus a local scan.  Each cell-tile block also clears its
 // own counters for the next step (the next step counts into the other parity).
+//
+// The host sizes tiles by the mean density, so where particles crowd together a tile holds
+// many times its share.  A tile with more than kTileCap members is shared by one block per
+// kTilePart of them: its own block and helper blocks, which find the parts beyond the first
+// from the counts alone (none, normally: they end after one load).  Every part counts the
+// whole tile, then sorts the cells that begin in its share.
+//
+// Bound: latency, a chain of about five dependent loads per block.  Blocks of 512 threads
+// with 26 KB of LDS (three per CU) and tiles of P / 390 particles put one round of blocks on
+// the chip: before (256 threads, 66 KB, tiles of 384 at any size) 37k took 7.4 us, 100k 8.6
+// and 11.1 with the graph, 200k 15.5, 500k 33.2, 20k of a preset (everything in a few
+// tiles) 148; now 5.8, 7.7 and 8.3, 9.0, 14.8, 20.5.
 
-constexpr int kSortThreads = 256;
-constexpr int kVisitBatch = 8;  // window slots per thread with their loads in flight together
-constexpr int kMoveBatch = 4;   // members per thread moved together
+constexpr int kSortThreads = 512;
+constexpr int kVisitBatch = 4;  // window slots per thread with their loads in flight together
+constexpr int kMoveBatch = 2;   // members per thread moved together
 
 // Flag word of a look-back tile: launch epoch (30 bits), status (0 none, 1 the tile's own
 // sum, 2 the inclusive prefix), value.
@@ -2524,31 +2541,53 @@ __device__ void edge_tile(const TileSortArgs& a, uint32_t* red, uint32_t* toff, 
   }
 }
 
-__global__ void __launch_bounds__(kSortThreads) k_tile_sort(TileSortArgs a) {
+// Blocks that share a tile with `members` members.
+__device__ __forceinline__ uint32_t tile_parts(uint32_t members) {
+  return members <= (uint32_t)kTileCap ? 1u : (members + (uint32_t)kTilePart - 1u) / (uint32_t)kTilePart;
+}
+
+// How many of the n indices in LDS are below `me`.
+constexpr uint32_t kRankBatch = 8;
+__device__ __forceinline__ uint32_t rank_in(const uint32_t* ids, uint32_t n, uint32_t me) {
+  uint32_t rank = 0, e = 0;
+  for (; e + kRankBatch <= n; e += kRankBatch) {
+    uint32_t v[kRankBatch];
+#pragma unroll
+    for (uint32_t u = 0; u < kRankBatch; ++u) v[u] = ids[e + u];
+#pragma unroll
+    for (uint32_t u = 0; u < kRankBatch; ++u) rank += (v[u] < me) ? 1u : 0u;
+  }
+  for (; e < n; ++e) rank += (ids[e] < me) ? 1u : 0u;
+  return rank;
+}
+
+// 80 VGPRs and 26 KB of LDS: three blocks of eight waves per CU.
+__global__ void __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(6, 8)))
+k_tile_sort(TileSortArgs a) {
   __shared__ uint32_t cnt_s[kTileCells];
   __shared__ uint32_t cofs[kTileCells + 1];
   __shared__ uint32_t fill_s[kTileCells];
-  __shared__ uint32_t mslot[kTileCap];
-  __shared__ uint32_t mid[kTileCap];
-  __shared__ uint16_t mlc[kTileCap];
-  __shared__ uint32_t aq[kTileCap];  // members in visit order (slot, index, local cell)
+  __shared__ uint32_t mid[kTileCap];  // the members' indices grouped by cell
+  // the members in visit order (slot, index, local cell)
+  __shared__ uint32_t aq[kTileCap];
   __shared__ uint32_t aid[kTileCap];
   __shared__ uint16_t alc[kTileCap];
   __shared__ uint32_t red[3 * (kSortThreads / kWave)];
   __shared__ uint32_t wq0[6], wq1[6];  // the window's slot runs
-  __shared__ int s_next;
+  __shared__ int s_next, s_ia, s_ib, s_tile, s_part;
   __shared__ uint32_t s_app;
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
-  if ((int)blockIdx.x >= a.ntiles) {
+  if ((int)blockIdx.x >= a.ntiles && (int)blockIdx.x < a.ntiles + a.netiles) {
     static_assert(kTileCells >= kEdgeTile && kTileCells >= kSortThreads, "edge tile scratch");
     edge_tile(a, red, cofs, fill_s, cnt_s);
     return;
   }
-  // consecutive tiles (consecutive slots) share an XCD, as in the force pass
-  const int t = xcd_map((int)blockIdx.x, a.ntiles);
+
+  // part `part` of the cells of tile t
+  auto sort_part = [&](const int t, const int part) {
   const SimDesc& sd = a.sims[a.one_sim ? 0 : (int)a.tile_sim[t]];
-  if (tid == 0) {
+  if (tid == 0 && part == 0) {
     a.tcount_next[t * kCtrStride] = 0u;
     a.ftn_next[t * kCtrStride] = 0u;
     if (t == 0) *a.far_n_next = 0u;
@@ -2577,8 +2616,8 @@ __global__ void __launch_bounds__(kSortThreads) k_tile_sort(TileSortArgs a) {
   }
 
   // the far lists' lengths do not depend on anything below either
-  const uint32_t nfar_t = min(a.ftn[t * kCtrStride], (uint32_t)kFarCap);
-  const uint32_t nfar = min(*a.far_n, (uint32_t)a.P);
+  const uint32_t nfar_t = uniform(min(a.ftn[t * kCtrStride], (uint32_t)kFarCap));
+  const uint32_t nfar = uniform(min(*a.far_n, (uint32_t)a.P));
 
   // fn(valid, q, key, id) for every slot of the window and of the far lists, called by
   // every lane of the block the same number of times (valid: a slot whose key is not a far
@@ -2588,10 +2627,13 @@ __global__ void __launch_bounds__(kSortThreads) k_tile_sort(TileSortArgs a) {
   // with all their loads in flight before any is used; fn's order does not matter (ranks
   // are by index).
   auto visit = [&](auto&& fn) {
-    uint32_t wp[7];
+    uint32_t wp[7], w0[6];
     wp[0] = 0u;
 #pragma unroll
-    for (int g = 0; g < 6; ++g) wp[g + 1] = wp[g] + (wq1[g] - wq0[g]);
+    for (int g = 0; g < 6; ++g) {
+      w0[g] = uniform(wq0[g]);
+      wp[g + 1] = wp[g] + (uniform(wq1[g]) - w0[g]);
+    }
     const uint32_t nw = wp[6];
     for (uint32_t b = 0; b < nw; b += kVisitBatch * kSortThreads) {
       uint32_t qv[kVisitBatch], kv[kVisitBatch], iv[kVisitBatch];
@@ -2602,10 +2644,10 @@ __global__ void __launch_bounds__(kSortThreads) k_tile_sort(TileSortArgs a) {
         kv[u] = kFarBit;  // nothing to visit
         iv[u] = 0u;
         if (i < nw) {
-          uint32_t q = wq0[0] + i;
+          uint32_t q = w0[0] + i;
 #pragma unroll
           for (int g = 1; g < 6; ++g)
-            if (i >= wp[g]) q = wq0[g] + (i - wp[g]);  // an empty run gives way to the next
+            if (i >= wp[g]) q = w0[g] + (i - wp[g]);  // an empty run gives way to the next
           qv[u] = q;
           kv[u] = a.key[q];
           iv[u] = a.src_id[q];
@@ -2637,22 +2679,40 @@ __global__ void __launch_bounds__(kSortThreads) k_tile_sort(TileSortArgs a) {
   };
 
   // The tile's cell counts come from its members.  Normally (the force pass counted at most
-  // kTileCap particles into the tile) one visit appends the members to LDS, a wave's
-  // members at one LDS atomic, and counts them per cell; else a visit only counts, and the
-  // cells are then sorted a chunk at a time below.
-  uint32_t part = 0;  // the particles of the simulation's tiles before this one
-  for (int u = sd.t0 + tid; u < t; u += kSortThreads) part += a.tcount[u * kCtrStride];
-  const uint32_t expect = a.tcount[t * kCtrStride];
+  // kTileCap particles into the tile) one visit appends the members to LDS, a wave's members
+  // at one LDS atomic, and counts them per cell.  Else the tile is shared: the first visit
+  // only counts, and each part's later visits append the members of its own cells, as many
+  // cells at a time as kTileCap members allow.
+  uint32_t ahead = 0;  // the particles of the simulation's tiles before this one
+  for (int u = sd.t0 + tid; u < t; u += kSortThreads) ahead += a.tcount[u * kCtrStride];
+  const uint32_t expect = uniform(a.tcount[t * kCtrStride]);
   for (int i = tid; i < nc; i += kSortThreads) {
     cnt_s[i] = 0u;
     fill_s[i] = 0u;
   }
-  if (tid == 0) s_app = 0u;
+  if (tid == 0) {
+    s_app = 0u;
+    s_ia = nc;
+    s_ib = 0;
+  }
   __syncthreads();
   const bool placed = expect <= (uint32_t)kTileCap;  // the same for the whole block
-  if (placed) {
+  // the members must be what the force pass counted into the tile (and the simulation's
+  // last tile must end at its last particle); if not, the tile writes nothing but clamped
+  // starts, and the call fails
+  const uint32_t lim = (uint32_t)(sd.p0 + sd.n);
+  const bool last = lt == sd.nz * sd.nyt - 1;
+  uint32_t base = 0u;  // the tile's first slot
+  // The members of cells [ia, ib) into LDS (append) and, with count, into their cells' counts.
+  auto collect = [&](int ia, int ib, auto count_kind, auto append_kind) {
+    constexpr bool kCount = decltype(count_kind)::value, kAppend = decltype(append_kind)::value;
+    const uint32_t ca = cA + (uint32_t)ia, cn = (uint32_t)(ib - ia);
     visit([&](bool valid, uint32_t q, uint32_t k, uint32_t id) {
-      const bool mem = valid && k >= cA && k - cA < (uint32_t)nc;
+      const bool mem = valid && k >= ca && k - ca < cn;
+      if constexpr (!kAppend) {
+        if (mem) atomicAdd(&cnt_s[k - cA], 1u);
+        return;
+      }
       const unsigned long long bal = __ballot(mem);
       if (bal == 0ull) return;
       const int lead = __ffsll((long long)bal) - 1;
@@ -2662,7 +2722,7 @@ __global__ void __launch_bounds__(kSortThreads) k_tile_sort(TileSortArgs a) {
       if (mem) {
         const uint32_t j = b0 + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull));
         const uint32_t lc = k - cA;
-        atomicAdd(&cnt_s[lc], 1u);
+        if (kCount) atomicAdd(&cnt_s[lc], 1u);
         if (j < (uint32_t)kTileCap) {
           aq[j] = q;
           aid[j] = id;
@@ -2670,171 +2730,124 @@ __global__ void __launch_bounds__(kSortThreads) k_tile_sort(TileSortArgs a) {
         }
       }
     });
-  } else {
-    visit([&](bool valid, uint32_t, uint32_t k, uint32_t) {
-      if (valid && k >= cA && k - cA < (uint32_t)nc) atomicAdd(&cnt_s[k - cA], 1u);
-    });
-  }
-  __syncthreads();
-
-  // A tile of at most kMoveBatch * kSortThreads appended members loads their states now,
-  // entry m = u * kSortThreads + tid by thread tid: the loads are in flight during the
-  // scan and the grouping below, and the same thread then moves them.
-  const uint32_t napp = placed ? s_app : 0u;
-  const bool preload = placed && napp <= (uint32_t)(kMoveBatch * kSortThreads);
+    __syncthreads();
+  };
+  // The appended members' states, entry m = u * kSortThreads + tid by thread tid: loaded
+  // before the scan and the grouping below, so in flight during them; the same thread then
+  // moves them.
+  static_assert(kTileCap == kMoveBatch * kSortThreads, "a thread's members fit its registers");
   float4 psp[kMoveBatch], psv[kMoveBatch];
+  auto preload = [&](uint32_t napp) {
 #pragma unroll
-  for (int u = 0; u < kMoveBatch; ++u) {
-    const uint32_t m = (uint32_t)(u * kSortThreads + tid);
-    psp[u] = psv[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-    if (preload && m < napp) {
-      psp[u] = a.src_pos[aq[m]];
-      psv[u] = a.src_vel[aq[m]];
+    for (int u = 0; u < kMoveBatch; ++u) {
+      const uint32_t m = (uint32_t)(u * kSortThreads + tid);
+      psp[u] = psv[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      if (m < napp) {
+        psp[u] = a.src_pos[aq[m]];
+        psv[u] = a.src_vel[aq[m]];
+      }
     }
-  }
-
-  // first slot of the tile, then its cells' starts
-  const int per = (nc + kSortThreads - 1) / kSortThreads;
-  const int i0 = min(tid * per, nc), i1 = min(i0 + per, nc);
-  uint32_t run = 0;
-  for (int i = i0; i < i1; ++i) run += cnt_s[i];
-  uint32_t before, unused, pre, M;
-  block_sums_excl_u32(part, 0u, run, red, before, unused, pre, M);
-  const uint32_t base = (uint32_t)sd.p0 + before;
-  // The members must be what the force pass counted into the tile (and the simulation's
-  // last tile must end at its last particle); if not, the tile writes nothing but clamped
-  // starts, and the call fails.
-  const uint32_t lim = (uint32_t)(sd.p0 + sd.n);
-  const bool last = lt == sd.nz * sd.nyt - 1;
-  const bool ok = M == expect && base + M <= lim && (!last || base + M == lim);
-  for (int i = i0; i < i1; ++i) {
-    cofs[i] = pre;
-    a.start_new[cA + i] = min(base + pre, lim);
-    pre += cnt_s[i];
-  }
-  if (tid == 0) {
-    cofs[nc] = M;
-    if (!ok) atomicOr(a.flag, 4u);
-    if (last) {  // the simulation's pad cell, and the start of what follows it
-      a.start_new[sd.c0 + sd.ncells] = lim;
-      a.start_new[sd.c0 + sd.ncells + 1] =
-          (uint32_t)(sd.p0 + (sd.n + kSlotAlign - 1) / kSlotAlign * kSlotAlign);
+  };
+  // The tile's first slot and its cells' starts; false: the members found are not those the
+  // force pass counted.
+  auto starts = [&]() {
+    const int per = (nc + kSortThreads - 1) / kSortThreads;
+    const int i0 = min(tid * per, nc), i1 = min(i0 + per, nc);
+    uint32_t run = 0;
+    for (int i = i0; i < i1; ++i) run += cnt_s[i];
+    uint32_t before, unused, pre, M;
+    block_sums_excl_u32(ahead, 0u, run, red, before, unused, pre, M);
+    M = uniform(M);
+    base = (uint32_t)sd.p0 + uniform(before);
+    const bool ok = M == expect && base + M <= lim && (!last || base + M == lim);
+    if (placed) {
+      for (int i = i0; i < i1; ++i) {
+        cofs[i] = pre;
+        a.start_new[cA + i] = min(base + pre, lim);
+        pre += cnt_s[i];
+      }
+    } else {
+      // this part's cells: those whose first member lies in its share of the tile's members
+      // (trailing empty cells go to the last part)
+      const int parts = (int)tile_parts(expect);
+      const uint32_t share = max((M + (uint32_t)parts - 1u) / (uint32_t)parts, 1u);
+      for (int i = i0; i < i1; ++i) {
+        cofs[i] = pre;
+        if (min((int)(pre / share), parts - 1) == part) {
+          a.start_new[cA + i] = min(base + pre, lim);
+          atomicMin(&s_ia, i);
+          atomicMax(&s_ib, i + 1);
+        }
+        pre += cnt_s[i];
+      }
     }
-  }
-  __syncthreads();
-  if (!ok) return;
-  if (placed) {  // group the appended members by cell (M == expect <= kTileCap: all kept)
-    for (uint32_t m = tid; m < M; m += kSortThreads) {
+    if (tid == 0) {
+      cofs[nc] = M;
+      if (!ok) atomicOr(a.flag, 4u);
+      if (last && part == 0) {  // the simulation's pad cell, and the start of what follows it
+        a.start_new[sd.c0 + sd.ncells] = lim;
+        a.start_new[sd.c0 + sd.ncells + 1] =
+            (uint32_t)(sd.p0 + (sd.n + kSlotAlign - 1) / kSlotAlign * kSlotAlign);
+      }
+    }
+    __syncthreads();
+    return ok;
+  };
+  // Groups the napp appended members' indices by cell (m0: the tile's members before them),
+  // then ranks each by index inside its cell and moves it.
+  auto place = [&](uint32_t napp, uint32_t m0) {
+    for (uint32_t m = tid; m < napp; m += kSortThreads) {
       const uint32_t lc = alc[m];
-      const uint32_t at = cofs[lc] + atomicAdd(&fill_s[lc], 1u);
-      mslot[at] = aq[m];
-      mid[at] = aid[m];
-      mlc[at] = (uint16_t)lc;
+      mid[cofs[lc] - m0 + atomicAdd(&fill_s[lc], 1u)] = aid[m];
     }
-  }
-  if (preload) {  // rank each preloaded member by index inside its cell and move it
     __syncthreads();
 #pragma unroll
     for (int u = 0; u < kMoveBatch; ++u) {
       const uint32_t m = (uint32_t)(u * kSortThreads + tid);
-      if (m < M) {
+      if (m < napp) {
         const uint32_t lc = alc[m], me = aid[m];
-        const uint32_t s0 = cofs[lc], sn = cnt_s[lc];
-        uint32_t rank = 0;
-        for (uint32_t e = 0; e < sn; ++e) rank += (mid[s0 + e] < me) ? 1u : 0u;
-        const uint32_t dst = base + s0 + rank;
+        const uint32_t s0 = cofs[lc];
+        const uint32_t dst = base + s0 + rank_in(mid + (s0 - m0), cnt_s[lc], me);
         a.dst_pos[dst] = psp[u];
         a.dst_vel[dst] = psv[u];
         a.dst_id[dst] = me;
       }
     }
+  };
+  if (placed) {
+    collect(0, nc, std::true_type{}, std::true_type{});
+    const uint32_t napp = min(uniform(s_app), (uint32_t)kTileCap);
+    preload(napp);
+    if (starts()) place(napp, 0u);  // M == expect <= kTileCap: all were kept
     return;
   }
-
-  // cells [ia, ib) at a time, as many as kTileCap members allow (all of them, normally)
-  int ia = 0;
-  while (ia < nc) {
-    int ib = nc;  // every member fits (the normal case): no search
-    if (M - cofs[ia] > (uint32_t)kTileCap) {
+  collect(0, nc, std::true_type{}, std::false_type{});
+  if (!starts()) return;
+  const int iend = (int)uniform((uint32_t)s_ib);
+  int ia = 0, ib = (int)uniform((uint32_t)s_ia);
+  while (true) {
+    // the part's next cells, as many as kTileCap members allow; a cell with more is sorted
+    // here through global scratch at its own slot range
+    while (true) {
+      ia = ib;
+      if (ia >= iend) return;
+      __syncthreads();  // the LDS lists are reused
       if (tid == 0) {
-        int lo = ia + 1, hi = nc;
+        int lo = ia + 1, hi = iend;
         while (lo < hi) {
           const int m = (lo + hi + 1) >> 1;
           if (cofs[m] - cofs[ia] <= (uint32_t)kTileCap) lo = m;
           else hi = m - 1;
         }
         s_next = lo;
+        s_app = 0u;
       }
       __syncthreads();
-      ib = s_next;
-    }
-    const uint32_t m0 = cofs[ia], mn = cofs[ib] - m0;
-    if (mn <= (uint32_t)kTileCap) {
-      if (!placed) {
-        for (int i = ia + tid; i < ib; i += kSortThreads) fill_s[i] = 0u;
-        for (uint32_t m = tid; m < mn; m += kSortThreads) mlc[m] = 0xFFFFu;
-        __syncthreads();
-        const uint32_t ca = cA + (uint32_t)ia, cb = cA + (uint32_t)ib;
-        visit([&](bool valid, uint32_t q, uint32_t k, uint32_t id) {
-          if (!valid || k < ca || k >= cb) return;
-          const uint32_t lc = k - cA;
-          const uint32_t at = atomicAdd(&fill_s[lc], 1u);
-          if (at >= cnt_s[lc]) {
-            atomicOr(a.flag, 4u);
-            return;
-          }
-          const uint32_t m = cofs[lc] - m0 + at;
-          mslot[m] = q;
-          mid[m] = id;
-          mlc[m] = (uint16_t)lc;
-        });
-      }
-      __syncthreads();
-      // kMoveBatch members per thread: their state loads are in flight during the ranking
-      for (uint32_t mb = 0; mb < mn; mb += kMoveBatch * kSortThreads) {
-        float4 sp[kMoveBatch], sv[kMoveBatch];
-        uint32_t lcv[kMoveBatch];
-#pragma unroll
-        for (int u = 0; u < kMoveBatch; ++u) {
-          const uint32_t m = mb + (uint32_t)(u * kSortThreads + tid);
-          lcv[u] = 0xFFFFu;
-          sp[u] = sv[u] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-          if (m < mn) {
-            const uint32_t lc = mlc[m];
-            if (lc >= (uint32_t)nc || fill_s[lc] != cnt_s[lc]) {
-              atomicOr(a.flag, 4u);  // a cell lost a particle: leave its slots alone
-            } else {
-              const uint32_t q = mslot[m];
-              sp[u] = a.src_pos[q];
-              sv[u] = a.src_vel[q];
-              lcv[u] = lc;
-            }
-          }
-        }
-#pragma unroll
-        for (int u = 0; u < kMoveBatch; ++u) {
-          const uint32_t lc = lcv[u];
-          if (lc != 0xFFFFu) {
-            const uint32_t m = mb + (uint32_t)(u * kSortThreads + tid);
-            const uint32_t s0 = cofs[lc] - m0, sn = cnt_s[lc], me = mid[m];
-            uint32_t rank = 0;
-            for (uint32_t e = 0; e < sn; ++e) rank += (mid[s0 + e] < me) ? 1u : 0u;
-            const uint32_t dst = base + cofs[lc] + rank;
-            a.dst_pos[dst] = sp[u];
-            a.dst_vel[dst] = sv[u];
-            a.dst_id[dst] = me;
-          }
-        }
-      }
-    } else {
-      // one cell (ib == ia + 1) holds more than the LDS takes: its ids and slots go to
-      // global scratch at the cell's own slot range, ranks by a pass over all of them
-      const uint32_t K = cnt_s[ia], g0 = base + cofs[ia], cg = cA + (uint32_t)ia;
-      if (tid == 0) {
-        fill_s[ia] = 0u;
-        atomicOr(a.flag, 2u);
-      }
-      __syncthreads();
+      ib = (int)uniform((uint32_t)s_next);
+      const uint32_t K = uniform(cnt_s[ia]);
+      if (K <= (uint32_t)kTileCap) break;
+      const uint32_t g0 = base + uniform(cofs[ia]), cg = cA + (uint32_t)ia;
+      if (tid == 0) atomicOr(a.flag, 2u);
       visit([&](bool valid, uint32_t q, uint32_t k, uint32_t id) {
         if (!valid || k != cg) return;
         const uint32_t at = atomicAdd(&fill_s[ia], 1u);
@@ -2846,22 +2859,86 @@ __global__ void __launch_bounds__(kSortThreads) k_tile_sort(TileSortArgs a) {
         a.tmp_slot[g0 + at] = q;
       });
       __syncthreads();
-      if (fill_s[ia] == K) {
-        for (uint32_t m = tid; m < K; m += kSortThreads) {
-          const uint32_t me = a.tmp_id[g0 + m];
-          uint32_t rank = 0;
-          for (uint32_t e = 0; e < K; ++e) rank += (a.tmp_id[g0 + e] < me) ? 1u : 0u;
-          const uint32_t q = a.tmp_slot[g0 + m];
-          a.dst_pos[g0 + rank] = a.src_pos[q];
-          a.dst_vel[g0 + rank] = a.src_vel[q];
-          a.dst_id[g0 + rank] = me;
+      if (uniform(fill_s[ia]) != K) {
+        if (tid == 0) atomicOr(a.flag, 4u);
+        return;
+      }
+      // kMoveBatch members per thread at a time; the ids pass through LDS, kTileCap at a time
+      for (uint32_t mb = 0; mb < K; mb += kMoveBatch * kSortThreads) {
+        uint32_t me[kMoveBatch], rank[kMoveBatch];
+#pragma unroll
+        for (int u = 0; u < kMoveBatch; ++u) {
+          const uint32_t m = mb + (uint32_t)(u * kSortThreads + tid);
+          me[u] = m < K ? a.tmp_id[g0 + m] : 0u;
+          rank[u] = 0u;
         }
-      } else if (tid == 0) {
-        atomicOr(a.flag, 4u);
+        for (uint32_t c0 = 0; c0 < K; c0 += kTileCap) {
+          const uint32_t cl = min((uint32_t)kTileCap, K - c0);
+          __syncthreads();
+          for (uint32_t m = tid; m < cl; m += kSortThreads) mid[m] = a.tmp_id[g0 + c0 + m];
+          __syncthreads();
+          for (uint32_t e = 0; e < cl; ++e) {
+            const uint32_t v = mid[e];
+#pragma unroll
+            for (int u = 0; u < kMoveBatch; ++u) rank[u] += (v < me[u]) ? 1u : 0u;
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kMoveBatch; ++u) {
+          const uint32_t m = mb + (uint32_t)(u * kSortThreads + tid);
+          if (m < K) {
+            const uint32_t q = a.tmp_slot[g0 + m];
+            a.dst_pos[g0 + rank[u]] = a.src_pos[q];
+            a.dst_vel[g0 + rank[u]] = a.src_vel[q];
+            a.dst_id[g0 + rank[u]] = me[u];
+          }
+        }
       }
     }
-    __syncthreads();  // the LDS lists are reused by the next cells
-    ia = ib;
+    collect(ia, ib, std::false_type{}, std::true_type{});
+    const uint32_t m0 = uniform(cofs[ia]), napp = uniform(s_app);
+    if (napp != uniform(cofs[ib]) - m0) {  // a particle was lost: leave its slots alone
+      if (tid == 0) atomicOr(a.flag, 4u);
+      return;
+    }
+    preload(napp);
+    place(napp, m0);
+  }
+  };
+
+  // a tile's block takes the tile's first part; a helper takes parts 1, 2, ... of the tiles
+  // with more than kTileCap members, in tile order, every a.nhelp-th of them
+  const bool helper = (int)blockIdx.x >= a.ntiles;
+  uint32_t mine = 0u, pre = 0u, total = 1u, j = 0u;
+  const int per = (a.ntiles + kSortThreads - 1) / kSortThreads;
+  const int u0 = min(tid * per, a.ntiles), u1 = min(u0 + per, a.ntiles);
+  if (helper) {
+    for (int u = u0; u < u1; ++u) mine += tile_parts(a.tcount[u * kCtrStride]) - 1u;
+    uint32_t un0, un1;
+    block_sums_excl_u32(0u, 0u, mine, red, un0, un1, pre, total);
+    j = blockIdx.x - (uint32_t)(a.ntiles + a.netiles);
+  }
+  for (; j < total; j += (uint32_t)max(a.nhelp, 1)) {
+    // consecutive tiles (consecutive slots) share an XCD, as in the force pass
+    int t = xcd_map((int)blockIdx.x, a.ntiles), part = 0;
+    if (helper) {
+      if (j >= pre && j < pre + mine) {
+        uint32_t r = j - pre;
+        int u = u0;
+        for (; u < u1; ++u) {
+          const uint32_t x = tile_parts(a.tcount[u * kCtrStride]) - 1u;
+          if (r < x) break;
+          r -= x;
+        }
+        s_tile = u;
+        s_part = (int)r + 1;
+      }
+      __syncthreads();
+      t = __builtin_amdgcn_readfirstlane(s_tile);
+      part = __builtin_amdgcn_readfirstlane(s_part);
+    }
+    sort_part(t, part);
+    __syncthreads();  // the LDS lists are reused
   }
 }
 
@@ -3452,7 +3529,7 @@ hipError_t launch_edges(const EdgeArgs& a, bool near, hipStream_t st) {
 }
 
 hipError_t launch_tile_sort(const TileSortArgs& a, hipStream_t st) {
-  const int g = a.ntiles + a.netiles;
+  const int g = a.ntiles + a.netiles + a.nhelp;
   if (g > 0) CF_LAUNCH(k_tile_sort, dim3(g), dim3(kSortThreads), 0, st, a);
   return hipGetLastError();
 }
