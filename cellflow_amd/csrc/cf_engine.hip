@@ -12,6 +12,7 @@
 #include "cf_tune_cache.h"
 
 #include <algorithm>
+#include <atomic>
 #include <cmath>
 #include <cstdarg>
 #include <cstdio>
@@ -110,6 +111,7 @@ int grid_dims(const cf_params& p, const float* rbt, int T, int n, int divisor, i
 constexpr size_t kScratchBytes = size_t(32) << 20;  // 32 MiB per GPU
 static __device__ __align__(256) unsigned char scratch[kScratchBytes];
 constexpr int kScratchDevices = 64;
+constexpr int kStatusWords = 4;  // error flag, pairs of the graph, pairs of the step's graph
 static std::mutex g_scratch_mu;
 static void* g_scratch_ptr[kScratchDevices] = {};
 
@@ -192,6 +194,10 @@ struct Engine {
   std::vector<int> grid_sig;       // dims/reach of the binning A is sorted for
   std::vector<SimDesc> hdesc;      // uploaded descriptors (kept alive for async copies)
   std::vector<PairConst> hpairs;
+  std::vector<SimDesc> ndesc;      // being built; uploaded when they differ
+  std::vector<PairConst> npairs;
+  bool counters_dirty = true;  // the tile sort's counters need clearing before the next step
+  bool flag_dirty = false;     // the flag word may hold bits of an earlier call
   std::vector<uint32_t> hhist;
   // scan plans: 0 = cells, 1 = cells + edge counts, 2 = edge counts
   unsigned long long* tickets = nullptr;
@@ -211,6 +217,7 @@ struct Engine {
   size_t vtx_cap = 0;          // floats `vtx` holds
   float* vcol = nullptr;       // the caller's colours on the device
   size_t vcol_cap = 0;         // floats `vcol` holds
+  std::vector<float> hcol;     // the colours in `vcol`
   unsigned char* iobuf = nullptr;  // staging of the host get/set calls, kept between calls
   size_t iobuf_cap = 0;            // bytes `iobuf` holds
   int edges_maxc = 0;
@@ -239,6 +246,10 @@ struct Engine {
   uint32_t* hsmall = nullptr;  // pinned readback words
   unsigned char* hpin = nullptr;  // pinned staging of the large readbacks, kept between calls
   size_t hpin_cap = 0;            // bytes `hpin` holds
+  // large copies pass through `hpin` in at most kSlices slices of at least kSlice bytes
+  static constexpr size_t kSlice = size_t(2) << 20, kSlices = 16;
+  static constexpr size_t kCopyGrain = size_t(128) << 10;  // bytes a host thread copies at once
+  hipEvent_t slice_ev[kSlices] = {};
   // Captured step graphs.  A graph bakes kernel arguments (buffer pointers, sizes, tuning),
   // so the cache is keyed on them and dropped whenever a buffer is reallocated.
   struct GraphEntry {
@@ -248,7 +259,13 @@ struct Engine {
   std::vector<GraphEntry> graphs;
   long long buf_gen = 0;  // bumped on every reallocation of a buffer a graph references
 
-  ~Engine() { release(); }
+  Engine() { host_pool_hold(); }
+  ~Engine() {
+    release();
+    host_pool_drop();
+  }
+  Engine(const Engine&) = delete;
+  Engine& operator=(const Engine&) = delete;
 
   void drop_graphs() {
     for (auto& g : graphs)
@@ -269,7 +286,8 @@ struct Engine {
     dfree(b.tpos); dfree(b.tvel); dfree(b.tid); dfree(b.key); dfree(b.arrival);
     dfree(b.hist); dfree(b.tmp_id); dfree(b.acc); dfree(b.pad);
     dfree(b.ecand_d2); dfree(b.ecand_id); dfree(b.estage); dfree(b.ecount); dfree(b.fcount); dfree(b.eoff);
-    dfree(b.edges); dfree(b.sedges); dfree(b.stotal); dfree(b.gtotal); dfree(b.sims); dfree(b.wave_sim); dfree(b.pairs); dfree(b.flag);
+    dfree(b.edges); dfree(b.sedges); dfree(b.sims); dfree(b.wave_sim); dfree(b.pairs); dfree(b.flag);
+    b.gtotal = b.stotal = nullptr;  // words of `flag`
     dfree(slot_of); dfree(tickets); dfree(tris); dfree(vtx); dfree(vcol); dfree(iobuf);
     tris_cap = 0;
     tri_count = -1;
@@ -285,6 +303,10 @@ struct Engine {
     if (hpin) (void)hipHostFree(hpin);
     hpin = nullptr;
     hpin_cap = 0;
+    for (auto& e : slice_ev) {
+      if (e) (void)hipEventDestroy(e);
+      e = nullptr;
+    }
     if (st) (void)hipStreamDestroy(st);
     st = nullptr;
   }
@@ -322,9 +344,9 @@ struct Engine {
     CFR(dalloc(&b.ecount, P + 1)); CFR(dalloc(&b.eoff, P + 1)); CFR(dalloc(&b.fcount, P + 1));
     CFR(dalloc(&b.sims, nsims)); CFR(dalloc(&b.wave_sim, nwaves));
     CFR(dalloc(&b.pairs, (size_t)nsims * kMaxTypes * kMaxTypes));
-    CFR(dalloc(&b.flag, 4)); CFR(dalloc(&tickets, 3)); CFR(dalloc(&slot_of, P));
-    CFR(dalloc(&b.stotal, 1));
-    CFR(dalloc(&b.gtotal, 1));
+    CFR(dalloc(&b.flag, kStatusWords)); CFR(dalloc(&tickets, 3)); CFR(dalloc(&slot_of, P));
+    b.gtotal = b.flag + 1;  // the edge totals lie beside the flag: one readback per call
+    b.stotal = b.flag + 2;
     netiles = (int)((P + kEdgeTile - 1) / kEdgeTile);
     CFR(dalloc(&eticket, 1)); CFR(dalloc(&eflags, netiles));
     HIPR(hipMemsetAsync(eticket, 0, sizeof(unsigned long long), st));
@@ -337,7 +359,7 @@ struct Engine {
     HIPR(hipMemsetAsync(b.tvel, 0, P * sizeof(float4), st));
     HIPR(hipMemsetAsync(b.acc, 0, P * sizeof(float4), st));
     HIPR(hipMemsetAsync(b.pad, 0, P * sizeof(float), st));
-    HIPR(hipMemsetAsync(b.flag, 0, 4 * sizeof(uint32_t), st));
+    HIPR(hipMemsetAsync(b.flag, 0, kStatusWords * sizeof(uint32_t), st));
     std::vector<uint32_t> ws(nwaves, 0);
     for (int s = 0; s < nsims; ++s) {
       const int w0 = sims[s].p0 / kWave;
@@ -357,15 +379,18 @@ struct Engine {
 
   // ---- descriptors and grid --------------------------------------------------------
 
-  int build_descs(const EdgeReq& er, bool* grid_changed) {
-    hdesc.assign(sims.size(), SimDesc{});
-    hpairs.assign(sims.size() * kMaxTypes * kMaxTypes, PairConst{});
+  // Descriptors for the current parameters, uploaded when they differ from those on the
+  // device.  `any_edges`: the caller reads no edge field of theirs (nor steps), so ones that
+  // differ in those alone stay.
+  int build_descs(const EdgeReq& er, bool* grid_changed, bool any_edges = false) {
+    ndesc.assign(sims.size(), SimDesc{});
+    npairs.assign(sims.size() * kMaxTypes * kMaxTypes, PairConst{});
     std::vector<int> sig;
     long c = 0;
     int nt = 0;
     for (size_t s = 0; s < sims.size(); ++s) {
       SimHost& h = sims[s];
-      SimDesc& d = hdesc[s];
+      SimDesc& d = ndesc[s];
       cf_params p = h.prm;
       if (!h.have_prm) {
         // No parameters yet: one cell holds everything (only loads/gets happen).
@@ -419,7 +444,7 @@ struct Engine {
         // squared distance is below thr - 1e-4 (FP32 rounding absorbed by the margin).
         double reach2 = 0.0;
         for (int bb = 0; bb < h.T; ++bb) {
-          PairConst& pc = hpairs[d.tab + a * h.T + bb];
+          PairConst& pc = npairs[d.tab + a * h.T + bb];
           const float e = h.have_prm ? eff_radius(p, h.rbt.data(), a, bb) : 0.0f;
           pc.thr = cutoff_threshold(e);
           pc.fv = h.table[a * h.T + bb];
@@ -428,8 +453,8 @@ struct Engine {
         }
         if (er.on) reach2 = std::max(reach2, (double)ed2);
         const float cut2 = (float)(reach2 * (1.0 + 1e-3) + 1e-12);
-        for (int bb = 0; bb < h.T; ++bb) hpairs[d.tab + a * h.T + bb].pad = cut2;
-        if (er.on && ed2 + 1e-4f < hpairs[d.tab + a * h.T + a].thr) d.edge_inside |= (1 << a);
+        for (int bb = 0; bb < h.T; ++bb) npairs[d.tab + a * h.T + bb].pad = cut2;
+        if (er.on && ed2 + 1e-4f < npairs[d.tab + a * h.T + a].thr) d.edge_inside |= (1 << a);
       }
       d.ident = h.have_prm ? 0 : 1;
       d.edge_on = er.on ? 1 : 0;
@@ -458,13 +483,36 @@ struct Engine {
       sig.push_back(d.nz);
       sig.push_back(d.reach);
     }
-    C = c;
     *grid_changed = (sig != grid_sig);
+    if (!*grid_changed && !counters_dirty && hdesc.size() == ndesc.size() &&
+        hpairs.size() == npairs.size()) {
+      if (any_edges) {
+        for (size_t s = 0; s < ndesc.size(); ++s) {
+          SimDesc& d = ndesc[s];
+          const SimDesc& o = hdesc[s];
+          d.edge_on = o.edge_on;
+          d.edge_d2 = o.edge_d2;
+          d.edge_maxc = o.edge_maxc;
+          d.edge_inside = o.edge_inside;
+          d.edge_rx = o.edge_rx;
+          d.edge_ry = o.edge_ry;
+          d.edge_rz = o.edge_rz;
+        }
+        for (size_t k = 0; k < npairs.size(); ++k) npairs[k].pad = hpairs[k].pad;
+      }
+      if (std::memcmp(ndesc.data(), hdesc.data(), hdesc.size() * sizeof(SimDesc)) == 0 &&
+          std::memcmp(npairs.data(), hpairs.data(), hpairs.size() * sizeof(PairConst)) == 0)
+        return CF_OK;
+    }
+    C = c;
     if (*grid_changed) {
       grid_sig = sig;
       CFR(ensure_cells());
     }
     HIPR(hipStreamSynchronize(st));  // descriptors may still be read by queued work
+    hdesc.swap(ndesc);
+    hpairs.swap(npairs);
+    counters_dirty = true;  // until everything below is queued
     if (nt > ntiles_cap) {
       drop_graphs();
       ++buf_gen;
@@ -502,6 +550,7 @@ struct Engine {
                         hipMemcpyHostToDevice, st));
     HIPR(hipMemcpyAsync(b.pairs, hpairs.data(), hpairs.size() * sizeof(PairConst),
                         hipMemcpyHostToDevice, st));
+    counters_dirty = false;
     return CF_OK;
   }
 
@@ -601,8 +650,13 @@ struct Engine {
 
   // Loads write index-order records of one simulation into the temporaries; the other
   // simulations' current state is copied there first, then everything is sorted once.
-  int begin_load() {
+  // `replace`: the caller writes all of its simulation's slots.
+  int begin_load(bool replace) {
     if (load_pending) return CF_OK;
+    if (replace && sims.size() == 1) {
+      load_pending = true;
+      return CF_OK;
+    }
     HIPR(hipMemcpyAsync(b.tpos, b.pos[cur], P * sizeof(float4), hipMemcpyDeviceToDevice, st));
     HIPR(hipMemcpyAsync(b.tvel, b.vel[cur], P * sizeof(float4), hipMemcpyDeviceToDevice, st));
     HIPR(hipMemcpyAsync(b.tid, b.id[cur], P * sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
@@ -614,7 +668,7 @@ struct Engine {
     if (!load_pending) return CF_OK;
     bool changed = false;
     EdgeReq none;
-    CFR(build_descs(none, &changed));
+    CFR(build_descs(none, &changed, true));
     CFR(sort_into(b.tpos, b.tvel, b.tid, cur));
     load_pending = false;
     edges_count = -1;  // a graph or mesh belongs to the state it was built on
@@ -624,10 +678,10 @@ struct Engine {
   }
 
   // Re-sort the current state when the grid changes (new parameters).
-  int prepare(const EdgeReq& er) {
+  int prepare(const EdgeReq& er, bool any_edges = false) {
     CFR(flush());
     bool changed = false;
-    CFR(build_descs(er, &changed));
+    CFR(build_descs(er, &changed, any_edges));
     if (changed) {
       CFR(sort_into(b.pos[cur], b.vel[cur], b.id[cur], 1 - cur));
       cur = 1 - cur;
@@ -799,6 +853,10 @@ struct Engine {
       return fail(CF_ERR_ARG, "force variants 3 and 4 take at most 2^%d particle slots",
                   kCodeShift);
     const int B = 1 - cur;
+    // the tile sort leaves the next step's counters cleared; anything else (the counting
+    // sort's steps, a failed launch) leaves them to build_descs
+    counters_dirty = true;
+    flag_dirty = true;
     ForceArgs fa = force_args(fused_edges, cap, write_acc);
     timed(ev, 0);
     const hipError_t e0 = launch_force(fa, fused_edges, tun.block_size, tun.force_variant,
@@ -827,6 +885,7 @@ struct Engine {
       HIPR(e3);
     }
     cur = B;
+    counters_dirty = tun.sort_variant != 1;
     return CF_OK;
   }
 
@@ -926,14 +985,12 @@ struct Engine {
   }
 
   int finish_call(bool edges_built, bool step_edges_built = false) {
-    HIPR(hipMemcpyAsync(hsmall, b.flag, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    if (edges_built)
-      HIPR(hipMemcpyAsync(hsmall + 1, b.gtotal, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
-    if (step_edges_built)
-      HIPR(hipMemcpyAsync(hsmall + 3, b.stotal, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    HIPR(hipMemcpyAsync(hsmall, b.flag, kStatusWords * sizeof(uint32_t), hipMemcpyDeviceToHost,
+                        st));
     HIPR(hipStreamSynchronize(st));
     if (edges_built) edges_count = (long long)hsmall[1];
-    if (step_edges_built) step_edges_count = (long long)hsmall[3];
+    if (step_edges_built) step_edges_count = (long long)hsmall[2];
+    flag_dirty = hsmall[0] != 0u;
     if (hsmall[0] & 1u) return fail(CF_ERR_NONFINITE, "a position or velocity became non-finite");
     if (hsmall[0] & 4u) return fail(CF_ERR_DEVICE, "internal: the step sort lost track of a particle");
     return CF_OK;
@@ -944,7 +1001,7 @@ struct Engine {
       if (!h.have_prm) return fail(CF_ERR_STATE, "parameters not set for every simulation");
     if (er.on) CFR(ensure_edge_bufs(er.maxc));
     CFR(prepare(er));
-    HIPR(hipMemsetAsync(b.flag, 0, sizeof(uint32_t), st));
+    if (flag_dirty) HIPR(hipMemsetAsync(b.flag, 0, sizeof(uint32_t), st));
     const bool fuse = fusable(er);
     const int cap = 2 * er.maxc;
     edges_count = -1;
@@ -999,34 +1056,83 @@ struct Engine {
     return CF_OK;
   }
 
+  // The pinned staging buffer of loads and readbacks, at least `bytes` long (each use ends
+  // with a stream synchronisation, so no two overlap).
+  int pin(size_t bytes) {
+    if (bytes <= hpin_cap) return CF_OK;
+    HIPR(hipStreamSynchronize(st));
+    if (hpin) (void)hipHostFree(hpin);
+    hpin = nullptr;
+    hpin_cap = 0;
+    HIPR(hipHostMalloc((void**)&hpin, bytes, hipHostMallocDefault));
+    hpin_cap = bytes;
+    return CF_OK;
+  }
+
   // Device-to-host copy of `bytes` into the caller's memory through the pinned staging
-  // buffer (a DMA into pinned memory, then one host copy); synchronous.  Splitting it into
-  // chunks whose host copies overlap the next DMA measured no faster.
+  // buffer; synchronous.  The DMAs of all slices are queued at once; each slice is then
+  // copied on by the host threads as it arrives, beside the DMA of the next ones.
   int to_host(void* dst, const void* src, size_t bytes) {
     if (bytes == 0) return CF_OK;
-    if (bytes > hpin_cap) {
-      HIPR(hipStreamSynchronize(st));
-      if (hpin) (void)hipHostFree(hpin);
-      hpin = nullptr;
-      hpin_cap = 0;
-      HIPR(hipHostMalloc((void**)&hpin, bytes, hipHostMallocDefault));
-      hpin_cap = bytes;
+    CFR(pin(bytes));
+    const size_t slice = std::max(kSlice, (bytes + kSlices - 1) / kSlices);
+    size_t k = 0;
+    for (size_t at = 0; at < bytes; at += slice, ++k) {
+      HIPR(hipMemcpyAsync(hpin + at, (const char*)src + at, std::min(slice, bytes - at),
+                          hipMemcpyDeviceToHost, st));
+      if (at + slice >= bytes) break;  // the stream's end serves as the last slice's event
+      if (!slice_ev[k]) HIPR(hipEventCreateWithFlags(&slice_ev[k], hipEventDisableTiming));
+      HIPR(hipEventRecord(slice_ev[k], st));
     }
-    HIPR(hipMemcpyAsync(hpin, src, bytes, hipMemcpyDeviceToHost, st));
-    HIPR(hipStreamSynchronize(st));
-    std::memcpy(dst, hpin, bytes);
+    k = 0;
+    for (size_t at = 0; at < bytes; at += slice, ++k) {
+      if (at + slice < bytes) HIPR(hipEventSynchronize(slice_ev[k]));
+      else HIPR(hipStreamSynchronize(st));
+      char* d = (char*)dst + at;
+      const unsigned char* s = hpin + at;
+      host_parallel(std::min(slice, bytes - at), kCopyGrain,
+                    [=](size_t i0, size_t i1) { std::memcpy(d + i0, s + i0, i1 - i0); });
+    }
     return CF_OK;
   }
 
   int load_aos(int s, const cf_particle* parts) {
     const SimHost& h = sims[s];
-    for (int i = 0; i < h.n; ++i)
-      if (parts[i].ptype >= (uint32_t)h.T)
-        return fail(CF_ERR_ARG, "particle %d has type %u >= num_types %d", i, parts[i].ptype, h.T);
-    CFR(begin_load());
+    const size_t n = (size_t)std::max(0, h.n), rec = sizeof(AosParticle);
     AosParticle* d = nullptr;
-    CFR(io_stage(&d, (size_t)std::max(1, h.n)));
-    HIPR(hipMemcpyAsync(d, parts, (size_t)h.n * sizeof(AosParticle), hipMemcpyHostToDevice, st));
+    CFR(io_stage(&d, std::max<size_t>(1, n)));
+    // A slice's records are checked and copied to pinned memory by the host threads beside
+    // the DMA of the slices before; nothing of the engine's state is touched until all passed.
+    // A small load goes straight from the caller's memory unless a readback has pinned a
+    // buffer already: pinning one takes 0.1-0.25 ms, more than it saves.
+    const bool staged = n * rec <= hpin_cap || n * rec >= 2 * kSlice;
+    if (staged) CFR(pin(n * rec));
+    const size_t slice = staged ? std::max(kSlice, (n * rec + kSlices - 1) / kSlices) / rec : n;
+    std::atomic<long long> bad{(long long)n};
+    for (size_t at = 0; at < n && bad.load() == (long long)n; at += slice) {
+      const size_t m = std::min(slice, n - at);
+      const uint32_t T = (uint32_t)h.T;
+      host_parallel(m, kCopyGrain / rec, [&](size_t i0, size_t i1) {
+        if (staged) std::memcpy(hpin + (at + i0) * rec, parts + at + i0, (i1 - i0) * rec);
+        for (size_t i = at + i0; i < at + i1; ++i)
+          if (parts[i].ptype >= T) {
+            long long b = bad.load();
+            while ((long long)i < b && !bad.compare_exchange_weak(b, (long long)i)) {
+            }
+            break;
+          }
+      });
+      if (bad.load() == (long long)n)
+        HIPR(hipMemcpyAsync(d + at, staged ? (const void*)(hpin + at * rec) : parts + at, m * rec,
+                            hipMemcpyHostToDevice, st));
+    }
+    const long long b0 = bad.load();
+    if (b0 < (long long)n) {
+      HIPR(hipStreamSynchronize(st));
+      return fail(CF_ERR_ARG, "particle %d has type %u >= num_types %d", (int)b0,
+                  parts[b0].ptype, h.T);
+    }
+    CFR(begin_load(true));
     IoArgs a = io_args(s);
     a.aos = d;
     HIPR(launch_io(0, a, h.n, st));
@@ -1053,9 +1159,7 @@ struct Engine {
     IoArgs a = io_args(s);
     a.counts_out = d;
     HIPR(launch_io(2, a, h.n, st));
-    HIPR(hipMemcpyAsync(out, d, (size_t)h.n * sizeof(int32_t), hipMemcpyDeviceToHost, st));
-    HIPR(hipStreamSynchronize(st));
-    return CF_OK;
+    return to_host(out, d, (size_t)h.n * sizeof(int32_t));
   }
 
   int set_counts(int s, const int32_t* in) {
@@ -1092,7 +1196,7 @@ struct Engine {
   // there and sorted again by the next flush.
   int move(int s, float dx, float dy, float dz, const float box[3]) {
     CFR(flush());
-    CFR(begin_load());
+    CFR(begin_load(false));
     IoArgs a = io_args(s);
     a.shift[0] = dx;
     a.shift[1] = dy;
@@ -1103,7 +1207,7 @@ struct Engine {
   }
 
   int init_particles(int s, uint64_t seed, const float canvas[3], float spawn) {
-    CFR(begin_load());
+    CFR(begin_load(true));
     // descriptors must carry this simulation's T before the init kernel runs
     bool changed = false;
     EdgeReq none;
@@ -1132,11 +1236,7 @@ struct Engine {
     if (capacity < edges_count)
       return fail(CF_ERR_CAPACITY, "edge buffer holds %lld pairs, %lld needed", capacity,
                   edges_count);
-    if (edges_count > 0)
-      HIPR(hipMemcpyAsync(pairs, b.edges, (size_t)edges_count * sizeof(int2),
-                          hipMemcpyDeviceToHost, st));
-    HIPR(hipStreamSynchronize(st));
-    return CF_OK;
+    return to_host(pairs, b.edges, (size_t)edges_count * sizeof(int2));
   }
 
   int get_step_edges(int32_t* pairs, long long capacity, long long* count) {
@@ -1147,11 +1247,7 @@ struct Engine {
     if (capacity < step_edges_count)
       return fail(CF_ERR_CAPACITY, "edge buffer holds %lld pairs, %lld needed", capacity,
                   step_edges_count);
-    if (step_edges_count > 0)
-      HIPR(hipMemcpyAsync(pairs, b.sedges, (size_t)step_edges_count * sizeof(int2),
-                          hipMemcpyDeviceToHost, st));
-    HIPR(hipStreamSynchronize(st));
-    return CF_OK;
+    return to_host(pairs, b.sedges, (size_t)step_edges_count * sizeof(int2));
   }
 
   // Triangle mesh of the current state (generateTriangleMesh, ParticleSimulation.cu:689-754)
@@ -1165,7 +1261,7 @@ struct Engine {
     }
     CFR(ensure_edge_bufs(maxc));
     EdgeReq none;
-    CFR(prepare(none));
+    CFR(prepare(none, true));
     const SimDesc& d = hdesc[0];
     // the counts are scanned in 32 bits: at most 64 triangles per owner must fit
     if ((long long)d.n * 64 > 0xFFFFFFFFll)
@@ -1199,9 +1295,9 @@ struct Engine {
     ta.rz = r[2];
     HIPR(launch_tri_count(ta, st));
     HIPR(launch_scan(plan(2, nullptr), st));
-    HIPR(hipMemcpyAsync(hsmall + 2, b.eoff + P, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    HIPR(hipMemcpyAsync(hsmall + 8, b.eoff + P, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
     HIPR(hipStreamSynchronize(st));
-    const long long total = (long long)hsmall[2];
+    const long long total = (long long)hsmall[8];
     if (total > tris_cap) {
       dfree(tris);
       tris_cap = 0;
@@ -1221,11 +1317,7 @@ struct Engine {
     *count = tri_count;
     if (capacity < tri_count)
       return fail(CF_ERR_CAPACITY, "triangle buffer holds %lld, %lld needed", capacity, tri_count);
-    if (tri_count > 0)
-      HIPR(hipMemcpyAsync(out, tris, (size_t)(3 * tri_count) * sizeof(int32_t),
-                          hipMemcpyDeviceToHost, st));
-    HIPR(hipStreamSynchronize(st));
-    return CF_OK;
+    return to_host(out, tris, (size_t)(3 * tri_count) * sizeof(int32_t));
   }
 
   // Device buffers of the vertex expansions, kept for the next call (a render loop calls
@@ -1244,12 +1336,19 @@ struct Engine {
       HIPR(hipStreamSynchronize(st));
       dfree(vcol);
       vcol_cap = 0;
+      hcol.clear();
       CFR(dalloc(&vcol, ncf));
       vcol_cap = ncf;
     }
-    if (ncolors > 0)
-      HIPR(hipMemcpyAsync(vcol, colors, 3 * (size_t)ncolors * sizeof(float),
-                          hipMemcpyHostToDevice, st));
+    // the colours are uploaded when their values differ from those on the device
+    const float* cf = reinterpret_cast<const float*>(colors);
+    static_assert(sizeof(cf_color) == 3 * sizeof(float), "colours are packed floats");
+    const size_t nc = 3 * (size_t)std::max(0, ncolors);
+    if (nc > 0 && (hcol.size() != nc || std::memcmp(hcol.data(), cf, nc * sizeof(float)) != 0)) {
+      HIPR(hipStreamSynchronize(st));  // `hcol` may still be read by a queued copy
+      hcol.assign(cf, cf + nc);
+      HIPR(hipMemcpyAsync(vcol, hcol.data(), nc * sizeof(float), hipMemcpyHostToDevice, st));
+    }
     HIPR(launch_slot_of(b.id[cur], slot_of, b.sims, 0, sims[0].n, st));
     return CF_OK;
   }
@@ -1596,7 +1695,7 @@ struct Engine {
     if (sims.size() != 1) return fail(CF_ERR_STATE, "histograms are defined for one simulation");
     if (!sims[0].have_prm) return fail(CF_ERR_STATE, "parameters not set");
     EdgeReq none;
-    CFR(prepare(none));
+    CFR(prepare(none, true));
     const int n = sims[0].n;
     const long stride = ((long)n + 127) / 128 * 128;
     StateBuf s;
@@ -1751,6 +1850,7 @@ struct Engine {
       sa.id = b.id[cur];
       sa.x64_next = shadow(0, false);
       sa.v64_next = shadow(0, true);
+      flag_dirty = true;  // until a call's status reads zero
       HIPR(launch_shadow_init(sa, n, st));
       // forward with checkpoints; the last segment's states are kept as they are made.
       // Every step lists its in-range pairs (for the shadow; the last segment's lists are

@@ -1,11 +1,20 @@
 // Host-only entry points and helpers of the C ABI: the error string, tuning validation and
 // the tuning-cache file calls.  No device code.
 
+#include <unistd.h>
+
+#include <algorithm>
+#include <atomic>
 #include <cmath>
+#include <condition_variable>
 #include <cstdarg>
 #include <cstdio>
 #include <map>
+#include <mutex>
+#include <new>
 #include <string>
+#include <thread>
+#include <vector>
 
 #include "cf_host.h"
 #include "cf_tune_cache.h"
@@ -25,6 +34,124 @@ int fail(int code, const char* fmt, ...) {
   va_end(ap);
   error_text() = buf;
   return code;
+}
+
+namespace {
+
+struct Pool {
+  std::mutex mu;
+  std::condition_variable wake, done;
+  std::vector<std::thread> threads;
+  const std::function<void(size_t, size_t)>* fn = nullptr;  // the job, null between jobs
+  size_t n = 0, grain = 0;
+  std::atomic<size_t> next{0};
+  unsigned long long job = 0;
+  int active = 0;
+  bool stop = false;
+
+  void take(const std::function<void(size_t, size_t)>& f, size_t count, size_t step) {
+    for (size_t i = next.fetch_add(step); i < count; i = next.fetch_add(step))
+      f(i, std::min(count, i + step));
+  }
+
+  void work() {
+    unsigned long long seen = 0;
+    std::unique_lock<std::mutex> l(mu);
+    while (true) {
+      wake.wait(l, [&] { return stop || job != seen; });
+      if (stop) return;
+      seen = job;
+      if (!fn) continue;  // the job ended before this thread woke
+      const auto* f = fn;
+      const size_t count = n, step = grain;
+      ++active;
+      l.unlock();
+      take(*f, count, step);
+      l.lock();
+      if (--active == 0) done.notify_all();
+    }
+  }
+};
+
+std::mutex g_pool_mu;  // guards the three below
+std::mutex g_run_mu;   // one job at a time
+Pool* g_pool = nullptr;
+int g_pool_users = 0;
+std::atomic<pid_t> g_pool_pid{0};  // the process the threads live in
+
+}  // namespace
+
+void host_pool_hold() {
+  std::lock_guard<std::mutex> l(g_pool_mu);
+  ++g_pool_users;
+}
+
+void host_pool_drop() {
+  const pid_t owner = g_pool_pid.load();
+  if (owner != 0 && owner != getpid()) return;  // a forked child has none of the threads
+  Pool* gone = nullptr;
+  {
+    std::lock_guard<std::mutex> l(g_pool_mu);
+    if (--g_pool_users == 0) {
+      gone = g_pool;
+      g_pool = nullptr;
+      g_pool_pid = 0;
+    }
+  }
+  if (!gone) return;
+  {
+    std::lock_guard<std::mutex> l(gone->mu);
+    gone->stop = true;
+  }
+  gone->wake.notify_all();
+  for (std::thread& t : gone->threads) t.join();
+  delete gone;
+}
+
+void host_parallel(size_t n, size_t grain, const std::function<void(size_t, size_t)>& fn) {
+  grain = std::max<size_t>(grain, 1);
+  const pid_t owner = g_pool_pid.load();
+  std::unique_lock<std::mutex> run(g_run_mu, std::defer_lock);
+  if (n <= 3 * grain || (owner != 0 && owner != getpid()) || !run.try_lock()) {
+    if (n) fn(0, n);
+    return;
+  }
+  Pool* p = nullptr;
+  {
+    std::unique_lock<std::mutex> l(g_pool_mu, std::try_to_lock);
+    if (l && g_pool_users > 0) {
+      if (!g_pool) {
+        g_pool = new (std::nothrow) Pool;
+        if (g_pool) {
+          g_pool_pid = getpid();
+          try {
+            for (int k = 0; k < kHostHelpers; ++k)
+              g_pool->threads.emplace_back([q = g_pool] { q->work(); });
+          } catch (...) {  // as many as the system gives
+          }
+        }
+      }
+      p = g_pool;
+    }
+  }
+  // the pool outlives this call: the caller's engine holds it
+  if (!p) {
+    fn(0, n);
+    return;
+  }
+  {
+    std::lock_guard<std::mutex> l(p->mu);
+    p->fn = &fn;
+    p->n = n;
+    p->grain = grain;
+    p->next = 0;
+    ++p->job;
+  }
+  p->wake.notify_all();
+  p->take(fn, n, grain);
+  std::unique_lock<std::mutex> l(p->mu);
+  p->fn = nullptr;  // a helper that wakes from here on skips the job
+  p->done.wait(l, [&] { return p->active == 0; });
 }
 
 int check_tuning(const cf_tuning* t) {
