@@ -1247,7 +1247,9 @@ __global__ void __launch_bounds__(256) k_force_grp(ForceArgs a) {
 // Measured against k_force_grp<16> (uniform states at 12,500 per unit volume, us per
 // launch): 1k 10.1 -> 5.8, 20k 11.6 -> 7.1, 100k 35 -> 18.4, 100k with edges 46.5 -> 24,
 // the same after 300 steps 48.5 -> 32, 500k 142 -> 71; 1M clustered (238 neighbours) with
-// edges 1171 -> 640, without 485 -> 440; 20k of a preset (516 neighbours) 82 -> 77.
+// edges 1171 -> 584, without 485 -> 400; 20k of a preset (516 neighbours) 82 -> 64 (the walk
+// with an index per candidate, one candidate per turn and a select per image shift: 640,
+// 435 and 79).
 
 constexpr int kWaveList = 640;  // candidate slots per wave
 constexpr int kListEdges = 24;  // LDS edge candidates per particle (more: the wave selects)
@@ -1674,6 +1676,7 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
     // dense neighbourhoods: no list (it would cost about as much as the pairs), the lanes
     // walk the runs themselves from a table in the list's place, entry 2 * row + half
     static_assert(kOwn * 2 * kRows * 2 <= kWaveList, "the run table fits the list");
+    static_assert((16ull << kCodeShift) + 256u <= 0xFFFFFFFFull, "byte offsets fit 32 bits");
     uint2* wr = reinterpret_cast<uint2*>(&lslot[wv][0]) + o * 2 * kRows;
     // entry of this lane's run pair i (-1: none); lane 3 also keeps the centre row (fast8)
     auto entry = [&](int i) {
@@ -1719,17 +1722,32 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
           const uint32_t len = e.y;
           if (len == 0u) continue;
           const uint32_t q0 = e.x & ((1u << kCodeShift) - 1u), code = e.x >> kCodeShift;
-          uint32_t t = (uint32_t)(v16 - (int)cum) & 15u;
+          const uint32_t t = (uint32_t)(v16 - (int)cum) & 15u;
           if (t < len) {
-            float4 pj = a.pos[q0 + t];
-            while (true) {
-              const uint32_t tn = t + 16u;
-              const float4 pn = a.pos[q0 + min(tn, len - 1u)];
-              pair(gen_kind, std::false_type{}, q0 + t, code, pj, 0u);
-              if (tn >= len) break;
-              t = tn;
-              pj = pn;
-            }
+            // by byte offset (one add and one clamp per candidate), the next candidate's load in
+            // flight, two candidates per turn so that none is copied, shifted runs apart: the
+            // loop is bound by instruction issue, 22 of them per candidate instead of 33
+            auto at = [&](uint32_t off) {
+              return *reinterpret_cast<const float4*>(reinterpret_cast<const char*>(a.pos) + off);
+            };
+            auto lane_run = [&](uint32_t run_code) {
+              constexpr uint32_t kStep = 16u * (uint32_t)sizeof(float4);
+              const uint32_t end = (q0 + len - 1u) * (uint32_t)sizeof(float4);
+              uint32_t off = (q0 + t) * (uint32_t)sizeof(float4);
+              float4 p0 = at(off);
+              while (true) {
+                const uint32_t off1 = off + kStep;
+                const float4 p1 = at(min(off1, end));
+                pair(gen_kind, std::false_type{}, off / (uint32_t)sizeof(float4), run_code, p0, 0u);
+                if (off1 > end) break;
+                off = off1 + kStep;
+                p0 = at(min(off, end));
+                pair(gen_kind, std::false_type{}, off1 / (uint32_t)sizeof(float4), run_code, p1, 0u);
+                if (off > end) break;
+              }
+            };
+            if (decltype(gen_kind)::value || code == 0u) lane_run(0u);
+            else lane_run(code);
           }
           cum += len;
         }
