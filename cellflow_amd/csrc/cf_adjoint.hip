@@ -23,6 +23,7 @@
 // L = sum_b (h_b - target_b)^2.
 
 #include "cf_internal.h"
+#include "cf_shadow.h"
 
 namespace cf {
 
@@ -46,32 +47,6 @@ __device__ __forceinline__ double bspline3_d(double u) {  // dB3/du
   return (-2.0 * a + 1.5 * a * a) * s;
 }
 
-// fmod(y, L) for L > 0, exactly: for y in [0, 2L) it is y or y - L (the subtraction is exact
-// there), else fmod itself.
-__device__ __forceinline__ double wrap_d(double y, double L) {
-  if (y >= 0.0 && y < 2.0 * L) return y >= L ? y - L : y;
-  return fmod(y, L);
-}
-
-__device__ __forceinline__ double min_image_d(double d, double L) {
-  if (d > L * 0.5) d -= L;
-  if (d < -L * 0.5) d += L;
-  return d;
-}
-
-__device__ __forceinline__ float min_image_f(float d, float L) {
-  if (d > L * 0.5f) d -= L;
-  if (d < -L * 0.5f) d += L;
-  return d;
-}
-
-__device__ __forceinline__ int bin_axis_a(float x, float ih, int n) {
-  float u = x * ih;
-  if (!(u >= 0.0f)) return 0;
-  if (u >= (float)n) return n - 1;
-  return (int)u;
-}
-
 // ---- histogram and its gradient ------------------------------------------------------
 
 // Fixed-order sum of `n` values with stride, one output per block (deterministic).
@@ -93,77 +68,27 @@ __global__ void __launch_bounds__(256) k_reduce_rows(const double* __restrict__ 
 
 // ---- one backward step -----------------------------------------------------------------
 
-// The FP64 density factor of a frozen count (the oracle's op order).
-__device__ __forceinline__ double shadow_fac(const AdjConst& c, int cnt, int prev) {
-  const double avg = (double)(cnt + prev) * 0.5;
-  const double dens = fmin(avg / c.max_exp, 1.0);
-  return 1.0 - (1.0 - c.balance) * dens;
+// phi_i = dt m_i (lv'_i + dt lx'_i),  lv_i = fr (lv'_i + dt lx'_i) of the particle with index
+// id, whose step had the counts cnt and prev: into phi[id] and lam_v[id].
+__device__ __forceinline__ void phi_of(const AdjConst& c, uint32_t id, int cnt, int prev,
+                                       const double4& lx, const double4& lv, double4* phi,
+                                       double4* lam_v) {
+  // the shadow's FP64 factor of the frozen counts (ParticleSimulation.cu:136-143)
+  const double m = c.fm * shadow_fac(c, cnt, prev);
+  const double dt = c.dt, fr = c.friction;
+  const double mx = lv.x + dt * lx.x, my = lv.y + dt * lx.y, mz = lv.z + dt * lx.z;
+  phi[id] = make_double4(dt * m * mx, dt * m * my, dt * m * mz, 0.0);
+  lam_v[id] = make_double4(fr * mx, fr * my, fr * mz, 0.0);
 }
 
-// phi_i = dt m_i (lv'_i + dt lx'_i),  lv_i = fr (lv'_i + dt lx'_i) of particle k; phi is
-// stored by the pre-step slot, where the pair kernel finds both ends of a pair without an
-// index lookup.  The walk kernel computes it on the side (it needs nothing the walk makes).
+// The same for particle k of the step being reversed.  The walk kernel computes it on the
+// side (it needs nothing the walk makes).
 __device__ __forceinline__ void adj_phi(const AdjArgs& a, const SimDesc& sd, int k) {
   const int p = sd.p0 + k;
   const uint32_t id = a.id[p];
   const int prev = __float_as_int(a.vel[p].w);
   const int cnt = __float_as_int(a.tvel[p].w);  // this step's count, by pre-step slot
-  // the shadow's FP64 factor of the frozen counts (ParticleSimulation.cu:136-143)
-  const double m = a.c.fm * shadow_fac(a.c, cnt, prev);
-  const double4 lx = a.lam_x_next[id], lv = a.lam_v_next[id];
-  const double dt = a.c.dt, fr = a.c.friction;
-  const double mx = lv.x + dt * lx.x, my = lv.y + dt * lx.y, mz = lv.z + dt * lx.z;
-  a.phi[p] = make_double4(dt * m * mx, dt * m * my, dt * m * mz, 0.0);  // by pre-step slot
-  a.lam_v[id] = make_double4(fr * mx, fr * my, fr * mz, 0.0);
-}
-
-// ---- pair kernels: G lanes per particle -----------------------------------------------
-//
-// One lane per particle would leave most of the GPU idle at a few tens of thousands of
-// particles and walk every candidate serially.  Instead the stencil's cells are split
-// over G lanes (cell index c = g, g+G, ...) and the lanes' partial sums are reduced in a
-// fixed order, so results are deterministic.
-
-constexpr int kAdjG = 8;                       // lanes per particle
-constexpr int kAdjBlock = 128;                 // threads per block
-constexpr int kAdjPer = kAdjBlock / kAdjG;     // particles per block
-constexpr int kAdjVals = 4 + kMaxTypes;        // lx, ly, lz, ratio, table row
-
-// Visit the stencil cells c = first, first + step, ... of the (2r+1)^3 cube around
-// (cx, cy, cz) (every cell once on axes with fewer than 2r+1 cells), in a fixed order:
-// for_cell_runs passes each cell's slot range, for_cells_split each of its slots.  Cell
-// coordinates come from float reciprocals: (c + 1/2) / m is at least 1/(2m) away from an
-// integer and m <= 25, far beyond the float error.
-template <class Fn>
-__device__ __forceinline__ void for_cell_runs(const SimDesc& sd, const uint32_t* start, int cx,
-                                              int cy, int cz, int r, int first, int step,
-                                              Fn&& fn) {
-  const bool gx = sd.nx < 2 * r + 1, gy = sd.ny < 2 * r + 1, gz = sd.nz < 2 * r + 1;
-  const int nxo = gx ? sd.nx : 2 * r + 1, nyo = gy ? sd.ny : 2 * r + 1,
-            nzo = gz ? sd.nz : 2 * r + 1;
-  const int ncell = nxo * nyo * nzo, nxy = nxo * nyo;
-  const float inxy = 1.0f / (float)nxy, inx = 1.0f / (float)nxo;
-  for (int ci = first; ci < ncell; ci += step) {
-    const int iz = (int)(((float)ci + 0.5f) * inxy);
-    const int rem = ci - iz * nxy;
-    const int iy = (int)(((float)rem + 0.5f) * inx);
-    const int ix = rem - iy * nxo;
-    int x = gx ? ix : cx + ix - r, y = gy ? iy : cy + iy - r, z = gz ? iz : cz + iz - r;
-    if (x < 0) x += sd.nx; else if (x >= sd.nx) x -= sd.nx;
-    if (y < 0) y += sd.ny; else if (y >= sd.ny) y -= sd.ny;
-    if (z < 0) z += sd.nz; else if (z >= sd.nz) z -= sd.nz;
-    const int cc = sd.c0 + x + sd.nx * (y + sd.ny * z);
-    fn(start[cc], start[cc + 1]);
-  }
-}
-
-template <class Fn>
-__device__ __forceinline__ void for_cells_split(const SimDesc& sd, const uint32_t* start, int cx,
-                                                int cy, int cz, int r, int first, int step,
-                                                Fn&& fn) {
-  for_cell_runs(sd, start, cx, cy, cz, r, first, step, [&](uint32_t q0, uint32_t q1) {
-    for (uint32_t q = q0; q < q1; ++q) fn(q);
-  });
+  phi_of(a.c, id, cnt, prev, a.lam_x_next[id], a.lam_v_next[id], a.phi, a.lam_v);
 }
 
 // Histogram partials, G lanes per particle.  The group's lanes add each pair's four spline
@@ -290,43 +215,6 @@ __device__ __forceinline__ uint32_t group_excl_scan(uint32_t v, int g) {
   return x - v;
 }
 
-constexpr int kAdjHits = kPairList;  // also the stride of the force kernel's lists
-
-// The pair kernel's particle context and its FP32 in-range decision, shared by the walk
-// kernel and the pair kernel.
-struct AdjOwn {
-  float4 pi;
-  int p, ti, cx, cy, cz;
-};
-
-__device__ __forceinline__ AdjOwn adj_own(const AdjArgs& a, const SimDesc& sd, int k, bool active) {
-  AdjOwn c;
-  c.p = sd.p0 + k;
-  c.pi = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  c.ti = -1;
-  c.cx = c.cy = c.cz = 0;
-  if (active) {
-    c.pi = a.pos[c.p];
-    c.ti = (int)__float_as_uint(c.pi.w);
-    c.cx = bin_axis_a(c.pi.x, sd.ihx, sd.nx);
-    c.cy = bin_axis_a(c.pi.y, sd.ihy, sd.ny);
-    c.cz = bin_axis_a(c.pi.z, sd.ihz, sd.nz);
-  }
-  return c;
-}
-
-// the forward's FP32 decision (ParticleSimulation.cu:92-112 with the engine's op order)
-__device__ __forceinline__ bool adj_in_range(const AdjArgs& a, const SimDesc& sd, const AdjOwn& c,
-                                             uint32_t q) {
-  if ((int)q == c.p) return false;
-  const float4 pj = a.pos[q];
-  const int tj = (int)__float_as_uint(pj.w);
-  const float fx = min_image_f(pj.x - c.pi.x, sd.Lx), fy = min_image_f(pj.y - c.pi.y, sd.Ly),
-              fz = min_image_f(pj.z - c.pi.z, sd.Lz);
-  const float s2f = fmaf(fz, fz, fmaf(fy, fy, fx * fx));
-  return s2f + 1e-4f < a.thr[c.ti * a.c.T + tj];
-}
-
 // ---- the FP64 shadow of the rollout ------------------------------------------------------
 //
 // The forward rollout is the FP32 step; its decisions (in-range pairs, counts) define the
@@ -354,82 +242,7 @@ __global__ void __launch_bounds__(256) k_shadow_init(AdjArgs a) {
 // most kAdjHits per particle, in slot order), or from a walk of the FP32 state's stencil with
 // the forward's FP32 decision (no lists, or a particle with more pairs than a list holds).
 __global__ void __launch_bounds__(kAdjBlock) k_shadow_step(AdjArgs a) {
-  constexpr int G = kAdjG;
-  const SimDesc sd = a.sims[0];
-  const int o = threadIdx.x / G, g = threadIdx.x % G;
-  const int k = blockIdx.x * kAdjPer + o;
-  const bool active = k < sd.n;
-  const AdjOwn c = adj_own(a, sd, k, active);
-  const int T = a.c.T;
-  double fx = 0.0, fy = 0.0, fz = 0.0;
-  int cnt = 0;
-  uint32_t idi = 0;
-  double4 xi = make_double4(0.0, 0.0, 0.0, 0.0);
-  const double R = a.c.radius, rho = a.c.ratio;
-  const double effi = active ? R * (1.0 + a.c.rbt[c.ti] * rho) : 0.0;
-  // the FP64 force term of one in-range pair (the oracle's op order), partner type tj at
-  // shadow position xj
-  auto pair = [&](int tj, const double4& xj) {
-    const double dx = min_image_d(xj.x - xi.x, sd.Lx);
-    const double dy = min_image_d(xj.y - xi.y, sd.Ly);
-    const double dz = min_image_d(xj.z - xi.z, sd.Lz);
-    const double dist = sqrt(dx * dx + dy * dy + dz * dz + (double)1e-4f);
-    const double eff = (effi + R * (1.0 + a.c.rbt[tj] * rho)) * 0.5;
-    const double r = dist / eff;
-    const double net = (a.c.rep * exp(-a.c.k * r * r) - a.c.att * r) * a.c.table[c.ti * T + tj];
-    fx += dx / dist * net;
-    fy += dy / dist * net;
-    fz += dz / dist * net;
-  };
-  int prev = 0;
-  double4 vi = make_double4(0.0, 0.0, 0.0, 0.0);
-  if (active) {
-    idi = a.id[c.p];
-    xi = a.x64[idi];
-    if (g == 0) {  // the integration's inputs, loaded before the pairs are summed
-      prev = __float_as_int(a.vel[c.p].w);
-      vi = a.v64[idi];
-    }
-    const uint32_t nh = a.hits ? a.nhits[k] : 0u;
-    if (a.hits && nh <= (uint32_t)kAdjHits) {
-      if (g == 0) cnt = (int)nh;
-      // the lane's entries two at a time, each stage's loads issued together (list entry,
-      // then type and index, then shadow position); pairs summed in entry order
-      const uint32_t* lst = a.hits + (long)k * kAdjHits;
-#pragma nounroll
-      for (uint32_t e = g; e < nh; e += 2 * G) {
-        const bool two = e + G < nh;
-        const uint32_t q0 = lst[e], q1 = two ? lst[e + G] : q0;
-        const int t0 = (int)__float_as_uint(a.pos[q0].w), t1 = (int)__float_as_uint(a.pos[q1].w);
-        const uint32_t j0 = a.id[q0], j1 = a.id[q1];
-        const double4 x0 = a.x64[j0], x1 = a.x64[j1];
-        pair(t0, x0);
-        if (two) pair(t1, x1);
-      }
-    } else {
-      for_cells_split(sd, a.start, c.cx, c.cy, c.cz, sd.reach, g, G, [&](uint32_t q) {
-        if (!adj_in_range(a, sd, c, q)) return;
-        ++cnt;
-        pair((int)__float_as_uint(a.pos[q].w), a.x64[a.id[q]]);
-      });
-    }
-  }
-#pragma unroll
-  for (int m = G / 2; m > 0; m >>= 1) {
-    fx += __shfl_xor(fx, m, 64);
-    fy += __shfl_xor(fy, m, 64);
-    fz += __shfl_xor(fz, m, 64);
-    cnt += __shfl_xor(cnt, m, 64);
-  }
-  if (!active || g != 0) return;
-  const double m = a.c.fm * shadow_fac(a.c, cnt, prev) * a.c.dt;
-  const double vx = vi.x * a.c.friction + fx * m;
-  const double vy = vi.y * a.c.friction + fy * m;
-  const double vz = vi.z * a.c.friction + fz * m;
-  a.v64_next[idi] = make_double4(vx, vy, vz, 0.0);
-  a.x64_next[idi] = make_double4(wrap_d(xi.x + vx * a.c.dt + (double)sd.Lx, (double)sd.Lx),
-                                 wrap_d(xi.y + vy * a.c.dt + (double)sd.Ly, (double)sd.Ly),
-                                 wrap_d(xi.z + vz * a.c.dt + (double)sd.Lz, (double)sd.Lz), 0.0);
+  shadow_block(a, blockIdx.x * kAdjBlock + threadIdx.x);
 }
 
 // Sets flag bit 3 when a shadow position lies more than slack/2 (periodic, per axis) from
@@ -492,7 +305,10 @@ __global__ void __launch_bounds__(kAdjBlock) k_adj_walk(AdjArgs a) {
 // of its particles summed in particle order and added to one column of `partial` (row r at
 // partial[r * stride + block]), which so sums the steps of the rollout in the order they are
 // reversed.  Every order is fixed by the data, so the results are deterministic.
-__global__ void __launch_bounds__(kAdjBlock) k_adj_pair_g(AdjArgs a) {
+// 168 VGPRs, three waves per SIMD: 20k particles are 2.4 waves per SIMD, so at two (212
+// VGPRs) some wait for a place (16.6 us instead of 14.3 per step); at four it spills (17.9).
+__global__ void __launch_bounds__(kAdjBlock) __attribute__((amdgpu_waves_per_eu(3, 8)))
+k_adj_pair_g(AdjArgs a) {
   constexpr int G = kAdjG;
   __shared__ double red[kAdjBlock][kAdjVals];
   __shared__ int btype[kAdjPer];
@@ -511,11 +327,18 @@ __global__ void __launch_bounds__(kAdjBlock) k_adj_pair_g(AdjArgs a) {
   uint32_t idi = 0, nh = 0;
   double4 phi_i = make_double4(0.0, 0.0, 0.0, 0.0);
   double4 xi = make_double4(0.0, 0.0, 0.0, 0.0);
+  const int rows = T * T + 1;
+  static_assert(kMaxTypes * kMaxTypes + 1 <= kAdjBlock, "one row per thread");
+  // what the tail adds to is loaded now, in flight through the pairs
+  double* const col = a.partial + (long)threadIdx.x * a.stride + blockIdx.x;
+  const double col0 = (int)threadIdx.x < rows ? *col : 0.0;
+  double4 lxn = make_double4(0.0, 0.0, 0.0, 0.0);
   if (active) {
     idi = a.id[p];
-    phi_i = a.phi[p];
+    phi_i = a.phi[idi];
     nh = a.nhits[k];
     xi = a.x64[idi];
+    if (g == 0) lxn = a.lam_x_next[idi];
   }
   // the FP64 terms of one in-range pair: partner type tj, shadow position xj, factor phi_j
   auto pair = [&](int tj, const double4& xj, const double4& phi_j) {
@@ -553,11 +376,12 @@ __global__ void __launch_bounds__(kAdjBlock) k_adj_pair_g(AdjArgs a) {
     });
   const uint32_t first = group_excl_scan<G>(nmine, g);
   auto pair_q = [&](uint32_t q) {
-    pair((int)__float_as_uint(a.pos[q].w), a.x64[a.id[q]], a.phi[q]);
+    const uint32_t j = a.id[q];
+    pair((int)__float_as_uint(a.pos[q].w), a.x64[j], a.phi[j]);
   };
   if (listed) {
     // the lane's entries two at a time, each stage's loads issued together (list entry, then
-    // type, index and factor, then shadow position); pairs summed in entry order
+    // type and index, then factor and shadow position); pairs summed in entry order
     const uint32_t* lst = a.hits + (long)k * kAdjHits;
 #pragma nounroll
     for (uint32_t e = g; e < nh; e += 2 * G) {
@@ -565,7 +389,7 @@ __global__ void __launch_bounds__(kAdjBlock) k_adj_pair_g(AdjArgs a) {
       const uint32_t q0 = lst[e], q1 = two ? lst[e + G] : q0;
       const int t0 = (int)__float_as_uint(a.pos[q0].w), t1 = (int)__float_as_uint(a.pos[q1].w);
       const uint32_t j0 = a.id[q0], j1 = a.id[q1];
-      const double4 f0 = a.phi[q0], f1 = a.phi[q1];
+      const double4 f0 = a.phi[j0], f1 = a.phi[j1];
       const double4 x0 = a.x64[j0], x1 = a.x64[j1];
       pair(t0, x0, f0);
       if (two) pair(t1, x1, f1);
@@ -605,14 +429,20 @@ __global__ void __launch_bounds__(kAdjBlock) k_adj_pair_g(AdjArgs a) {
   }
   __syncthreads();
   if (active && g == 0) {
-    const double4 lxn = a.lam_x_next[idi];
-    a.lam_x[idi] = make_double4(lxn.x + red[o * G][0], lxn.y + red[o * G][1],
-                                lxn.z + red[o * G][2], 0.0);
+    const double4 lxi = make_double4(lxn.x + red[o * G][0], lxn.y + red[o * G][1],
+                                     lxn.z + red[o * G][2], 0.0);
+    a.lam_x[idi] = lxi;
+    // the factor of the step before, whose counts the state carries (its own count in the
+    // velocity's w, the one before in the shadow position's): a launch of its own took 4 us
+    // and a gap per step
+    if (a.phi_prev)
+      phi_of(a.c, idi, __float_as_int(a.vel[p].w), (int)xi.w, lxi, a.lam_v[idi], a.phi_prev,
+             a.lam_v_prev);
   }
   // block partials: row (a2 * T + t) sums the table term of particles of type a2, row T*T
   // the ratio term, each over the block's particles in order
-  const int rows = T * T + 1;
-  for (int row = threadIdx.x; row < rows; row += kAdjBlock) {
+  const int row = threadIdx.x;
+  if (row < rows) {
     double acc = 0.0;
     if (row < T * T) {
       const int a2 = row / T, t = row % T;
@@ -622,7 +452,7 @@ __global__ void __launch_bounds__(kAdjBlock) k_adj_pair_g(AdjArgs a) {
       for (int oo = 0; oo < kAdjPer; ++oo)
         if (btype[oo] >= 0) acc += red[oo * G][3];
     }
-    a.partial[(long)row * a.stride + blockIdx.x] += acc;
+    *col = col0 + acc;
   }
 }
 
@@ -640,20 +470,22 @@ hipError_t launch_hist_grad(const HistArgs& a, int n, hipStream_t st) {
   return hipGetLastError();
 }
 
-// The density-factor terms alone, for steps whose lists the recompute's force kernel wrote.
+// The density-factor terms alone, for the last step when its lists came from the force
+// kernel; the pair kernel then makes those of the step before.
 __global__ void __launch_bounds__(128) k_adj_phi(AdjArgs a) {
   const SimDesc sd = a.sims[0];
   const int k = blockIdx.x * blockDim.x + threadIdx.x;
   if (k < sd.n) adj_phi(a, sd, k);
 }
 
+hipError_t launch_adj_phi(const AdjArgs& a, int n, hipStream_t st) {
+  hipLaunchKernelGGL(k_adj_phi, dim3((n + 127) / 128), dim3(128), 0, st, a);
+  return hipGetLastError();
+}
+
 hipError_t launch_adj_step(const AdjArgs& a, int n, hipStream_t st, bool walk) {
-  if (!walk) {
-    hipLaunchKernelGGL(k_adj_phi, dim3((n + 127) / 128), dim3(128), 0, st, a);
-    hipLaunchKernelGGL(k_adj_pair_g, dim3(adj_pair_blocks(n)), dim3(kAdjBlock), 0, st, a);
-    return hipGetLastError();
-  }
-  hipLaunchKernelGGL(k_adj_walk, dim3(adj_pair_blocks(n)), dim3(kAdjBlock), 0, st, a);
+  if (walk)
+    hipLaunchKernelGGL(k_adj_walk, dim3(adj_pair_blocks(n)), dim3(kAdjBlock), 0, st, a);
   hipLaunchKernelGGL(k_adj_pair_g, dim3(adj_pair_blocks(n)), dim3(kAdjBlock), 0, st, a);
   return hipGetLastError();
 }

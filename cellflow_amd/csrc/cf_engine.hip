@@ -241,6 +241,8 @@ struct Engine {
   // in-range partners (ForceArgs::hits)
   uint32_t* fhits = nullptr;
   uint32_t* fnhits = nullptr;
+  // ... and the shadow step that a step's tile sort takes along (k_sort_shadow)
+  const AdjArgs* with_shadow = nullptr;
   std::vector<uint32_t> htile_sim;
   cf_tuning tun{1, 0, 16, 256, 32, 1};
   uint32_t* hsmall = nullptr;  // pinned readback words
@@ -866,7 +868,9 @@ struct Engine {
     HIPR(e0);
     if (tun.sort_variant == 1) {
       timed(ev, 1);
-      const hipError_t e1 = launch_tile_sort(tile_sort_args(fused_edges), st);
+      const hipError_t e1 =
+          with_shadow ? launch_sort_shadow(tile_sort_args(fused_edges), *with_shadow, sims[0].n, st)
+                      : launch_tile_sort(tile_sort_args(fused_edges), st);
       arm_kernel_timer(nullptr, nullptr);
       HIPR(e1);
     } else {
@@ -1578,74 +1582,107 @@ struct Engine {
     double4* fwv[2] = {nullptr, nullptr};
     double4* lx[2] = {nullptr, nullptr};
     double4* lv[2] = {nullptr, nullptr};
-    double4* phi = nullptr;
+    double4* phi[2] = {nullptr, nullptr};
+    unsigned char* arena = nullptr;  // everything above and below lies in it
     // in-range lists of each segment step (the force kernel writes them during the
     // recompute with variant 0; with other variants the walk fills the first)
     std::vector<uint32_t*> hits, nhits;
     double *partial = nullptr, *hd = nullptr, *gh = nullptr, *gacc = nullptr;
     float* thr = nullptr;
     std::vector<long> shape;  // empty: nothing allocated
+    long ckpt = 0;            // steps between checkpoints (all of them: every state is kept)
   } adj;
+  static constexpr size_t kKeepBytes = size_t(4) << 30, kKeepTimes = 16;
 
   void free_adj() {
-    for (auto& s : adj.ck) free_state(s);
-    for (auto& s : adj.seg) free_state(s);
-    for (auto& t : adj.tv) dfree(t);
-    free_state(adj.fin);
-    for (int i = 0; i < 2; ++i) {
-      dfree(adj.lx[i]);
-      dfree(adj.lv[i]);
-      dfree(adj.fwx[i]);
-      dfree(adj.fwv[i]);
-    }
-    dfree(adj.phi);
-    for (auto& x : adj.hits) dfree(x);
-    for (auto& x : adj.nhits) dfree(x);
-    adj.hits.clear();
-    adj.nhits.clear();
-    dfree(adj.partial);
-    dfree(adj.hd);
-    dfree(adj.gh);
-    dfree(adj.gacc);
-    dfree(adj.thr);
-    adj.ck.clear();
-    adj.seg.clear();
-    adj.tv.clear();
-    adj.shape.clear();
+    dfree(adj.arena);
+    adj = AdjBufs{};
   }
 
-  // shape = {P, C, n, segments, checkpoint interval, bins, T, partial rows, partial stride}
-  int alloc_adj(const std::vector<long>& shape) {
-    if (adj.shape == shape) return CF_OK;
-    free_adj();
-    const long n = shape[2], nseg = shape[3], ckpt = shape[4], bins = shape[5], T = shape[6],
-               rows = shape[7], stride = shape[8];
+  // Lays the gradient's buffers out from `base` (null: only counts): one allocation, as a
+  // rollout whose every state is kept has thousands of buffers.  Returns the bytes.
+  size_t lay_adj(unsigned char* base, long n, long nseg, long ckpt, long bins, long T, long rows,
+                 long stride) {
+    size_t off = 0;
+    auto take = [&](auto*& p, size_t count) {
+      using E = std::remove_reference_t<decltype(*p)>;
+      p = base ? reinterpret_cast<E*>(base + off) : nullptr;
+      off += (std::max<size_t>(count, 1) * sizeof(E) + 255) / 256 * 256;
+    };
+    auto state = [&](StateBuf& b, bool shadow) {
+      take(b.pos, P);
+      take(b.vel, P);
+      take(b.id, P);
+      take(b.start, C + 1);
+      if (shadow) {
+        take(b.x64, P);
+        take(b.v64, P);
+      }
+    };
     adj.ck.resize((size_t)std::max(nseg, 1L));
     adj.seg.resize((size_t)ckpt + 1);
     adj.tv.assign((size_t)ckpt, nullptr);
-    for (auto& s : adj.ck) CFR(alloc_state(s, true));
-    for (size_t i = 1; i < adj.seg.size(); ++i) CFR(alloc_state(adj.seg[i], true));
-    for (auto& t : adj.tv) CFR(dalloc(&t, P));
-    CFR(alloc_state(adj.fin));
+    for (auto& c : adj.ck) state(c, true);
+    for (size_t i = 1; i < adj.seg.size(); ++i) state(adj.seg[i], true);
+    for (auto& t : adj.tv) take(t, P);
+    state(adj.fin, false);
     for (int i = 0; i < 2; ++i) {
-      CFR(dalloc(&adj.lx[i], P));
-      CFR(dalloc(&adj.lv[i], P));
-      CFR(dalloc(&adj.fwx[i], P));
-      CFR(dalloc(&adj.fwv[i], P));
+      take(adj.lx[i], P);
+      take(adj.lv[i], P);
+      take(adj.fwx[i], P);
+      take(adj.fwv[i], P);
+      take(adj.phi[i], P);
     }
-    CFR(dalloc(&adj.phi, P));
     adj.hits.assign((size_t)ckpt, nullptr);
     adj.nhits.assign((size_t)ckpt, nullptr);
     for (long i = 0; i < ckpt; ++i) {
-      CFR(dalloc(&adj.hits[i], (size_t)std::max(n, 1L) * kPairList));
-      CFR(dalloc(&adj.nhits[i], (size_t)std::max(n, 1L)));
+      take(adj.hits[i], (size_t)std::max(n, 1L) * kPairList);
+      take(adj.nhits[i], (size_t)std::max(n, 1L));
     }
-    CFR(dalloc(&adj.partial, (size_t)(rows * stride)));
-    CFR(dalloc(&adj.hd, (size_t)bins));
-    CFR(dalloc(&adj.gh, (size_t)bins));
-    CFR(dalloc(&adj.gacc, (size_t)(T * T + 1)));
-    CFR(dalloc(&adj.thr, (size_t)(T * T)));
+    take(adj.partial, (size_t)(rows * stride));
+    take(adj.hd, (size_t)bins);
+    take(adj.gh, (size_t)bins);
+    take(adj.gacc, (size_t)(T * T + 1));
+    take(adj.thr, (size_t)(T * T));
+    return off;
+  }
+
+  // The buffers of a rollout of `nsteps` steps with checkpoints every *ckpt of them.  When
+  // all states fit kKeepBytes, kKeepTimes what the caller's interval takes and an eighth of
+  // the free memory, *ckpt becomes nsteps: every state is then kept as it is made and none
+  // recomputed, which was a third of a gradient (20k particles, 200 steps, checkpoints every
+  // 20: 180 of 380 steps; the buffers take 1.6 GB).  The interval does not change a bit of
+  // the result.
+  int alloc_adj(long n, long nsteps, long* ckpt, long bins, long T, long rows, long stride) {
+    const std::vector<long> shape = {P, C, n, nsteps, *ckpt, bins, T, rows, stride};
+    if (adj.shape == shape) {
+      *ckpt = adj.ckpt;
+      return CF_OK;
+    }
+    free_adj();
+    auto lay = [&](unsigned char* base, long every) {
+      return lay_adj(base, n, (nsteps + every - 1) / every, every, bins, T, rows, stride);
+    };
+    long every = std::min(*ckpt, std::max(nsteps, 1L));
+    if (every < nsteps) {
+      const size_t asked = lay(nullptr, every), all = lay(nullptr, nsteps);
+      size_t avail = 0, total = 0;
+      if (all <= kKeepBytes && all <= kKeepTimes * asked && hipMemGetInfo(&avail, &total) == hipSuccess && all <= avail / 8)
+        every = nsteps;
+    }
+    size_t bytes = lay(nullptr, every);
+    if (hipMalloc((void**)&adj.arena, bytes) != hipSuccess) {
+      (void)hipGetLastError();
+      adj.arena = nullptr;
+      if (every <= *ckpt) return fail(CF_ERR_DEVICE, "%zu bytes of gradient buffers: out of device memory", bytes);
+      every = *ckpt;
+      bytes = lay(nullptr, every);
+      CFR(dalloc(&adj.arena, bytes));
+    }
+    lay(adj.arena, every);
+    adj.ckpt = every;
     adj.shape = shape;
+    *ckpt = every;
     return CF_OK;
   }
 
@@ -1763,7 +1800,7 @@ struct Engine {
 
   // Gradient of the final-state histogram loss after `nsteps` steps with respect to the
   // force table and the ratio, by the adjoint method with checkpoints every `ckpt` steps.
-  int rollout_grad(int nsteps, int ckpt, int bins, double r_max, const double* target,
+  int rollout_grad(int nsteps, int ckpt_asked, int bins, double r_max, const double* target,
                    double* loss_out, double* hist_out, double* gtab, double* grat) {
     if (sims.size() != 1) return fail(CF_ERR_STATE, "gradients are defined for one simulation");
     SimHost& h = sims[0];
@@ -1776,20 +1813,22 @@ struct Engine {
     tri_count = -1;
     const int n = h.n, T = h.T;
     const long stride = ((long)n + 127) / 128 * 128;
-    const int nseg = (nsteps + ckpt - 1) / ckpt;
     const int rows = std::max(bins, T * T + 1);
     int rc = CF_OK;
     const DevBufs own = b;  // the engine's state buffers (the recompute re-points them)
     auto body = [&]() -> int {
-      CFR(alloc_adj({P, C, (long)n, (long)nseg, (long)ckpt, (long)bins, (long)T, (long)rows,
-                     stride}));
+      long every = ckpt_asked;
+      CFR(alloc_adj(n, nsteps, &every, bins, T, rows, stride));
+      const int ckpt = (int)every, nseg = (nsteps + ckpt - 1) / ckpt;
+      // the accelerations (output-only) left by a call are those of the last step of the
+      // first segment asked for, whether segments are recomputed or kept
+      const int acc_step = std::min(ckpt_asked, nsteps) - 1;
       std::vector<StateBuf>& ck = adj.ck;
       std::vector<StateBuf>& seg = adj.seg;  // seg[0] is never allocated: it is ck[sg]
       std::vector<float4*>& tv = adj.tv;     // each segment step's new velocities + counts
       StateBuf& fin = adj.fin;
       double4** lx = adj.lx;
       double4** lv = adj.lv;
-      double4* phi = adj.phi;
       // variant 0 lists each step's in-range partners during the recompute; the other
       // variants leave that to the adjoint's walk kernel
       const bool lists = tun.force_variant == 0;
@@ -1828,10 +1867,11 @@ struct Engine {
         if (s % ckpt == 0) return vel ? ck[s / ckpt].v64 : ck[s / ckpt].x64;
         return vel ? adj.fwv[s & 1] : adj.fwx[s & 1];
       };
-      // one shadow step of an FP32 pre-step state, after the FP32 step whose force kernel
-      // listed the state's in-range pairs into list buffer `li` (no lists: the shadow walks)
-      auto shadow_step = [&](const StateBuf& pre, int li, const double4* x, const double4* v,
-                             double4* xn, double4* vn) -> int {
+      // one FP32 step and the shadow step of its pre-step state, over the in-range pairs that
+      // its force kernel lists into list buffer `li` (no lists: the shadow walks); the tile
+      // sort takes the shadow step along
+      auto shadowed_step = [&](bool write_acc, const StateBuf& pre, int li, const double4* x,
+                               const double4* v, double4* xn, double4* vn) -> int {
         sa.pos = pre.pos;
         sa.vel = pre.vel;
         sa.id = pre.id;
@@ -1842,7 +1882,14 @@ struct Engine {
         sa.v64 = v;
         sa.x64_next = xn;
         sa.v64_next = vn;
-        HIPR(launch_shadow_step(sa, n, st));
+        listing(li);
+        const bool along = tun.sort_variant == 1;
+        with_shadow = along ? &sa : nullptr;
+        const int rc = step(false, 0, nullptr, write_acc);
+        with_shadow = nullptr;
+        fhits = fnhits = nullptr;
+        CFR(rc);
+        if (!along) HIPR(launch_shadow_step(sa, n, st));
         return CF_OK;
       };
       sa.pos = b.pos[cur];
@@ -1866,12 +1913,9 @@ struct Engine {
           point(1 - cur, seg[s - last0 + 1]);
           b.tvel = tv[s - last0];
         }
-        listing(s % ckpt);
-        CFR(step(false, 0));
-        CFR(shadow_step(pre, s % ckpt, shadow(s, false), shadow(s, true), shadow(s + 1, false),
-                        shadow(s + 1, true)));
+        CFR(shadowed_step(s == acc_step, pre, s % ckpt, shadow(s, false), shadow(s, true),
+                          shadow(s + 1, false), shadow(s + 1, true)));
       }
-      fhits = fnhits = nullptr;
       CFR(save_state(fin));
       b = own;
       const double4* xfin = shadow(nsteps, false);
@@ -1910,7 +1954,6 @@ struct Engine {
       aa.sims = b.sims;
       aa.thr = thr;
       aa.c = sa.c;
-      aa.phi = phi;
       aa.partial = partial;
       aa.stride = nblk;
       int L = 0;  // lx[L] holds dL/dx of the state after the step being reversed
@@ -1922,12 +1965,9 @@ struct Engine {
             const StateBuf& sp = (s == k0) ? ck[sg] : seg[s - k0];
             point(1 - cur, seg[s - k0 + 1]);
             b.tvel = tv[s - k0];
-            listing(s - k0);
-            CFR(step(false, 0));
-            CFR(shadow_step(sp, s - k0, sp.x64, sp.v64, seg[s - k0 + 1].x64,
-                            seg[s - k0 + 1].v64));
+            CFR(shadowed_step(s == acc_step, sp, s - k0, sp.x64, sp.v64, seg[s - k0 + 1].x64,
+                              seg[s - k0 + 1].v64));
           }
-          fhits = fnhits = nullptr;
           b = own;
         }
         for (int s = k1 - 1; s >= k0; --s) {
@@ -1942,6 +1982,11 @@ struct Engine {
           aa.lam_v_next = lv[L];
           aa.lam_x = lx[1 - L];
           aa.lam_v = lv[1 - L];
+          aa.phi = adj.phi[L];
+          // with lists, the pair kernel makes the factors of the step before
+          aa.phi_prev = lists && s > 0 ? adj.phi[1 - L] : nullptr;
+          aa.lam_v_prev = lv[L];
+          if (lists && s == nsteps - 1) HIPR(launch_adj_phi(aa, n, st));
           aa.hits = adj.hits[lists ? s - k0 : 0];
           aa.nhits = adj.nhits[lists ? s - k0 : 0];
           HIPR(launch_adj_step(aa, n, st, !lists));
@@ -1963,6 +2008,7 @@ struct Engine {
     (void)hipStreamSynchronize(st);
     b = own;  // the engine's own state buffers, whatever the recompute pointed them at
     fhits = fnhits = nullptr;
+    with_shadow = nullptr;
     if (rc != CF_OK) free_adj();
     return rc;
   }

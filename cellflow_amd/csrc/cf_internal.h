@@ -408,7 +408,10 @@ struct AdjArgs {
   const double4* lam_v_next;
   double4* lam_x;
   double4* lam_v;
-  double4* phi;
+  double4* phi;             // density-factor terms of the step, by particle index
+  // where the pair kernel leaves those of the step before (and its dL/dv); null: nowhere
+  double4* phi_prev;
+  double4* lam_v_prev;
   uint32_t* hits;           // [n][64] in-range slots of each particle, slot order (walk)
   uint32_t* nhits;          // [n] their number (more than 64: the pair kernel walks again)
   double* partial;          // [T*T + 1][stride] parameter partials, one column per block,
@@ -430,7 +433,9 @@ hipError_t launch_reduce_rows(const double* in, long stride, int n, int rows, do
                               double* out, int accumulate, hipStream_t st);
 // One backward step: with `walk`, the FP32 walk lists each particle's in-range partners
 // (and computes the density-factor terms); without, the lists in AdjArgs::hits came from
-// the recompute's force kernel.
+// the force kernel, and the terms from launch_adj_phi (the last step) or the pair kernel of
+// the step after.
+hipError_t launch_adj_phi(const AdjArgs& a, int n, hipStream_t st);
 hipError_t launch_adj_step(const AdjArgs& a, int n, hipStream_t st, bool walk);
 // The rollout's FP64 shadow: the pre-step FP32 state promoted (index order); one FP64 step
 // with the decisions of the FP32 pre-step state; the drift check of a shadow state against
@@ -452,6 +457,8 @@ hipError_t launch_force(const ForceArgs& a, bool edges, int block, int variant, 
 // near: every simulation's edge reach is one cell on every axis.
 hipError_t launch_edges(const EdgeArgs& a, bool near, hipStream_t st);
 hipError_t launch_tile_sort(const TileSortArgs& a, hipStream_t st);
+// The tile sort of a rollout step (no edges) and its shadow step in one launch.
+hipError_t launch_sort_shadow(const TileSortArgs& a, const AdjArgs& s, int n, hipStream_t st);
 hipError_t launch_scan(const ScanPlan& p, hipStream_t st);
 hipError_t launch_fill(const SortArgs& a, hipStream_t st);
 hipError_t launch_rank_scatter(const SortArgs& a, hipStream_t st);

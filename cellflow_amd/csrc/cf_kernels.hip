@@ -30,6 +30,7 @@
 #include <type_traits>
 
 #include "cf_internal.h"
+#include "cf_shadow.h"
 
 namespace cf {
 
@@ -2579,9 +2580,7 @@ __device__ __forceinline__ uint32_t rank_in(const uint32_t* ids, uint32_t n, uin
   return rank;
 }
 
-// 80 VGPRs and 26 KB of LDS: three blocks of eight waves per CU.
-__global__ void __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(6, 8)))
-k_tile_sort(TileSortArgs a) {
+__device__ __forceinline__ void tile_sort(const TileSortArgs& a) {
   __shared__ uint32_t cnt_s[kTileCells];
   __shared__ uint32_t cofs[kTileCells + 1];
   __shared__ uint32_t fill_s[kTileCells];
@@ -2958,6 +2957,22 @@ k_tile_sort(TileSortArgs a) {
     sort_part(t, part);
     __syncthreads();  // the LDS lists are reused
   }
+}
+
+// 80 VGPRs and 26 KB of LDS: three blocks of eight waves per CU.
+__global__ void __launch_bounds__(kSortThreads) __attribute__((amdgpu_waves_per_eu(6, 8)))
+k_tile_sort(TileSortArgs a) {
+  tile_sort(a);
+}
+
+// A rollout step's sort (without edges) and, in the blocks after the sort's, its FP64 shadow
+// step: both need only the force pass, and each leaves most of the chip idle at the tens of
+// thousands of particles a gradient has (20k: 5.8 us and 8.2 us one after the other, and a
+// launch's gap).
+__global__ void __launch_bounds__(kSortThreads) k_sort_shadow(TileSortArgs a, AdjArgs s) {
+  const int nsort = a.ntiles + a.netiles + a.nhelp;
+  if ((int)blockIdx.x < nsort) tile_sort(a);
+  else shadow_block(s, ((int)blockIdx.x - nsort) * kSortThreads + (int)threadIdx.x);
 }
 
 // ------------------------------------------------------------------------------------
@@ -3549,6 +3564,13 @@ hipError_t launch_edges(const EdgeArgs& a, bool near, hipStream_t st) {
 hipError_t launch_tile_sort(const TileSortArgs& a, hipStream_t st) {
   const int g = a.ntiles + a.netiles + a.nhelp;
   if (g > 0) CF_LAUNCH(k_tile_sort, dim3(g), dim3(kSortThreads), 0, st, a);
+  return hipGetLastError();
+}
+
+hipError_t launch_sort_shadow(const TileSortArgs& a, const AdjArgs& s, int n, hipStream_t st) {
+  constexpr int per = kSortThreads / kAdjG;
+  CF_LAUNCH(k_sort_shadow, dim3(a.ntiles + a.netiles + a.nhelp + (n + per - 1) / per),
+            dim3(kSortThreads), 0, st, a, s);
   return hipGetLastError();
 }
 

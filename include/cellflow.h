@@ -262,7 +262,9 @@ int cf_pair_histogram_noalloc(cf_sim* sim, int bins, float r_max, double* hist);
 /* Runs `nsteps` steps from the current state (leaving the simulation at the final state)
  * and returns the loss L = sum_b (h_b - target_b)^2 of the final histogram and its gradient
  * with respect to the num_types^2 force-table entries (row-major) and ratio_with_lfo, by
- * a hand-written adjoint with state checkpoints every `checkpoint_every` steps.  The
+ * a hand-written adjoint with state checkpoints every `checkpoint_every` steps (or with all
+ * states kept, when they fit 4 GiB, an eighth of the free device memory and 16 times what the
+ * interval takes; the result is the same bit for bit).  The
  * rollout's discrete decisions (which pairs interact, neighbour counts) are those of the
  * FP32 steps and are held fixed; the loss, the histogram and the gradient are of the FP64
  * rollout along those decisions (an FP64 shadow of the state, stepped beside the FP32
