@@ -152,6 +152,7 @@ struct SimHost {
   std::vector<float> raw;    // T*T raw table (updateForceTable input)
   std::vector<float> rbt;    // T radius modifiers
   cf_params prm{};
+  bool loaded = false;  // loaded by the caller before (later loads are staged)
   bool have_prm = false;
   int dims[3] = {1, 1, 1};
   int reach = 1;
@@ -1107,9 +1108,11 @@ struct Engine {
     CFR(io_stage(&d, std::max<size_t>(1, n)));
     // A slice's records are checked and copied to pinned memory by the host threads beside
     // the DMA of the slices before; nothing of the engine's state is touched until all passed.
-    // A small load goes straight from the caller's memory unless a readback has pinned a
-    // buffer already: pinning one takes 0.1-0.25 ms, more than it saves.
-    const bool staged = n * rec <= hpin_cap || n * rec >= 2 * kSlice;
+    // A simulation's first load goes straight from the caller's memory unless a readback has
+    // pinned a buffer already: pinning one takes longer (0.1-0.25 ms for 1 MB, 5 ms for 44)
+    // than one load gains, and a program may load once and never read.
+    const bool staged = n * rec <= hpin_cap || sims[s].loaded;
+    sims[s].loaded = true;
     if (staged) CFR(pin(n * rec));
     const size_t slice = staged ? std::max(kSlice, (n * rec + kSlices - 1) / kSlices) / rec : n;
     std::atomic<long long> bad{(long long)n};
