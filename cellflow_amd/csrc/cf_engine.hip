@@ -1276,33 +1276,46 @@ struct Engine {
                   0xFFFFFFFFll / 64);
     const float hm = 1.2f;                             // :722, a 20% larger radius
     const float d2 = distance * distance * (hm * hm);  // :723, FP32 left to right
-    TriArgs ta{};
-    ta.pos = b.pos[cur];
-    ta.id = b.id[cur];
-    ta.start = b.start[cur];
-    ta.sims = b.sims;
-    ta.wave_sim = b.wave_sim;
-    ta.cand_d2 = b.ecand_d2;
-    ta.cand_id = b.ecand_id;
-    ta.sorted = b.estage;
-    ta.nsel = b.tmp_id;
-    ta.count = b.ecount;
-    ta.off = b.eoff;
-    ta.P = P;
-    ta.nwaves = nwaves;
-    ta.maxc = maxc;
-    ta.d2 = d2;
-    // cells within reach of sqrt(d2) on each axis (non-periodic, as :314-317)
+    EdgeArgs ea{};
+    ea.pos = b.pos[cur];
+    ea.id = b.id[cur];
+    ea.start = b.start[cur];
+    ea.sims = b.sims;
+    ea.wave_sim = b.wave_sim;
+    ea.estage = b.estage;
+    ea.estride = edge_maxc_alloc;
+    ea.ecount = b.ecount;
+    ea.nabove = b.tmp_id;
+    ea.nwaves = nwaves;
+    ea.edge_cap = maxc;
+    ea.d2 = d2;
+    // cells within reach of sqrt(d2) on each axis (non-periodic, as :314-317), at most the
+    // whole axis
     const double reach = std::sqrt((double)d2) * (1.0 + 1.0 / 1024.0);
     const float ih[3] = {d.ihx, d.ihy, d.ihz};
+    const int nc[3] = {d.nx, d.ny, d.nz};
     int r[3];
-    for (int a = 0; a < 3; ++a) r[a] = (int)std::max(1.0, std::min(std::ceil(reach * ih[a]), 1024.0));
-    ta.rx = r[0];
-    ta.ry = r[1];
-    ta.rz = r[2];
-    HIPR(launch_tri_count(ta, st));
+    for (int a = 0; a < 3; ++a) {
+      r[a] = (int)std::max(1.0, std::min(std::ceil(reach * ih[a]), 1024.0));
+      r[a] = std::min(r[a], std::max(1, nc[a] - 1));
+    }
+    ea.rx = r[0];
+    ea.ry = r[1];
+    ea.rz = r[2];
+    TriArgs ta{};
+    ta.rec = b.estage;
+    ta.nabove = b.tmp_id;
+    ta.count = b.ecount;
+    ta.off = b.eoff;
+    ta.tris = tris;
+    ta.cap = tris_cap;
+    ta.estride = edge_maxc_alloc;
+    ta.n = d.n;
+    HIPR(launch_tri_count(ea, r[0] == 1 && r[1] == 1 && r[2] == 1, st));
     HIPR(launch_scan(plan(2, nullptr), st));
     HIPR(hipMemcpyAsync(hsmall + 8, b.eoff + P, sizeof(uint32_t), hipMemcpyDeviceToHost, st));
+    // into the last mesh's buffer, before the host knows whether it holds this one
+    if (tris_cap > 0) HIPR(launch_tri_write(ta, st));
     HIPR(hipStreamSynchronize(st));
     const long long total = (long long)hsmall[8];
     if (total > tris_cap) {
@@ -1310,10 +1323,11 @@ struct Engine {
       tris_cap = 0;
       CFR(dalloc(&tris, (size_t)(3 * total)));
       tris_cap = total;
+      ta.tris = tris;
+      ta.cap = tris_cap;
+      HIPR(launch_tri_write(ta, st));
+      HIPR(hipStreamSynchronize(st));
     }
-    ta.tris = tris;
-    if (total > 0) HIPR(launch_tri_write(ta, st));
-    HIPR(hipStreamSynchronize(st));
     tri_count = total;
     return CF_OK;
   }

@@ -199,6 +199,11 @@ struct EdgeArgs {
   long estride;
   int nwaves;
   int edge_cap;
+  // the triangle mesh only: its squared distance, its reach in cells (non-periodic) and, per
+  // owner index, the kept partners above the owner (estage holds those; ecount the triangles)
+  float d2;
+  int rx, ry, rz;
+  uint32_t* nabove;
 };
 
 struct SortArgs {
@@ -328,26 +333,17 @@ struct LineArgs {
   int p0;
 };
 
-// Triangle mesh of the current state (generateTriangleMeshKernel): per owner slot, the
-// kept same-type neighbours and the owner's triangle count, then the canonical triangles.
+// Triangle mesh of the current state (generateTriangleMeshKernel): the canonical triangles
+// from each owner's list of kept neighbours (EdgeArgs), by owner index.
 struct TriArgs {
-  const float4* __restrict__ pos;
-  const uint32_t* __restrict__ id;
-  const uint32_t* __restrict__ start;
-  const SimDesc* __restrict__ sims;
-  const uint32_t* __restrict__ wave_sim;
-  float* cand_d2;        // [maxc][P] scratch of the index selection
-  uint32_t* cand_id;
-  uint32_t* sorted;      // [maxc][P] each owner's kept neighbours, ascending
-  uint32_t* nsel;        // [P] their number, by owner slot
-  uint32_t* count;       // [P] triangles of each owner, by owner index
-  const uint32_t* off;   // exclusive scan of count
+  const uint32_t* __restrict__ rec;     // [P][estride] kept neighbours above the owner, ascending
+  const uint32_t* __restrict__ nabove;  // [P] their number
+  const uint32_t* __restrict__ count;   // [P] triangles of each owner
+  const uint32_t* __restrict__ off;     // exclusive scan of count
   int32_t* tris;         // 3 indices per triangle
-  long P;
-  int nwaves;
-  int maxc;              // min(maxConnectionsPerParticle, 32)
-  float d2;              // squared distance threshold, hysteresis included
-  int rx, ry, rz;        // non-periodic stencil reach in cells
+  long cap;              // triangles that `tris` holds; later ones are not written
+  long estride;
+  long n;                // owners
 };
 
 struct TriVertArgs {
@@ -360,7 +356,7 @@ struct TriVertArgs {
   int ncolors;
   int T;
 };
-hipError_t launch_tri_count(const TriArgs& a, hipStream_t st);
+hipError_t launch_tri_count(const EdgeArgs& a, bool near, hipStream_t st);
 hipError_t launch_tri_write(const TriArgs& a, hipStream_t st);
 hipError_t launch_tri_vertices(const TriVertArgs& a, hipStream_t st);
 

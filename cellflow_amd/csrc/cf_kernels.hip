@@ -1309,7 +1309,8 @@ __device__ __forceinline__ void wave_sel_cut(WaveSel& s, int cap, int lane) {
 // Walks `nruns` runs (first slot, length; CODED: the slot carries an image-shift code above
 // kCodeShift, and a shifted run holds no partner) of the owner `me` with index `myid`.
 // GEN: the grid is too small for shifted runs, so the pair must be its own nearest image.
-template <bool CODED>
+// MESH: partners of any other index (the triangle mesh), else larger ones only.
+template <bool CODED, bool MESH = false>
 __device__ __forceinline__ void wave_sel_runs(WaveSel& s, const float4* __restrict__ pos,
                                               const uint32_t* __restrict__ id,
                                               const uint2* runs, int nruns, const float4& me,
@@ -1330,7 +1331,7 @@ __device__ __forceinline__ void wave_sel_runs(WaveSel& s, const float4* __restri
         const float ux = pj.x - me.x, uy = pj.y - me.y, uz = pj.z - me.z;
         d2 = fmaf(uz, uz, fmaf(uy, uy, ux * ux));
         hit = __float_as_uint(pj.w) == __float_as_uint(me.w) && d2 < sd.edge_d2 &&
-              jid > myid && jid < s.below;
+              (MESH ? jid != myid : jid > myid) && jid < s.below;
         if (CODED && gen)
           hit = hit && min_image(ux, sd.Lx) == ux && min_image(uy, sd.Ly) == uy &&
                 min_image(uz, sd.Lz) == uz;
@@ -1361,6 +1362,24 @@ __device__ __forceinline__ uint32_t wave_sel_finish(WaveSel& s, int cap, int max
   if (in && rank < maxc) rec[rank] = __float_as_uint(e.y);
   wave_lds_sync();  // the list is reused for the next owner
   return (uint32_t)min(s.n, maxc);
+}
+
+// The mesh's counterpart: those of the cap smallest indices that lie above the owner's own,
+// ascending, to the owner's record; returns how many.
+__device__ __forceinline__ uint32_t wave_sel_above(WaveSel& s, int cap, uint32_t myid,
+                                                   uint32_t* __restrict__ rec, int lane) {
+  if (s.n > cap) wave_sel_cut(s, cap, lane);
+  wave_lds_sync();
+  const uint32_t ix = lane < s.n ? __float_as_uint(s.buf[lane].y) : 0u;
+  const bool up = lane < s.n && ix > myid;
+  uint32_t rank = 0;  // among the kept ones above the owner
+  for (int k = 0; k < s.n; ++k) {
+    const uint32_t f = __float_as_uint(s.buf[k].y);
+    rank += (f > myid && f < ix) ? 1u : 0u;
+  }
+  if (up) rec[rank] = ix;
+  wave_lds_sync();  // the list is reused for the next owner
+  return (uint32_t)__popcll(__ballot(up));
 }
 
 // Sum over aligned groups of G lanes (G in 4, 8, 16, 32), every lane gets its group's sum.
@@ -2119,7 +2138,7 @@ __device__ __forceinline__ void edge_walk(const EdgeArgs& a, const SimDesc& sd,
   }
 }
 
-template <int ER>
+template <int ER, bool MESH>
 __device__ __forceinline__ void edges_owner(const EdgeArgs& a, const SimDesc& sd, int o, int g,
                                             int lane, int base, bool active, const float4& pi,
                                             uint32_t idi, float2 (*el_d)[kListEdges],
@@ -2153,7 +2172,7 @@ __device__ __forceinline__ void edges_owner(const EdgeArgs& a, const SimDesc& sd
     const float dx = pj.x - pi.x, dy = pj.y - pi.y, dz = pj.z - pi.z;
     const float s2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
     if (!(s2 < sd.edge_d2)) return;                  // :227
-    if (jid <= idi) return;                          // j > i, :215
+    if (MESH ? jid == idi : jid <= idi) return;      // j > i, :215; the mesh: j != i, :307
     const uint32_t kk = atomicAdd(&el_n[o], 1u);
     if (kk < (uint32_t)kListEdges) {
       el_d[o][kk] = make_float2(s2, 0.0f);
@@ -2223,8 +2242,25 @@ __device__ __forceinline__ void edges_owner(const EdgeArgs& a, const SimDesc& sd
   const uint32_t n = active ? el_n[o] : 0u;
   const bool fits = n <= (uint32_t)kListEdges;
   const int cap = a.edge_cap, maxc = sd.edge_maxc;
+  uint32_t above = 0u;  // the mesh: kept partners above the owner's index
+  if constexpr (MESH) {
+    // the cap smallest indices; those above the owner's own are recorded, ascending
+    if (fits) {
+      uint32_t low = 0;
+      for (uint32_t k = g; k < n; k += G) low += (el_i[o][k] < idi) ? 1u : 0u;
+      low = (uint32_t)dpp_group_sum_i<G>((int)low);
+      for (uint32_t k = g; k < n; k += G) {
+        const uint32_t ik = el_i[o][k];
+        if (ik < idi) continue;
+        uint32_t below = 0;
+        for (uint32_t k2 = 0; k2 < n; ++k2) below += (el_i[o][k2] < ik) ? 1u : 0u;
+        if (below < (uint32_t)cap) a.estage[(long)idi * a.estride + (below - low)] = ik;
+      }
+      above = min(n, (uint32_t)cap) - min(low, (uint32_t)cap);
+    }
+  }
   // phase 1: keep the `cap` smallest indices (the reference's first 2*maxC by index, :215)
-  if (fits)
+  if (!MESH && fits)
     for (uint32_t k = g; k < n; k += G) {
       const uint32_t ik = el_i[o][k];
       uint32_t below = 0;
@@ -2233,7 +2269,7 @@ __device__ __forceinline__ void edges_owner(const EdgeArgs& a, const SimDesc& sd
     }
   wave_lds_sync();
   // phase 2: rank the kept ones by (d^2, index), keep the first maxC (:235-246)
-  if (fits)
+  if (!MESH && fits)
     for (uint32_t k = g; k < n; k += G) {
       const float2 dk = el_d[o][k];
       if (dk.y == 0.0f) continue;
@@ -2258,9 +2294,10 @@ __device__ __forceinline__ void edges_owner(const EdgeArgs& a, const SimDesc& sd
     const uint32_t myid = a.id[so];
     WaveSel sel{&el_d[0][0], 0, 0xFFFFFFFFu};
     if constexpr (ER == 1) {
-      wave_sel_runs<false>(sel, a.pos, a.id, el_r[L / G], 9, me, myid, sd, false, cap, lane);
+      wave_sel_runs<false, MESH>(sel, a.pos, a.id, el_r[L / G], 9, me, myid, sd, false, cap,
+                                 lane);
     } else {
-      // 64 rows at a time, one per lane, listed in el_i's place
+      // 64 rows at a time, one per lane, those that hold slots listed in el_i's place
       uint2* rows = reinterpret_cast<uint2*>(&el_i[0][0]);
       for (int r0 = 0; r0 < nrows; r0 += kWave) {
         const int r = r0 + lane;
@@ -2275,22 +2312,31 @@ __device__ __forceinline__ void edges_owner(const EdgeArgs& a, const SimDesc& sd
           e.x = a.start[c0];
           e.y = a.start[c1 + 1] - e.x;
         }
+        const unsigned long long some = __ballot(e.y != 0u);
         wave_lds_sync();
-        rows[lane] = e;
+        if (e.y != 0u) rows[__popcll(some & ((1ull << lane) - 1ull))] = e;
         wave_lds_sync();
-        wave_sel_runs<false>(sel, a.pos, a.id, rows, min(kWave, nrows - r0), me, myid, sd, false,
-                             cap, lane);
+        wave_sel_runs<false, MESH>(sel, a.pos, a.id, rows, __popcll(some), me, myid, sd, false,
+                                   cap, lane);
       }
     }
-    const uint32_t e = wave_sel_finish(sel, cap, maxc, a.estage + (long)myid * a.estride, lane);
+    uint32_t* rec = a.estage + (long)myid * a.estride;
+    const uint32_t e = MESH ? wave_sel_above(sel, cap, myid, rec, lane)
+                            : wave_sel_finish(sel, cap, maxc, rec, lane);
     if (lane == L) ovf_e = e;
   }
   if (!active || g != 0) return;
+  if constexpr (MESH) {
+    if (!fits) above = ovf_e;
+    a.nabove[idi] = above;
+    a.ecount[idi] = min(64u, above * (above - (above != 0u ? 1u : 0u)) / 2u);  // :334-348
+    return;
+  }
   const uint32_t e = fits ? (uint32_t)min(min((int)n, cap), maxc) : ovf_e;
   if (e) a.ecount[idi] = e;  // zero already: the edge tiles that read the counts clear them
 }
 
-template <int ER>
+template <int ER, bool MESH = false>
 __device__ __forceinline__ void edges_body(const EdgeArgs& a) {
   constexpr int G = kEdgeLanes;
   constexpr int kOwn = kWave / G;
@@ -2308,7 +2354,13 @@ __device__ __forceinline__ void edges_body(const EdgeArgs& a) {
   const int o = lane / G, g = lane % G;
   const int p = (int)base + o;
   const int s = __builtin_amdgcn_readfirstlane(wave_ok ? (int)a.wave_sim[base / kWave] : 0);
-  const SimDesc sd = a.sims[s];
+  SimDesc sd = a.sims[s];
+  if constexpr (MESH) {  // the mesh's own distance
+    sd.edge_d2 = a.d2;
+    sd.edge_rx = a.rx;
+    sd.edge_ry = a.ry;
+    sd.edge_rz = a.rz;
+  }
   const bool active = wave_ok && (p - sd.p0) < sd.n;
   float4 pi = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   uint32_t idi = 0;
@@ -2316,7 +2368,7 @@ __device__ __forceinline__ void edges_body(const EdgeArgs& a) {
     pi = a.pos[p];
     idi = a.id[p];
   }
-  edges_owner<ER>(a, sd, o, g, lane, (int)base, active, pi, idi, el_d[wv], el_i[wv], el_n[wv],
+  edges_owner<ER, MESH>(a, sd, o, g, lane, (int)base, active, pi, idi, el_d[wv], el_i[wv], el_n[wv],
                   el_r[wv]);
 }
 
@@ -3289,82 +3341,51 @@ __global__ void k_line_vertices(LineArgs a) {
 // the first maxc particles j != i of its type, in index order, whose non-periodic squared
 // distance is below d2 (:306-324), that is the maxc smallest such indices; its triangles are
 // (i, a, b) for the pairs a < b of that list with i < a, in list order, at most 64
-// (:334-348).  The owners are visited by slot over a non-periodic stencil.
+// (:334-348).
+//
+// k_tri_count is the graph pass's walk (k_edges_g) with the mesh's selection: kept
+// neighbours above the owner's index, ascending, by owner index, and the owner's number of
+// triangles.  Bound: latency, as the graph pass (50k in clumps of 62: 95 us with a lane per
+// owner and its list in memory, 17.6 now; 20k in four blobs, hundreds of partners each:
+// 4-5 ms per mesh, 0.5 now).
+// k_tri_write: one wave per 64 owners, whose triangles are one run of the output, one lane
+// per triangle, so the writes are contiguous (a lane per owner wrote up to 64 triangles in a
+// row, each lane to places of its own: 15.5 us for 285k triangles, 6.8 now).
 
-__global__ void __launch_bounds__(256) k_tri_count(TriArgs a) {
-  const int lane = threadIdx.x & (kWave - 1);
-  const int gw = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (gw >= a.nwaves) return;
-  const SimDesc sd = a.sims[a.wave_sim[gw]];
-  const int p = gw * kWave + lane;
-  if (p - sd.p0 >= sd.n) return;
-  const float4 pi = a.pos[p];
-  const uint32_t idi = a.id[p];
-  const uint32_t ti = __float_as_uint(pi.w);
-  const int cx = bin_axis(pi.x, sd.ihx, sd.nx);
-  const int cy = bin_axis(pi.y, sd.ihy, sd.ny);
-  const int cz = bin_axis(pi.z, sd.ihz, sd.nz);
-  const int xlo = max(cx - a.rx, 0), xhi = min(cx + a.rx, sd.nx - 1);
-  const int ylo = max(cy - a.ry, 0), yhi = min(cy + a.ry, sd.ny - 1);
-  const int zlo = max(cz - a.rz, 0), zhi = min(cz + a.rz, sd.nz - 1);
-  EdgeAcc ea;
-  ea.q = 0;
-  ea.maxid = 0;
-  ea.maxk = 0;
-  for (int z = zlo; z <= zhi; ++z)
-    for (int y = ylo; y <= yhi; ++y) {
-      const int rowc = sd.c0 + sd.nx * (y + sd.ny * z);
-      const int q0 = (int)a.start[rowc + xlo];
-      const int q1 = (int)a.start[rowc + xhi + 1];
-      for (int q = q0; q < q1; ++q) {
-        if (q == p) continue;                             // :307
-        const float4 pj = a.pos[q];
-        if (__float_as_uint(pj.w) != ti) continue;       // :311
-        const float dx = pj.x - pi.x;                     // :314-317
-        const float dy = pj.y - pi.y;
-        const float dz = pj.z - pi.z;
-        const float s2 = fmaf(dz, dz, fmaf(dy, dy, dx * dx));
-        if (!(s2 < a.d2)) continue;                       // :319
-        edge_push(ea, s2, a.id[q], a.maxc, a.cand_d2, a.cand_id, a.P, p);
-      }
-    }
-  // the kept indices in ascending order (distinct, so rank by counting), and the owner's
-  // triangles: pairs among the kept indices above its own
-  const int m = min(ea.q, a.maxc);
-  int above = 0;
-  for (int k = 0; k < m; ++k) {
-    const uint32_t ik = a.cand_id[(long)k * a.P + p];
-    int rank = 0;
-    for (int k2 = 0; k2 < m; ++k2) rank += (a.cand_id[(long)k2 * a.P + p] < ik) ? 1 : 0;
-    a.sorted[(long)rank * a.P + p] = ik;
-    above += (ik > idi) ? 1 : 0;
-  }
-  a.nsel[p] = (uint32_t)m;
-  a.count[idi] = (uint32_t)min(64, above * (above - 1) / 2);
-}
+__global__ void __launch_bounds__(256) k_tri_count(EdgeArgs a) { edges_body<1, true>(a); }
+__global__ void __launch_bounds__(256) k_tri_count_far(EdgeArgs a) { edges_body<0, true>(a); }
 
 __global__ void __launch_bounds__(256) k_tri_write(TriArgs a) {
+  __shared__ uint32_t first[4][kWave];  // each owner's first triangle within the wave's run
   const int lane = threadIdx.x & (kWave - 1);
-  const int gw = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (gw >= a.nwaves) return;
-  const SimDesc sd = a.sims[a.wave_sim[gw]];
-  const int p = gw * kWave + lane;
-  if (p - sd.p0 >= sd.n) return;
-  const uint32_t idi = a.id[p];
-  const uint32_t nt = a.count[idi];
-  if (nt == 0u) return;
-  const int m = (int)a.nsel[p];
-  int s0 = 0;  // the first kept index above the owner's
-  while (s0 < m && a.sorted[(long)s0 * a.P + p] <= idi) ++s0;
-  long w = (long)a.off[idi];
-  uint32_t t = 0;
-  for (int i1 = s0; i1 < m && t < nt; ++i1) {
-    const uint32_t n1 = a.sorted[(long)i1 * a.P + p];
-    for (int i2 = i1 + 1; i2 < m && t < nt; ++i2, ++t, ++w) {
-      a.tris[3 * w] = (int32_t)idi - sd.p0;
-      a.tris[3 * w + 1] = (int32_t)n1 - sd.p0;
-      a.tris[3 * w + 2] = (int32_t)a.sorted[(long)i2 * a.P + p] - sd.p0;
-    }
+  const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const long k0 = ((long)blockIdx.x * 4 + wv) * kWave;
+  if (k0 >= a.n) return;
+  const long k = k0 + lane;
+  const uint32_t nt = k < a.n ? a.count[k] : 0u;
+  const uint32_t incl = wave_inclusive_scan(nt, lane);
+  const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+  first[wv][lane] = incl - nt;
+  wave_lds_sync();
+  const long w0 = (long)a.off[k0];
+  for (uint32_t t0 = 0; t0 < total; t0 += (uint32_t)kWave) {
+    const uint32_t t = t0 + (uint32_t)lane;
+    const long w = w0 + (long)t;
+    if (t >= total || w >= a.cap) continue;
+    // t's owner: the last whose first triangle is at or before t (owners without triangles
+    // share the next one's, which is later)
+    int lo = 0;
+#pragma unroll
+    for (int d = kWave / 2; d > 0; d >>= 1)
+      if (first[wv][lo + d] <= t) lo += d;
+    const long ko = k0 + lo;
+    const uint32_t m = a.nabove[ko];
+    uint32_t r = t - first[wv][lo], i1 = 0;  // the r-th pair of the owner's list
+    for (; r >= m - 1u - i1; ++i1) r -= m - 1u - i1;
+    const uint32_t* rec = a.rec + ko * a.estride;
+    a.tris[3 * w] = (int32_t)ko;
+    a.tris[3 * w + 1] = (int32_t)rec[i1];
+    a.tris[3 * w + 2] = (int32_t)rec[i1 + 1u + r];
   }
 }
 
@@ -3589,13 +3610,16 @@ hipError_t launch_rank_scatter(const SortArgs& a, hipStream_t st) {
   return hipGetLastError();
 }
 
-hipError_t launch_tri_count(const TriArgs& a, hipStream_t st) {
-  CF_LAUNCH(k_tri_count, dim3(grid_for(a.nwaves, 256)), dim3(256), 0, st, a);
+hipError_t launch_tri_count(const EdgeArgs& a, bool near, hipStream_t st) {
+  const dim3 g((a.nwaves * kEdgeLanes + 3) / 4), b(256);
+  if (near) CF_LAUNCH(k_tri_count, g, b, 0, st, a);
+  else CF_LAUNCH(k_tri_count_far, g, b, 0, st, a);
   return hipGetLastError();
 }
 
 hipError_t launch_tri_write(const TriArgs& a, hipStream_t st) {
-  CF_LAUNCH(k_tri_write, dim3(grid_for(a.nwaves, 256)), dim3(256), 0, st, a);
+  const long g = (a.n + 4 * kWave - 1) / (4 * kWave);
+  if (g > 0) CF_LAUNCH(k_tri_write, dim3((unsigned)g), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 
