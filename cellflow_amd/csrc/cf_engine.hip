@@ -754,6 +754,7 @@ struct Engine {
     fa.ecount = b.fcount;
     fa.P = P;
     fa.nwaves = nwaves;
+    fa.one_sim = sims.size() == 1 ? 1 : 0;
     fa.edges = edges ? 1 : 0;
     fa.edge_cap = cap;
     fa.tile_sort = tun.sort_variant == 1 ? 1 : 0;

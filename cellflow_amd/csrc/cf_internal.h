@@ -167,6 +167,7 @@ struct ForceArgs {
   long P;
   long estride;     // words per owner record in estage (the largest maxc allocated)
   int nwaves;
+  int one_sim;      // 1: the only simulation (wave_sim is all 0)
   int edges;        // fused edge candidates requested for this launch
   int edge_cap;
   // 1: the tile sort follows (keys with kFarBit, tile counts, far lists, estage by owner

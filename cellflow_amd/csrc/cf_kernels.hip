@@ -1244,16 +1244,21 @@ __global__ void __launch_bounds__(256) k_force_grp(ForceArgs a) {
 // lanes 8 apart and keeps two sums.  A wave with more than kWalkFrom candidates walks the
 // runs from a table in the list's place, 16 lanes per particle: building a list costs
 // about as much as the pairs it saves once runs are long.
-// Bound: instruction issue (the same pairs in about half of k_force_grp's instructions).
+// Bound: instruction issue (the same pairs in about half of k_force_grp's instructions),
+// then latency: a wave lives for a handful of loads that wait for each other.
 // Measured against k_force_grp<16> (uniform states at 12,500 per unit volume, us per
-// launch): 1k 10.1 -> 5.8, 20k 11.6 -> 7.1, 100k 35 -> 18.4, 100k with edges 46.5 -> 24,
-// the same after 300 steps 48.5 -> 32, 500k 142 -> 71; 1M clustered (238 neighbours) with
-// edges 1171 -> 584, without 485 -> 400; 20k of a preset (516 neighbours) 82 -> 64 (the walk
+// launch): 1k 10.1 -> 5.7, 20k 11.6 -> 7, 100k 35 -> 17.9, 100k with edges 46.5 -> 23.2,
+// the same after 300 steps 48.5 -> 27.4, 500k 142 -> 66; 1M clustered (238 neighbours) with
+// edges 1171 -> 550, without 485 -> 385; 20k of a preset (516 neighbours) 82 -> 62.5 (the walk
 // with an index per candidate, one candidate per turn and a select per image shift: 640,
 // 435 and 79).
+// Edge candidates are listed by slot alone, and their indices read once the pair loops are
+// done: an index loaded with every candidate, or waited for at each edge candidate, cost
+// 31.7 against 27.1 us on the 100k state after 300 steps (variant 4 there: 29.6 -> 26.5).
 
 constexpr int kWaveList = 640;  // candidate slots per wave
-constexpr int kListEdges = 24;  // LDS edge candidates per particle (more: the wave selects)
+constexpr int kListEdges = 24;  // LDS edge candidates per owner (more: the wave selects)
+constexpr int kForceEdges = 64; // the force pass's, of either index
 
 // The proximity-graph partners of one owner with more candidates than its LDS list holds,
 // chosen by the whole wave: its lanes walk the owner's slot runs together and append the
@@ -1492,10 +1497,11 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
   // list entries: slot | image-shift code << kCodeShift (slots stay below 2^kCodeShift),
   // the wave's particles one after another
   __shared__ __align__(16) uint32_t lslot[4][kWaveList];
-  // edge candidates listed per particle; together at least the wave selection's list
-  constexpr int kLE = kSelCap / kOwn > kListEdges ? kSelCap / kOwn : kListEdges;
-  __shared__ float2 el_d[EDGES ? 4 : 1][EDGES ? kOwn : 1][EDGES ? kLE : 1];
-  __shared__ __align__(8) uint32_t el_i[EDGES ? 4 : 1][EDGES ? kOwn : 1][EDGES ? kLE : 1];
+  // edge candidates of a particle: kLE slots of either index in the pair loops, then, in the
+  // candidate list's place, the kLV or fewer of them with the larger index (d^2, index)
+  constexpr int kLE = kForceEdges;
+  constexpr int kLV = kWaveList / kOwn / 2 < kLE ? kWaveList / kOwn / 2 : kLE;
+  __shared__ uint32_t el_q[EDGES ? 4 : 1][EDGES ? kOwn : 1][EDGES ? kLE : 1];
   __shared__ uint32_t el_n[4][kOwn];
   __shared__ uint32_t hl[HITS ? 4 : 1][HITS ? kOwn : 1][HITS ? kPairList : 1];
   __shared__ uint32_t hn[HITS ? 4 : 1][HITS ? kOwn : 1];
@@ -1503,36 +1509,35 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
   __shared__ uint32_t cedge[CONS ? 4 * kOwn : 1];  // kept edges | active << 30 | edges << 31
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int gw = xcd_block() * (blockDim.x >> 6) + wv;
-  const long base = (long)gw * kOwn;
-  const bool wave_ok = base < (long)a.nwaves * kWave;
+  // The chain of loads that every wave waits for is kept short (four deep: arguments; state
+  // and descriptor; pruning radius and pair table; cell starts): the block size is a constant,
+  // not the implicit argument (a load of its own), a wave past the end reads the last wave's
+  // particles, so that no load stands behind a branch, and the only simulation is number 0.
+  const int gw = xcd_block() * 4 + wv;
+  const int nw = a.nwaves * (kWave / kOwn);
+  const bool wave_ok = gw < nw;
+  const long base = (long)min(gw, nw - 1) * kOwn;
   const int o = lane / G, g = lane % G;
   const int p = (int)base + o;
   // the slot's state loads do not wait for the descriptor: every slot below nwaves * 64
   // is allocated (a padding slot's values are loaded but never used)
   Own c;
-  float4 vi = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  uint32_t idi = 0;
-  c.pi = vi;
-  if (wave_ok) {
-    c.pi = a.pos[p];
-    vi = a.vel[p];
-    idi = a.id[p];
-  }
-  const int s = __builtin_amdgcn_readfirstlane(wave_ok ? (int)a.wave_sim[base / kWave] : 0);
+  c.pi = a.pos[p];
+  const float4 vi = a.vel[p];
+  const uint32_t idi = a.id[p];
+  const int s = a.one_sim ? 0 : __builtin_amdgcn_readfirstlane((int)a.wave_sim[base / kWave]);
   const SimDesc sd = a.sims[s];
-  if (wave_ok)
-    for (int t = lane; t < sd.T * sd.T; t += kWave) {
-      const PairConst pt = a.pairs[sd.tab + t];
-      ptab[t] = pt.thr;
-      ptab[kTT + t] = sd.rep * pt.fv;
-      ptab[2 * kTT + t] = sd.att * pt.fv * pt.inv_eff;
-      ptab[3 * kTT + t] = sd.kexp2 * pt.inv_eff * pt.inv_eff;
-    }
+  // the pair table's first kWave entries; they go to LDS when the runs are built
+  const int ntab = sd.T * sd.T;
+  const PairConst pt0 = a.pairs[sd.tab + min(lane, ntab - 1)];
   const bool active = wave_ok && (p - sd.p0) < sd.n;
   const float4 pi = c.pi;
   c.ti = active ? __float_as_uint(pi.w) : 0u;
   const uint32_t ti = c.ti;
+  // the pruning radius straight from the pair table in memory, so the stencil rows (and
+  // their cell-start loads) overlap the copy of the table into LDS
+  const float reach2 = a.pairs[sd.tab + ti * sd.T].pad;
+  c.cut2 = active ? reach2 : 0.0f;
   c.cx = bin_axis(pi.x, sd.ihx, sd.nx);
   c.cy = bin_axis(pi.y, sd.ihy, sd.ny);
   c.cz = bin_axis(pi.z, sd.ihz, sd.nz);
@@ -1546,9 +1551,6 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
   own_gaps<R>(c, sd);
   if (EDGES && g == 0) el_n[wv][o] = 0u;
   if (HITS && g == 0) hn[wv][o] = 0u;
-  // the pruning radius straight from the pair table in memory, so the stencil rows (and
-  // their cell-start loads) overlap the copy of the table into LDS
-  c.cut2 = active ? a.pairs[sd.tab + ti * sd.T].pad : 0.0f;
 
   // ---- this lane's runs, their place in the particle's flattened candidate order ----
   uint32_t rs[2 * kRpl], rl[2 * kRpl], rk[2 * kRpl];
@@ -1610,6 +1612,16 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
   const bool packed = wave_total <= (uint32_t)kWaveList;
   const uint32_t obase = packed ? incl - total : (uint32_t)o * kQuota;
   const uint32_t quota = packed ? (uint32_t)kWaveList : kQuota;
+  {
+    auto put = [&](int t, const PairConst& pc) {
+      ptab[t] = pc.thr;
+      ptab[kTT + t] = sd.rep * pc.fv;
+      ptab[2 * kTT + t] = sd.att * pc.fv * pc.inv_eff;
+      ptab[3 * kTT + t] = sd.kexp2 * pc.inv_eff * pc.inv_eff;
+    };
+    if (lane < ntab) put(lane, pt0);
+    for (int t = lane + kWave; t < ntab; t += kWave) put(t, a.pairs[sd.tab + t]);
+  }
   wave_lds_sync();  // pair table ready
   const float* row = &ptab[ti * sd.T];
 
@@ -1625,21 +1637,19 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
   // the particle whose candidates this lane takes (its own; in the dense walk at G = 8 one
   // of the wave's, 16 lanes each)
   float px = pi.x, py = pi.y, pz = pi.z;
-  uint32_t pt = ti, pid = idi;
+  uint32_t pt = ti;
   int ps = p, po = o;
-  bool pe = do_edges;
   const float* prow = row;
+  const float ed2 = want_edges ? sd.edge_d2 : -1.0f;  // (an inactive particle has no runs)
   auto swap_sums = [&]() {
     float t = fx; fx = hx; hx = t;
     t = fy; fy = hy; hy = t;
     t = fz; fz = hz; hz = t;
   };
   // ParticleSimulation.cu:92-131 for candidate q: cutoff, count, force, edge candidate.
-  // code: image shift of a shifted run (0: none); jq: the candidate's index where HAVE_ID
-  auto pair = [&](auto gen_kind, auto have_id, uint32_t q, uint32_t code, const float4& pj,
-                  uint32_t jq) {
+  // code: image shift of a shifted run (0: none)
+  auto pair = [&](auto gen_kind, uint32_t q, uint32_t code, const float4& pj) {
     constexpr bool GEN = decltype(gen_kind)::value;
-    constexpr bool HAVE_ID = decltype(have_id)::value;
     float dx = pj.x - px, dy = pj.y - py, dz = pj.z - pz;
     bool raw;
     if constexpr (!GEN) {
@@ -1678,17 +1688,13 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
       }
     }
     if (EDGES) {
-      // edges are non-periodic (ParticleSimulation.cu:222-227): unshifted pairs only
-      if (pe && raw && tj == pt && s2 < sd.edge_d2) {
-        const uint32_t jid = HAVE_ID ? jq : a.id[q];
-        if (jid > pid) {
+      // edges are non-periodic (ParticleSimulation.cu:222-227): unshifted pairs only.  The
+      // slot alone is listed: its index would be a load to wait for here
+      if (__builtin_expect(s2 < ed2 && tj == pt, 0))  // rare: the other tests behind a branch
+        if (raw && q != (uint32_t)ps) {
           const uint32_t kk = atomicAdd(&el_n[wv][po], 1u);
-          if (kk < (uint32_t)kLE) {
-            el_d[wv][po][kk] = make_float2(s2, 0.0f);
-            el_i[wv][po][kk] = jid;
-          }
+          if (kk < (uint32_t)kLE) el_q[wv][po][kk] = q;
         }
-      }
     }
   };
   const bool walk = V != 0 && wave_total > kWalkFrom;
@@ -1724,13 +1730,11 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
         if (G != 16) {
           po = b4 + (lane >> 4);
           ps = (int)base + po;
-          pe = want_edges;  // an inactive particle has no runs
           const float4 pw = a.pos[ps];
           px = pw.x;
           py = pw.y;
           pz = pw.z;
           pt = ps - sd.p0 < sd.n ? __float_as_uint(pw.w) : 0u;
-          pid = a.id[ps];
           prow = &ptab[pt * sd.T];
           fx = fy = fz = 0.0f;
           cnt = 0;
@@ -1753,16 +1757,24 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
             auto lane_run = [&](uint32_t run_code) {
               constexpr uint32_t kStep = 16u * (uint32_t)sizeof(float4);
               const uint32_t end = (q0 + len - 1u) * (uint32_t)sizeof(float4);
-              uint32_t off = (q0 + t) * (uint32_t)sizeof(float4);
+              // each address is made one candidate before its load (an address made at the load
+              // may take a register of the load still in flight, and wait for it)
+              uint32_t off = (q0 + t) * (uint32_t)sizeof(float4), next = min(off + kStep, end);
+              auto pin = [&]() { asm volatile("" : "+v"(next)); };
               float4 p0 = at(off);
+              pin();
               while (true) {
-                const uint32_t off1 = off + kStep;
-                const float4 p1 = at(min(off1, end));
-                pair(gen_kind, std::false_type{}, off / (uint32_t)sizeof(float4), run_code, p0, 0u);
-                if (off1 > end) break;
-                off = off1 + kStep;
-                p0 = at(min(off, end));
-                pair(gen_kind, std::false_type{}, off1 / (uint32_t)sizeof(float4), run_code, p1, 0u);
+                const float4 p1 = at(next);
+                next = min(off + 2u * kStep, end);
+                pin();
+                pair(gen_kind, off / (uint32_t)sizeof(float4), run_code, p0);
+                off += kStep;
+                if (off > end) break;
+                p0 = at(next);
+                next = min(off + 2u * kStep, end);
+                pin();
+                pair(gen_kind, off / (uint32_t)sizeof(float4), run_code, p1);
+                off += kStep;
                 if (off > end) break;
               }
             };
@@ -1828,10 +1840,8 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
         for (uint32_t k = (uint32_t)(gv + h * G); k < nb; k += (uint32_t)VL) {
           const uint32_t e = lslot[wv][obase + k];
           const uint32_t q = e & ((1u << kCodeShift) - 1u);
-          const float4 pj = a.pos[q];
-          // the index travels with the position: an edge candidate then waits for no load
-          const uint32_t jq = want_edges ? a.id[q] : 0u;
-          pair(gen_kind, std::true_type{}, q, e >> kCodeShift, pj, jq);
+          const float4 pj = a.pos[q];  // one load (not a reference: that reads it in parts)
+          pair(gen_kind, q, e >> kCodeShift, pj);
         }
         if (kSub > 1) swap_sums();
       }
@@ -1882,45 +1892,76 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
 
   uint32_t ekept = 0u;  // kept edges of the particle (lane g == 0), passed on by CONS
   if (EDGES) {
-    // the wave's candidate lists are complete
+    // the wave's candidate lists are complete, and the candidate list's place is free
     wave_lds_sync();
-    const uint32_t n = do_edges ? el_n[wv][o] : 0u;
-    const bool fits = n <= (uint32_t)kLE;
+    const uint32_t nq = do_edges ? el_n[wv][o] : 0u;
     const int cap = a.edge_cap, maxc = sd.edge_maxc;
-    // the owner's record: by index when the tile sort follows, else by slot
-    const uint32_t orec = TILE ? idi : (uint32_t)p;
-    if (fits)
-      for (uint32_t k = g; k < n; k += G) {
-        const uint32_t ik = el_i[wv][o][k];
-        uint32_t below = 0;
-        for (uint32_t k2 = 0; k2 < n; ++k2) below += (el_i[wv][o][k2] < ik) ? 1u : 0u;
-        el_d[wv][o][k].y = (below < (uint32_t)cap) ? 1.0f : 0.0f;
-      }
-    wave_lds_sync();
-    if (fits)
-      for (uint32_t k = g; k < n; k += G) {
-        const float2 dk = el_d[wv][o][k];
-        if (dk.y == 0.0f) continue;
-        const uint32_t ik = el_i[wv][o][k];
-        uint32_t rank = 0;
-        for (uint32_t k2 = 0; k2 < n; ++k2) {
-          const float2 d2 = el_d[wv][o][k2];
-          const uint32_t i2 = el_i[wv][o][k2];
-          rank += (d2.y != 0.0f && (d2.x < dk.x || (d2.x == dk.x && i2 < ik))) ? 1u : 0u;
+    float2* const lv = reinterpret_cast<float2*>(&lslot[wv][0]);
+    float2* const mv = lv + o * kLV;
+    uint32_t n = 0u;  // candidates with the larger index (j > i, :215)
+    uint32_t ovf_e = 0u;  // kept edges of an owner the whole wave chose for (its lane g == 0)
+    bool fits = true;
+    if (__any(nq != 0u)) {
+      const float4 me = nq != 0u ? a.pos[p] : pi;
+      fits = nq <= (uint32_t)kLE;
+      const uint32_t ne = fits ? nq : 0u;
+      for (uint32_t k = g; __any(k < ne); k += G) {
+        bool up = false;
+        float2 e = make_float2(0.0f, 0.0f);
+        if (k < ne) {
+          const uint32_t q = el_q[wv][o][k];
+          const float4 pj = a.pos[q];
+          const uint32_t jid = a.id[q];
+          const float ux = pj.x - me.x, uy = pj.y - me.y, uz = pj.z - me.z;
+          e = make_float2(fmaf(uz, uz, fmaf(uy, uy, ux * ux)), __uint_as_float(jid));
+          up = jid > idi;
         }
-        if (rank < (uint32_t)maxc)
-          a.estage[(long)orec * a.estride + rank] = ik;
+        const unsigned long long m = (__ballot(up) >> (o * G)) & ((1ull << G) - 1ull);
+        const uint32_t at = n + (uint32_t)__popcll(m & ((1ull << g) - 1ull));
+        if (up && at < (uint32_t)kLV) mv[at] = e;
+        n += (uint32_t)__popcll(m);
       }
-    // Owners with more candidates than their LDS list holds (n counts them all): the whole
-    // wave takes them one at a time, in the wave's LDS lists (free then: every fitting
-    // owner's selection above is done)
-    uint32_t ovf_e = 0u;  // kept edges of an owner this handled (its lane g == 0)
-    {
-      static_assert(kOwn * kLE >= kSelCap, "the selection fits the wave's el_d");
-      static_assert(G * 2 * kRpl * 2 <= kOwn * kLE, "an owner's runs fit the wave's el_i");
-      uint2* ov_r = reinterpret_cast<uint2*>(&el_i[wv][0][0]);
+      fits = fits && n <= (uint32_t)kLV;
+      wave_lds_sync();
+      // the `cap` smallest indices (the reference's first 2*maxC by index, :215): the others'
+      // distances are made negative
+      if (__any(fits && n > (uint32_t)cap)) {
+        if (fits)
+          for (uint32_t k = g; k < n; k += G) {
+            const float ik = mv[k].y;
+            uint32_t below = 0;
+            for (uint32_t k2 = 0; k2 < n; ++k2)
+              below += (__float_as_uint(mv[k2].y) < __float_as_uint(ik)) ? 1u : 0u;
+            if (below >= (uint32_t)cap) mv[k].x = -1.0f;
+          }
+        wave_lds_sync();
+      }
+      // ranked by (d^2, index), the first maxC kept (:235-246).  The owner's record: by
+      // index when the tile sort follows, else by slot
+      const uint32_t orec = TILE ? idi : (uint32_t)p;
+      if (fits)
+        for (uint32_t k = g; k < n; k += G) {
+          const float2 ek = mv[k];
+          if (ek.x < 0.0f) continue;
+          uint32_t rank = 0;
+          for (uint32_t k2 = 0; k2 < n; ++k2) {
+            const float2 f = mv[k2];
+            rank += (f.x >= 0.0f &&
+                     (f.x < ek.x ||
+                      (f.x == ek.x && __float_as_uint(f.y) < __float_as_uint(ek.y))))
+                        ? 1u
+                        : 0u;
+          }
+          if (rank < (uint32_t)maxc)
+            a.estage[(long)orec * a.estride + rank] = __float_as_uint(ek.y);
+        }
+      // Owners with more candidates than their lists hold: the whole wave takes them one at a
+      // time, in the same place (free then: every fitting owner's selection above is done)
+      static_assert(2 * kSelCap + G * 2 * kRpl * 2 <= kWaveList,
+                    "the selection and an owner's runs fit the candidate list");
+      uint2* ov_r = reinterpret_cast<uint2*>(&lslot[wv][2 * kSelCap]);
       unsigned long long left = __ballot(do_edges && g == 0 && !fits);
-      if (left) wave_lds_sync();  // the fitting owners' reads of el_d, el_i are done
+      if (left) wave_lds_sync();  // the fitting owners' reads are done
       while (left) {
         const int L = __ffsll((long long)left) - 1;
         left &= left - 1ull;
@@ -1933,7 +1974,7 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
         const int so = __builtin_amdgcn_readfirstlane((int)base + os);
         const float4 me = a.pos[so];
         const uint32_t myid = a.id[so];
-        WaveSel sel{&el_d[wv][0][0], 0, 0xFFFFFFFFu};
+        WaveSel sel{lv, 0, 0xFFFFFFFFu};
         wave_sel_runs<true>(sel, a.pos, a.id, ov_r, G * 2 * kRpl, me, myid, sd, c.gen, cap, lane);
         const uint32_t e = wave_sel_finish(
             sel, cap, maxc, a.estage + (long)(TILE ? myid : (uint32_t)so) * a.estride, lane);
