@@ -1247,9 +1247,9 @@ __global__ void __launch_bounds__(256) k_force_grp(ForceArgs a) {
 // Bound: instruction issue (the same pairs in about half of k_force_grp's instructions),
 // then latency: a wave lives for a handful of loads that wait for each other.
 // Measured against k_force_grp<16> (uniform states at 12,500 per unit volume, us per
-// launch): 1k 10.1 -> 5.7, 20k 11.6 -> 7, 100k 35 -> 17.9, 100k with edges 46.5 -> 23.2,
+// launch): 1k 10.1 -> 5.7, 20k 11.6 -> 7, 100k 35 -> 17.9, 100k with edges 46.5 -> 22.5,
 // the same after 300 steps 48.5 -> 27.4, 500k 142 -> 66; 1M clustered (238 neighbours) with
-// edges 1171 -> 550, without 485 -> 385; 20k of a preset (516 neighbours) 82 -> 62.5 (the walk
+// edges 1171 -> 530, without 485 -> 385; 20k of a preset (516 neighbours) 82 -> 62.5 (the walk
 // with an index per candidate, one candidate per turn and a select per image shift: 640,
 // 435 and 79).
 // Edge candidates are listed by slot alone, and their indices read once the pair loops are
@@ -1902,7 +1902,8 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
     uint32_t ovf_e = 0u;  // kept edges of an owner the whole wave chose for (its lane g == 0)
     bool fits = true;
     if (__any(nq != 0u)) {
-      const float4 me = nq != 0u ? a.pos[p] : pi;
+      const float4 me = a.pos[p];  // again: they take no registers until here
+      const uint32_t myid = a.id[p];
       fits = nq <= (uint32_t)kLE;
       const uint32_t ne = fits ? nq : 0u;
       for (uint32_t k = g; __any(k < ne); k += G) {
@@ -1914,7 +1915,7 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
           const uint32_t jid = a.id[q];
           const float ux = pj.x - me.x, uy = pj.y - me.y, uz = pj.z - me.z;
           e = make_float2(fmaf(uz, uz, fmaf(uy, uy, ux * ux)), __uint_as_float(jid));
-          up = jid > idi;
+          up = jid > myid;
         }
         const unsigned long long m = (__ballot(up) >> (o * G)) & ((1ull << G) - 1ull);
         const uint32_t at = n + (uint32_t)__popcll(m & ((1ull << g) - 1ull));
@@ -1938,7 +1939,7 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
       }
       // ranked by (d^2, index), the first maxC kept (:235-246).  The owner's record: by
       // index when the tile sort follows, else by slot
-      const uint32_t orec = TILE ? idi : (uint32_t)p;
+      const uint32_t orec = TILE ? myid : (uint32_t)p;
       if (fits)
         for (uint32_t k = g; k < n; k += G) {
           const float2 ek = mv[k];
@@ -1970,14 +1971,14 @@ __device__ __forceinline__ void force_list(const ForceArgs& a) {
 #pragma unroll
           for (int k = 0; k < 2 * kRpl; ++k) ov_r[g * 2 * kRpl + k] = make_uint2(rs[k], rl[k]);
         wave_lds_sync();
-        // the owner's state again, at a uniform address: it takes no registers until here
+        // the owner's state, at a uniform address
         const int so = __builtin_amdgcn_readfirstlane((int)base + os);
-        const float4 me = a.pos[so];
-        const uint32_t myid = a.id[so];
+        const float4 po4 = a.pos[so];
+        const uint32_t ido = a.id[so];
         WaveSel sel{lv, 0, 0xFFFFFFFFu};
-        wave_sel_runs<true>(sel, a.pos, a.id, ov_r, G * 2 * kRpl, me, myid, sd, c.gen, cap, lane);
+        wave_sel_runs<true>(sel, a.pos, a.id, ov_r, G * 2 * kRpl, po4, ido, sd, c.gen, cap, lane);
         const uint32_t e = wave_sel_finish(
-            sel, cap, maxc, a.estage + (long)(TILE ? myid : (uint32_t)so) * a.estride, lane);
+            sel, cap, maxc, a.estage + (long)(TILE ? ido : (uint32_t)so) * a.estride, lane);
         if (lane == L) ovf_e = e;
       }
     }
