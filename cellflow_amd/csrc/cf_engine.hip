@@ -646,6 +646,7 @@ struct Engine {
     sa.wave_sim = b.wave_sim;
     sa.P = P;
     sa.nwaves = nwaves;
+    sa.one_sim = sims.size() == 1 ? 1 : 0;
     HIPR(launch_fill(sa, st));
     HIPR(launch_rank_scatter(sa, st));
     return CF_OK;
@@ -794,6 +795,7 @@ struct Engine {
     }
     sa.P = P;
     sa.nwaves = nwaves;
+    sa.one_sim = sims.size() == 1 ? 1 : 0;
     return sa;
   }
 
@@ -908,6 +910,7 @@ struct Engine {
     ea.estride = edge_maxc_alloc;
     ea.ecount = b.fcount;
     ea.nwaves = nwaves;
+    ea.one_sim = sims.size() == 1 ? 1 : 0;
     ea.edge_cap = cap;
     bool near = true;
     for (const SimDesc& d : hdesc)
@@ -1288,6 +1291,7 @@ struct Engine {
     ea.ecount = b.ecount;
     ea.nabove = b.tmp_id;
     ea.nwaves = nwaves;
+    ea.one_sim = sims.size() == 1 ? 1 : 0;
     ea.edge_cap = maxc;
     ea.d2 = d2;
     // cells within reach of sqrt(d2) on each axis (non-periodic, as :314-317), at most the

@@ -199,6 +199,7 @@ struct EdgeArgs {
                         // passes: the edge tiles clear what they read)
   long estride;
   int nwaves;
+  int one_sim;          // 1: the only simulation (wave_sim is all 0)
   int edge_cap;
   // the triangle mesh only: its squared distance, its reach in cells (non-periodic) and, per
   // owner index, the kept partners above the owner (estage holds those; ecount the triangles)
@@ -230,6 +231,7 @@ struct SortArgs {
   long P;
   long estride;
   int nwaves;
+  int one_sim;          // 1: the only simulation (wave_sim is all 0)
 };
 
 // One step's sort after the force pass (k_tile_sort): blocks [0, ntiles) each place the

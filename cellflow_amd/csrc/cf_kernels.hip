@@ -2051,8 +2051,8 @@ k_force_ord(ForceArgs a) {
 // is chosen for by its whole wave (WaveSel).  Rows longer than kEdgeShare slots are shared by
 // the owner's lanes.  Kept partners are staged by owner index (estage[index * estride +
 // rank]), the non-zero per-owner counts go to `ecount`, and k_tile_sort's edge tiles write the
-// canonical list.  Bound: latency in sparse states (100k: 15.5 us), issue in dense ones (20k
-// of a preset, 516 neighbours: 55 -> 33 us; 1M clustered 1353 -> 290 us).
+// canonical list.  Bound: latency in sparse states (100k: 14.6 us), issue in dense ones (20k
+// of a preset, 516 neighbours: 55 -> 33 us; 1M clustered 1353 -> 284 us).
 
 constexpr int kEdgeLanes = 8;
 
@@ -2390,12 +2390,16 @@ __device__ __forceinline__ void edges_body(const EdgeArgs& a) {
   __shared__ uint2 el_r[4][kOwn][ER == 1 ? kEdgeRuns : 1];
   const int lane = threadIdx.x & (kWave - 1);
   const int wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int gw = xcd_block() * (blockDim.x >> 6) + wv;
-  const long base = (long)gw * kOwn;
-  const bool wave_ok = base < (long)a.nwaves * kWave;
+  // as the force kernels: no load behind a branch or a load that it does not need
+  const int gw = xcd_block() * 4 + wv;
+  const int nw = a.nwaves * (kWave / kOwn);
+  const bool wave_ok = gw < nw;
+  const long base = (long)min(gw, nw - 1) * kOwn;
   const int o = lane / G, g = lane % G;
   const int p = (int)base + o;
-  const int s = __builtin_amdgcn_readfirstlane(wave_ok ? (int)a.wave_sim[base / kWave] : 0);
+  const float4 pi = a.pos[p];
+  const uint32_t idi = a.id[p];
+  const int s = a.one_sim ? 0 : __builtin_amdgcn_readfirstlane((int)a.wave_sim[base / kWave]);
   SimDesc sd = a.sims[s];
   if constexpr (MESH) {  // the mesh's own distance
     sd.edge_d2 = a.d2;
@@ -2404,12 +2408,6 @@ __device__ __forceinline__ void edges_body(const EdgeArgs& a) {
     sd.edge_rz = a.rz;
   }
   const bool active = wave_ok && (p - sd.p0) < sd.n;
-  float4 pi = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  uint32_t idi = 0;
-  if (active) {
-    pi = a.pos[p];
-    idi = a.id[p];
-  }
   edges_owner<ER, MESH>(a, sd, o, g, lane, (int)base, active, pi, idi, el_d[wv], el_i[wv], el_n[wv],
                   el_r[wv]);
 }
@@ -3146,53 +3144,85 @@ __global__ void __launch_bounds__(kScanThreads) k_scan(ScanPlan plan) {
 
 // ------------------------------------------------------------------------------------
 // k_fill / k_rank_scatter: the two halves of the stable counting sort.
+//
+// Bound: latency (a lane's loads wait for each other: key, cell start, members or edges), and
+// for the ensemble's sizes the bandwidth of the scattered copy.  A wave's state loads wait
+// neither for the descriptor nor for each other, and the edges of an owner and the members of
+// a cell are read several at a time (us per launch, before -> now: k_rank_scatter 1M clustered
+// 61 -> 48, 60-member ensemble 28 -> 23.5; k_fill 1M clustered with edges 46 -> 42, without
+// 7.8 -> 7).
 
+// A wave's simulation, its slot's lane and whether a particle lives there.
+__device__ __forceinline__ bool sort_lane(const SortArgs& a, int gw, int p, SimDesc& sd) {
+  sd = a.sims[a.one_sim ? 0 : __builtin_amdgcn_readfirstlane((int)a.wave_sim[gw])];
+  return p - sd.p0 < sd.n;
+}
 
 __global__ void __launch_bounds__(256) k_fill(SortArgs a) {
-  const int gw = xcd_block() * (blockDim.x >> 6) + (threadIdx.x >> 6);
-  if (a.edges && gw == 0 && threadIdx.x % kWave == 0) *a.etotal = a.eoff[a.P];
+  const int gw = xcd_block() * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+  const int lane = threadIdx.x & (kWave - 1);
+  if (a.edges && gw == 0 && lane == 0) *a.etotal = a.eoff[a.P];
   if (gw >= a.nwaves) return;
-  const SimDesc sd = a.sims[a.wave_sim[gw]];
-  const int p = gw * kWave + (threadIdx.x & (kWave - 1));
-  if (p - sd.p0 >= sd.n) return;
-  const uint32_t c = a.key[p];
+  const int p = gw * kWave + lane;
+  const uint32_t key = a.key[p];
   const uint32_t me = a.src_id[p];
   const uint32_t arr = a.arrival[p];
-  a.tmp_id[a.start[c] + arr] = me;
-  a.hist[c] = 0u;  // every writer stores 0; pad cells are never keys and keep their size
-  // canonical edge list of the pre-step state (offsets from the same scan as the cells)
+  SimDesc sd;
+  if (!sort_lane(a, gw, p, sd)) return;
+  // the owner's edge offsets beside its cell's start
+  uint32_t off = 0u, end = 0u;
   if (a.edges) {
-    const uint32_t off = a.eoff[me];
-    const int e = (int)(a.eoff[me + 1] - off);
-    if (e) a.fcount[me] = 0u;  // the next step's force pass writes only non-zero counts
-    for (int k = 0; k < e; ++k)
-      a.edges[off + k] =
-          make_int2((int)(me - sd.p0), (int)(a.estage[(long)p * a.estride + k] - sd.p0));
+    off = a.eoff[me];
+    end = a.eoff[me + 1];
+  }
+  a.tmp_id[a.start[key] + arr] = me;
+  a.hist[key] = 0u;  // every writer stores 0; pad cells are never keys and keep their size
+  // canonical edge list of the pre-step state (offsets from the same scan as the cells)
+  if (end != off) {
+    a.fcount[me] = 0u;  // the next step's force pass writes only non-zero counts
+    const uint32_t* rec = a.estage + (long)p * a.estride;
+    const uint32_t e = end - off;
+    constexpr uint32_t kBatch = 4;
+    for (uint32_t k0 = 0; k0 < e; k0 += kBatch) {
+      uint32_t to[kBatch];
+#pragma unroll
+      for (uint32_t u = 0; u < kBatch; ++u) to[u] = rec[min(k0 + u, e - 1u)];
+#pragma unroll
+      for (uint32_t u = 0; u < kBatch; ++u)
+        if (k0 + u < e) a.edges[off + k0 + u] = make_int2((int)me - sd.p0, (int)to[u] - sd.p0);
+    }
   }
 }
 
 __global__ void __launch_bounds__(256) k_rank_scatter(SortArgs a) {
-  const int gw = xcd_block() * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int gw = xcd_block() * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (gw >= a.nwaves) return;
-  const SimDesc sd = a.sims[a.wave_sim[gw]];
   const int p = gw * kWave + (threadIdx.x & (kWave - 1));
-  if (p - sd.p0 >= sd.n) return;
-  const uint32_t c = a.key[p];
+  const uint32_t key = a.key[p];
   const uint32_t me = a.src_id[p];
   const float4 sp = a.src_pos[p];
   const float4 sv = a.src_vel[p];
-  const uint32_t s0 = a.start[c], s1 = a.start[c + 1];
+  const uint32_t arr = a.arrival[p];
+  SimDesc sd;
+  if (!sort_lane(a, gw, p, sd)) return;
+  const uint32_t s0 = a.start[key], n = a.start[key + 1] - s0;
   uint32_t rank = 0;
   if (sd.ident) {
-    rank = a.arrival[p];  // source already in index order
+    rank = arr;  // source already in index order
   } else {
-    uint32_t q = s0;
-    for (; q + 4 <= s1; q += 4) {  // four independent loads per trip
-      const uint32_t i0 = a.tmp_id[q], i1 = a.tmp_id[q + 1], i2 = a.tmp_id[q + 2],
-                     i3 = a.tmp_id[q + 3];
-      rank += (i0 < me) + (i1 < me) + (i2 < me) + (i3 < me);
-    }
-    for (; q < s1; ++q) rank += (a.tmp_id[q] < me) ? 1u : 0u;
+    // n is at least 1 (the particle itself); reads past the cell repeat its last member
+    const uint32_t* ids = a.tmp_id + s0;
+    auto trip = [&](uint32_t e, auto batch) {
+      constexpr uint32_t kBatch = decltype(batch)::value;
+      uint32_t v[kBatch];
+#pragma unroll
+      for (uint32_t u = 0; u < kBatch; ++u) v[u] = ids[min(e + u, n - 1u)];
+#pragma unroll
+      for (uint32_t u = 0; u < kBatch; ++u) rank += (e + u < n && v[u] < me) ? 1u : 0u;
+    };
+    uint32_t e = 0u;
+    for (; e + 8u < n; e += 16u) trip(e, std::integral_constant<uint32_t, 16>{});
+    if (e < n) trip(e, std::integral_constant<uint32_t, 8>{});
   }
   const uint32_t dst = s0 + rank;
   a.dst_pos[dst] = sp;
@@ -3205,10 +3235,11 @@ __global__ void __launch_bounds__(256) k_rank_scatter(SortArgs a) {
 
 
 __global__ void __launch_bounds__(256) k_bin(BinArgs a) {
-  const int gw = blockIdx.x * (blockDim.x >> 6) + (threadIdx.x >> 6);
+  const int gw = blockIdx.x * 4 + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   if (gw >= a.nwaves) return;
-  const SimDesc sd = a.sims[a.wave_sim[gw]];
   const int p = gw * kWave + (threadIdx.x & (kWave - 1));
+  const float4 pi = a.pos[p];
+  const SimDesc sd = a.sims[a.wave_sim[gw]];
   if (p - sd.p0 >= sd.n) return;
   if (sd.ident) {  // one cell in index order: no atomics, the count is known
     a.key[p] = (uint32_t)sd.c0;
@@ -3216,7 +3247,6 @@ __global__ void __launch_bounds__(256) k_bin(BinArgs a) {
     if (p == sd.p0) a.hist[sd.c0] = (uint32_t)sd.n;
     return;
   }
-  const float4 pi = a.pos[p];
   const uint32_t c = (uint32_t)(sd.c0 + bin_axis(pi.x, sd.ihx, sd.nx) +
                                 sd.nx * (bin_axis(pi.y, sd.ihy, sd.ny) +
                                          sd.ny * bin_axis(pi.z, sd.ihz, sd.nz)));
