@@ -1237,7 +1237,9 @@ struct Engine {
     a.cd = canvas[2];
     a.spawn = spawn;
     HIPR(launch_init(a, sims[s].n, st));
-    return flush();
+    CFR(flush());
+    HIPR(hipStreamSynchronize(st));  // done on return, whether or not descriptors were uploaded
+    return CF_OK;
   }
 
   int get_edges(int32_t* pairs, long long capacity, long long* count) {
