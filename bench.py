@@ -36,12 +36,16 @@ def log(msg):
     print(msg, file=sys.stderr, flush=True)
 
 
-def force_kernel_name(t, edges=True):
-    """The force kernel a tuning launches, as rocprofv3 names it."""
+def force_kernel_name(t, n, edges=True):
+    """The force kernel a tuning launches for a simulation of n particles, as rocprofv3
+    names it."""
     e = "true" if edges else "false"
     r, g = t["cell_divisor"], t["lanes_per_particle"]
     tl = "true" if t.get("sort_variant", 1) == 1 else "false"
-    return {0: f"k_force_grp<{e}, {r}, {g}, {tl}>", 1: f"k_force<{e}>",
+    og = 16 if r == 2 or (n + 63) // 64 * 64 < 28672 else 8  # lanes of the default's kernel
+    grp = f"k_force_ord<{e}, {r}, {og}, {tl}, false>" if g == 16 else \
+        f"k_force_grp<{e}, {r}, {g}, {tl}, false>"
+    return {0: grp, 1: f"k_force<{e}>",
             2: f"k_force_lds<{e}, {r}>", 3: f"k_force_list<{e}, {r}, {g}, {tl}, false>",
             4: f"k_force_list<{e}, {r}, {g}, {tl}, true>"}[t["force_variant"]]
 
@@ -494,7 +498,7 @@ def main():
     force_ms = kt["force"]
     alg_bytes = n * (STEP_BYTES + EDGE_BYTES) + EDGE_PAIR_BYTES * nedges
     achieved = alg_bytes / (force_ms * 1e-3) / 1e9
-    kname = force_kernel_name(tuned["tuning"])
+    kname = force_kernel_name(tuned["tuning"], n)
     roof = {"bound": "hbm", "kernel": kname, "achieved": achieved, "peak": HBM_PEAK_GBS,
             "unit": "GB/s", "frac": achieved / HBM_PEAK_GBS,
             "traffic": read_traffic(os.path.join(ROOT, "profiles", "k_force_c2_traffic.txt"),
