@@ -333,7 +333,14 @@ k_adj_pair_g(AdjArgs a) {
   double* const col = a.partial + (long)threadIdx.x * a.stride + blockIdx.x;
   const double col0 = (int)threadIdx.x < rows ? *col : 0.0;
   double4 lxn = make_double4(0.0, 0.0, 0.0, 0.0);
+  // the lane's first two list entries, beside the list's length (entries past the length are
+  // never used)
+  static_assert(2 * G <= kAdjHits, "two entries per lane");
+  const uint32_t* lst = a.hits + (long)k * kAdjHits;
+  uint32_t qa = 0u, qb = 0u;
   if (active) {
+    qa = lst[g];
+    qb = lst[g + G];
     idi = a.id[p];
     phi_i = a.phi[idi];
     nh = a.nhits[k];
@@ -380,13 +387,15 @@ k_adj_pair_g(AdjArgs a) {
     pair((int)__float_as_uint(a.pos[q].w), a.x64[j], a.phi[j]);
   };
   if (listed) {
-    // the lane's entries two at a time, each stage's loads issued together (list entry, then
-    // type and index, then factor and shadow position); pairs summed in entry order
-    const uint32_t* lst = a.hits + (long)k * kAdjHits;
+    // the lane's entries two at a time, each stage's loads issued together (list entry a trip
+    // ahead, then type and index, then factor and shadow position: 14.2 -> 13.9 us with 20k
+    // particles for the entries ahead); pairs summed in entry order
 #pragma nounroll
     for (uint32_t e = g; e < nh; e += 2 * G) {
       const bool two = e + G < nh;
-      const uint32_t q0 = lst[e], q1 = two ? lst[e + G] : q0;
+      const uint32_t q0 = qa, q1 = two ? qb : q0;
+      qa = lst[min(e + 2 * G, (uint32_t)kAdjHits - 1u)];  // the next trip's
+      qb = lst[min(e + 3 * G, (uint32_t)kAdjHits - 1u)];
       const int t0 = (int)__float_as_uint(a.pos[q0].w), t1 = (int)__float_as_uint(a.pos[q1].w);
       const uint32_t j0 = a.id[q0], j1 = a.id[q1];
       const double4 f0 = a.phi[j0], f1 = a.phi[j1];

@@ -164,16 +164,26 @@ __device__ __forceinline__ void shadow_block(const AdjArgs& a, int thread) {
       prev = __float_as_int(a.vel[c.p].w);
       vi = a.v64[idi];
     }
-    const uint32_t nh = a.hits ? a.nhits[k] : 0u;
+    // the lane's first two list entries beside the list's length, and below the next trip's
+    // beside this one's pairs (entries past the length are never used)
+    static_assert(2 * G <= kAdjHits, "two entries per lane");
+    const uint32_t* lst = a.hits + (long)k * kAdjHits;
+    uint32_t nh = 0u, qa = 0u, qb = 0u;
+    if (a.hits) {
+      nh = a.nhits[k];
+      qa = lst[g];
+      qb = lst[g + G];
+    }
     if (a.hits && nh <= (uint32_t)kAdjHits) {
       if (g == 0) cnt = (int)nh;
       // the lane's entries two at a time, each stage's loads issued together (list entry,
       // then type and index, then shadow position); pairs summed in entry order
-      const uint32_t* lst = a.hits + (long)k * kAdjHits;
 #pragma nounroll
       for (uint32_t e = g; e < nh; e += 2 * G) {
         const bool two = e + G < nh;
-        const uint32_t q0 = lst[e], q1 = two ? lst[e + G] : q0;
+        const uint32_t q0 = qa, q1 = two ? qb : q0;
+        qa = lst[min(e + 2 * G, (uint32_t)kAdjHits - 1u)];
+        qb = lst[min(e + 3 * G, (uint32_t)kAdjHits - 1u)];
         const int t0 = (int)__float_as_uint(a.pos[q0].w), t1 = (int)__float_as_uint(a.pos[q1].w);
         const uint32_t j0 = a.id[q0], j1 = a.id[q1];
         const double4 x0 = a.x64[j0], x1 = a.x64[j1];
