@@ -654,17 +654,14 @@ struct Engine {
 
   // Loads write index-order records of one simulation into the temporaries; the other
   // simulations' current state is copied there first, then everything is sorted once.
-  // `replace`: the caller writes all of its simulation's slots.
+  // `replace`: the caller writes all of its simulation's slots, so a single simulation's
+  // temporaries hold no state until it has: load_pending is the caller's to set, once the
+  // kernel that fills them is queued.
   int begin_load(bool replace) {
-    if (load_pending) return CF_OK;
-    if (replace && sims.size() == 1) {
-      load_pending = true;
-      return CF_OK;
-    }
+    if (load_pending || (replace && sims.size() == 1)) return CF_OK;
     HIPR(hipMemcpyAsync(b.tpos, b.pos[cur], P * sizeof(float4), hipMemcpyDeviceToDevice, st));
     HIPR(hipMemcpyAsync(b.tvel, b.vel[cur], P * sizeof(float4), hipMemcpyDeviceToDevice, st));
     HIPR(hipMemcpyAsync(b.tid, b.id[cur], P * sizeof(uint32_t), hipMemcpyDeviceToDevice, st));
-    load_pending = true;
     return CF_OK;
   }
 
@@ -1147,6 +1144,7 @@ struct Engine {
     IoArgs a = io_args(s);
     a.aos = d;
     HIPR(launch_io(0, a, h.n, st));
+    load_pending = true;
     HIPR(hipStreamSynchronize(st));
     return CF_OK;
   }
@@ -1214,15 +1212,17 @@ struct Engine {
     a.shift[2] = dz;
     for (int k = 0; k < 3; ++k) a.box[k] = box[k];
     HIPR(launch_io(5, a, sims[s].n, st));
+    load_pending = true;
     return flush();
   }
 
   int init_particles(int s, uint64_t seed, const float canvas[3], float spawn) {
-    CFR(begin_load(true));
-    // descriptors must carry this simulation's T before the init kernel runs
-    bool changed = false;
+    // The descriptors must carry this simulation's T before the init kernel runs.  The state
+    // is binned for them first: a call that fails there (an effective radius that is not
+    // finite) leaves it as it was.
     EdgeReq none;
-    CFR(build_descs(none, &changed));
+    CFR(prepare(none));
+    CFR(begin_load(true));
     InitArgs a{};
     a.tpos = b.tpos;
     a.tvel = b.tvel;
@@ -1237,6 +1237,7 @@ struct Engine {
     a.cd = canvas[2];
     a.spawn = spawn;
     HIPR(launch_init(a, sims[s].n, st));
+    load_pending = true;
     CFR(flush());
     HIPR(hipStreamSynchronize(st));  // done on return, whether or not descriptors were uploaded
     return CF_OK;
