@@ -192,7 +192,8 @@ struct Engine {
   DevBufs b{};
   int cur = 0;
   bool load_pending = false;
-  std::vector<int> grid_sig;       // dims/reach of the binning A is sorted for
+  std::vector<int> cell_sig;       // dims/reach the cell arrays are laid out for
+  std::vector<int> grid_sig;       // those and the cell sizes of the binning A is sorted for
   std::vector<SimDesc> hdesc;      // uploaded descriptors (kept alive for async copies)
   std::vector<PairConst> hpairs;
   std::vector<SimDesc> ndesc;      // being built; uploaded when they differ
@@ -388,7 +389,7 @@ struct Engine {
   int build_descs(const EdgeReq& er, bool* grid_changed, bool any_edges = false) {
     ndesc.assign(sims.size(), SimDesc{});
     npairs.assign(sims.size() * kMaxTypes * kMaxTypes, PairConst{});
-    std::vector<int> sig;
+    std::vector<int> cells, sig;
     long c = 0;
     int nt = 0;
     for (size_t s = 0; s < sims.size(); ++s) {
@@ -481,11 +482,16 @@ struct Engine {
       d.t0 = nt;
       nt += d.nz * d.nyt;
       c += (long)d.ncells + 1;
-      sig.push_back(d.nx);
-      sig.push_back(d.ny);
-      sig.push_back(d.nz);
-      sig.push_back(d.reach);
+      cells.insert(cells.end(), {d.nx, d.ny, d.nz, d.reach});
+      // a particle's cell follows from the numbers of cells and these (bin_axis), so a box
+      // of another size is another binning also when the numbers stay
+      for (const float f : ih) {
+        int bits;
+        std::memcpy(&bits, &f, sizeof bits);
+        sig.push_back(bits);
+      }
     }
+    sig.insert(sig.end(), cells.begin(), cells.end());
     *grid_changed = (sig != grid_sig);
     if (!*grid_changed && !counters_dirty && hdesc.size() == ndesc.size() &&
         hpairs.size() == npairs.size()) {
@@ -508,8 +514,9 @@ struct Engine {
         return CF_OK;
     }
     C = c;
-    if (*grid_changed) {
-      grid_sig = sig;
+    if (*grid_changed) grid_sig = sig;
+    if (cells != cell_sig) {
+      cell_sig = cells;
       CFR(ensure_cells());
     }
     HIPR(hipStreamSynchronize(st));  // descriptors may still be read by queued work
