@@ -32,10 +32,15 @@ namespace cf {
 // fail() and the thread's error text live in cf_host.cpp (host-only, shared with the
 // preset and tuning-cache code).
 
+// A failed call's error is reported here, once: left with the runtime, it would be the result
+// of the next kernel launch, which asks for the last error.
 #define HIPR(call)                                                                         \
   do {                                                                                     \
     hipError_t e_ = (call);                                                                \
-    if (e_ != hipSuccess) return fail(CF_ERR_DEVICE, "%s: %s", #call, hipGetErrorString(e_)); \
+    if (e_ != hipSuccess) {                                                                \
+      (void)hipGetLastError();                                                             \
+      return fail(CF_ERR_DEVICE, "%s: %s", #call, hipGetErrorString(e_));                  \
+    }                                                                                      \
   } while (0)
 
 #define CFR(call)            \
@@ -192,8 +197,9 @@ struct Engine {
   DevBufs b{};
   int cur = 0;
   bool load_pending = false;
-  std::vector<int> cell_sig;       // dims/reach the cell arrays are laid out for
-  std::vector<int> grid_sig;       // those and the cell sizes of the binning A is sorted for
+  // dims/reach the cell arrays are laid out for, and with the cell sizes the binning that A
+  // is sorted for (empty: none, after a call that failed in between) and the descriptors'
+  std::vector<int> cell_sig, grid_sig, desc_sig;
   std::vector<SimDesc> hdesc;      // uploaded descriptors (kept alive for async copies)
   std::vector<PairConst> hpairs;
   std::vector<SimDesc> ndesc;      // being built; uploaded when they differ
@@ -514,10 +520,12 @@ struct Engine {
         return CF_OK;
     }
     C = c;
-    if (*grid_changed) grid_sig = sig;
+    if (*grid_changed) grid_sig.clear();  // until the caller's sort is queued
+    desc_sig = sig;
     if (cells != cell_sig) {
-      cell_sig = cells;
+      cell_sig.clear();
       CFR(ensure_cells());
+      cell_sig = cells;
     }
     HIPR(hipStreamSynchronize(st));  // descriptors may still be read by queued work
     hdesc.swap(ndesc);
@@ -526,6 +534,7 @@ struct Engine {
     if (nt > ntiles_cap) {
       drop_graphs();
       ++buf_gen;
+      ntiles_cap = 0;  // here and below: a size holds again once its buffers do
       for (int i = 0; i < 2; ++i) {
         dfree(tcnt[i]);
         CFR(dalloc(&tcnt[i], (size_t)nt * kCtrStride));
@@ -570,6 +579,7 @@ struct Engine {
     drop_graphs();
     ++buf_gen;
     if (C > Ccap) {
+      Ccap = 0;
       dfree(b.hist);
       dfree(b.start[0]);
       dfree(b.start[1]);
@@ -591,6 +601,7 @@ struct Engine {
     const int tiles[3] = {tc, tc + te, te};
     for (int i = 0; i < 3; ++i) {
       if (tiles[i] > plan_tiles[i]) {
+        plan_tiles[i] = 0;
         dfree(flags[i]);
         CFR(dalloc(&flags[i], tiles[i]));
       }
@@ -678,6 +689,7 @@ struct Engine {
     EdgeReq none;
     CFR(build_descs(none, &changed, true));
     CFR(sort_into(b.tpos, b.tvel, b.tid, cur));
+    grid_sig = desc_sig;
     load_pending = false;
     edges_count = -1;  // a graph or mesh belongs to the state it was built on
     step_edges_count = -1;
@@ -692,6 +704,7 @@ struct Engine {
     CFR(build_descs(er, &changed, any_edges));
     if (changed) {
       CFR(sort_into(b.pos[cur], b.vel[cur], b.id[cur], 1 - cur));
+      grid_sig = desc_sig;
       cur = 1 - cur;
     }
     return CF_OK;
@@ -706,6 +719,7 @@ struct Engine {
     }
     if (cap > edge_cap_alloc) {
       HIPR(hipStreamSynchronize(st));
+      edge_cap_alloc = 0;
       dfree(b.ecand_d2);
       dfree(b.ecand_id);
       CFR(dalloc(&b.ecand_d2, (size_t)cap * P));
@@ -714,6 +728,7 @@ struct Engine {
     }
     if (maxc > edge_maxc_alloc) {
       HIPR(hipStreamSynchronize(st));
+      edge_maxc_alloc = 0;
       dfree(b.estage);
       CFR(dalloc(&b.estage, (size_t)maxc * P));
       // the last graph stays readable when a mesh with a longer list grows the buffers
@@ -1813,7 +1828,7 @@ struct Engine {
     if (need > kScratchBytes)
       return fail(CF_ERR_ARG, "%d particles x %d bins need %zu bytes of scratch; the "
                   "allocation-free histogram holds at most %zu", n, bins, need, kScratchBytes);
-    if (!sims[0].have_prm || load_pending)
+    if (!sims[0].have_prm || load_pending || grid_sig.empty())
       return fail(CF_ERR_STATE, "the state is not binned: step it (cf_simulate, 0 steps "
                                 "bins it) after loading, before the allocation-free histogram");
     double* partial = static_cast<double*>(scratch_ptr(device));
@@ -2100,7 +2115,9 @@ struct Engine {
     tun = orig;
     bool changed = false;
     CFR(build_descs(er, &changed));
-    return load_state(snap);
+    CFR(load_state(snap));
+    grid_sig = desc_sig;
+    return CF_OK;
   }
 
   // Average microseconds per step over `nsteps` steps as cf_simulate runs them after its

@@ -1,0 +1,273 @@
+// The engine's host side against a HIP runtime that lives in this program: device memory is
+// host memory, a kernel launch is a line of the log, and any allocation can be made to fail.
+// The definitions here come before the real runtime's in symbol order, so libcellflow.so binds
+// to them; nothing needs a GPU.  Each case checks which calls the engine makes, and that none
+// of them touches memory that was never allocated or was freed.
+//
+//   engine_host_check CASE   exits 0 when the case holds
+#include <hip/hip_runtime_api.h>
+
+#include <cstdarg>
+#include <cstdio>
+#include <cstdlib>
+#include <cstring>
+#include <functional>
+#include <map>
+#include <string>
+#include <vector>
+
+#include "cellflow.h"
+
+// ---- the runtime -----------------------------------------------------------------------
+
+namespace {
+
+struct Runtime {
+  std::map<const void*, std::string> kernels;   // host function -> device name
+  std::map<const char*, size_t> mem;            // live allocations
+  std::vector<std::string> log;
+  hipError_t last = hipSuccess;
+  // the countdowns reach a failure at 0; negative: never
+  int fail_malloc = -1, fail_copy = -1;
+  size_t host_limit = ~size_t(0);               // larger pinned allocations fail
+  dim3 grid, block;
+  size_t shm = 0;
+  hipStream_t stream = nullptr;
+};
+
+Runtime& rt() {
+  static Runtime* r = new Runtime;  // outlives the library's own destructors
+  return *r;
+}
+
+hipError_t result(hipError_t e) {
+  if (e != hipSuccess) rt().last = e;
+  return e;
+}
+
+bool due(int& countdown) { return countdown >= 0 && countdown-- == 0; }
+
+[[noreturn]] void die(const char* fmt, ...) {
+  va_list ap;
+  va_start(ap, fmt);
+  std::vfprintf(stderr, fmt, ap);
+  va_end(ap);
+  std::fputc('\n', stderr);
+  std::_Exit(1);
+}
+
+// Whether [p, p + n) lies in one live allocation.
+bool live(const void* p, size_t n) {
+  const char* c = (const char*)p;
+  auto it = rt().mem.upper_bound(c);
+  if (it == rt().mem.begin()) return false;
+  --it;
+  return c + n <= it->first + it->second;
+}
+
+hipError_t allocate(void** p, size_t n) {
+  char* c = (char*)std::calloc(1, n);
+  rt().mem[c] = n;
+  *p = c;
+  return hipSuccess;
+}
+
+hipError_t release(void* p) {
+  if (!rt().mem.erase((const char*)p)) die("free of %p, which is not allocated", p);
+  std::free(p);
+  return hipSuccess;
+}
+
+}  // namespace
+
+extern "C" {
+
+void** __hipRegisterFatBinary(const void*) {
+  static void* handle = nullptr;
+  return &handle;
+}
+void __hipUnregisterFatBinary(void**) {}
+void __hipRegisterFunction(void**, const void* host, char*, const char* name, unsigned, void*,
+                           void*, void*, void*, int*) {
+  rt().kernels[host] = name;
+}
+void __hipRegisterVar(void**, void*, char*, char*, int, size_t, int, int) {}
+hipError_t __hipPushCallConfiguration(dim3 grid, dim3 block, size_t shm, hipStream_t st) {
+  rt().grid = grid;
+  rt().block = block;
+  rt().shm = shm;
+  rt().stream = st;
+  return hipSuccess;
+}
+hipError_t __hipPopCallConfiguration(dim3* grid, dim3* block, size_t* shm, hipStream_t* st) {
+  *grid = rt().grid;
+  *block = rt().block;
+  *shm = rt().shm;
+  *st = rt().stream;
+  return hipSuccess;
+}
+hipError_t hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, hipStream_t) {
+  auto it = rt().kernels.find(f);
+  if (it == rt().kernels.end()) die("launch of an unknown kernel");
+  rt().log.push_back(it->second);
+  return hipSuccess;
+}
+
+hipError_t hipGetDeviceCount(int* n) {
+  *n = 1;
+  return hipSuccess;
+}
+hipError_t hipGetDevice(int* d) {
+  *d = 0;
+  return hipSuccess;
+}
+hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipGetLastError(void) {
+  const hipError_t e = rt().last;
+  rt().last = hipSuccess;
+  return e;
+}
+hipError_t hipGetSymbolAddress(void** p, const void*) { return allocate(p, 64); }
+hipError_t hipMemGetInfo(size_t* avail, size_t* total) {
+  *avail = *total = size_t(256) << 30;
+  return hipSuccess;
+}
+
+hipError_t hipMalloc(void** p, size_t n) {
+  rt().log.push_back("malloc");
+  if (due(rt().fail_malloc)) return result(hipErrorOutOfMemory);
+  return allocate(p, n);
+}
+hipError_t hipFree(void* p) { return release(p); }
+hipError_t hipHostMalloc(void** p, size_t n, unsigned) {
+  if (n > rt().host_limit) return result(hipErrorOutOfMemory);
+  return allocate(p, n);
+}
+hipError_t hipHostFree(void* p) { return release(p); }
+
+hipError_t hipMemsetAsync(void* p, int v, size_t n, hipStream_t) {
+  if (!live(p, n)) die("memset of %zu bytes at %p", n, p);
+  std::memset(p, v, n);
+  rt().log.push_back("memset");
+  return hipSuccess;
+}
+hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind kind, hipStream_t) {
+  if (kind != hipMemcpyDeviceToHost && !live(d, n)) die("copy of %zu bytes to %p", n, d);
+  if (kind != hipMemcpyHostToDevice && !live(s, n)) die("copy of %zu bytes from %p", n, s);
+  if (due(rt().fail_copy)) return result(hipErrorUnknown);
+  std::memcpy(d, s, n);
+  rt().log.push_back("copy");
+  return hipSuccess;
+}
+
+hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
+  static int handle;
+  *s = (hipStream_t)&handle;
+  return hipSuccess;
+}
+hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamSynchronize(hipStream_t) {
+  rt().log.push_back("sync");
+  return hipSuccess;
+}
+hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
+  static int handle;
+  *e = (hipEvent_t)&handle;
+  return hipSuccess;
+}
+hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+
+}  // extern "C"
+
+// ---- the cases -------------------------------------------------------------------------
+
+namespace {
+
+#define HOLDS(x)                                                        \
+  do {                                                                  \
+    if (!(x)) die("line %d: %s does not hold", __LINE__, #x);           \
+  } while (0)
+#define OK(x)                                                           \
+  do {                                                                  \
+    const int rc_ = (x);                                                \
+    if (rc_ != CF_OK) die("line %d: %s: %s", __LINE__, #x, cf_last_error_string()); \
+  } while (0)
+
+cf_params params(float radius, float side) {
+  cf_params p{};
+  p.radius = radius;
+  p.delta_t = 0.01f;
+  p.friction = 0.9f;
+  p.repulsion = p.attraction = p.k = 1.0f;
+  p.canvas_width = p.canvas_height = p.canvas_depth = side;
+  p.num_particle_types = 2;
+  p.force_multiplier = 1.0f;
+  p.max_expected_neighbors = 100;
+  return p;
+}
+
+int logged(const char* what) {
+  int k = 0;
+  for (const std::string& s : rt().log) k += s.find(what) != std::string::npos;
+  return k;
+}
+
+struct Sim {
+  cf_sim* h = nullptr;
+  int n;
+  explicit Sim(int count) : n(count) { OK(cf_create(count, 2, &h)); }
+  ~Sim() { OK(cf_destroy(h)); }
+};
+
+// Every allocation of a call that needs larger buffers fails once, in turn: the call reports
+// it, and the next calls, at the old sizes and at the new, allocate what the failed one gave
+// up and sort the state again before they walk its cells.
+void grow_cells() {
+  const cf_params coarse = params(0.2f, 2.0f), fine = params(0.05f, 2.0f);
+  const cf_edge_opts few{0.02f, 4}, many{0.02f, 16};
+  for (const bool edges : {false, true}) {
+    for (const bool back : {false, true}) {
+      int failures = 0;
+      for (int k = 0;; ++k) {
+        Sim s(20000);
+        const cf_params& next = edges ? coarse : fine;
+        OK(cf_simulate(s.h, &coarse, 2, edges ? &few : nullptr));
+        rt().fail_malloc = k;
+        const int rc = cf_simulate(s.h, &next, 2, edges ? &many : nullptr);
+        const bool failed = rt().fail_malloc < 0;
+        rt().fail_malloc = -1;
+        HOLDS(failed == (rc == CF_ERR_DEVICE));
+        if (!failed) break;
+        ++failures;
+        double hist[8];
+        rt().log.clear();
+        if (!edges) HOLDS(cf_pair_histogram_noalloc(s.h, 8, 0.05f, hist) == CF_ERR_STATE);
+        HOLDS(logged("k_") == 0);
+        OK(cf_simulate(s.h, back ? &coarse : &next, 2,
+                       !edges ? nullptr : back ? &few : &many));
+        HOLDS(logged("malloc") > 0);
+        if (!edges) HOLDS(logged("k_bin") == 1);
+        rt().log.clear();
+        OK(cf_simulate(s.h, back ? &coarse : &next, 2,
+                       !edges ? nullptr : back ? &few : &many));
+        HOLDS(logged("malloc") == 0 && logged("k_bin") == 0);
+      }
+      HOLDS(failures >= (edges ? 5 : 6));
+    }
+  }
+}
+
+}  // namespace
+
+int main(int argc, char** argv) {
+  const std::map<std::string, std::function<void()>> cases = {
+      {"grow_cells", grow_cells},
+  };
+  const auto it = argc == 2 ? cases.find(argv[1]) : cases.end();
+  if (it == cases.end()) die("usage: engine_host_check CASE");
+  it->second();
+  std::printf("%s ok\n", argv[1]);
+  return 0;
+}
