@@ -1235,7 +1235,9 @@ struct Engine {
     for (int k = 0; k < 3; ++k) a.box[k] = box[k];
     HIPR(launch_io(5, a, sims[s].n, st));
     load_pending = true;
-    return flush();
+    CFR(flush());
+    HIPR(hipStreamSynchronize(st));  // done on return, whether or not descriptors were uploaded
+    return CF_OK;
   }
 
   int init_particles(int s, uint64_t seed, const float canvas[3], float spawn) {

@@ -259,11 +259,28 @@ void grow_cells() {
   }
 }
 
+// The calls that change a whole state have nothing outstanding when they return.
+void changes_wait() {
+  const cf_params p = params(0.1f, 2.0f);
+  const float canvas[3] = {2.0f, 2.0f, 2.0f};
+  Sim s(5000);
+  OK(cf_simulate(s.h, &p, 3, nullptr));
+  for (int k = 0; k < 2; ++k) {  // with and without new descriptors before
+    rt().log.clear();
+    OK(cf_move_universe(s.h, 0.1f, 0.2f, 0.0f, canvas));
+    HOLDS(logged("k_move") == 1 && rt().log.back() == "sync");
+    rt().log.clear();
+    OK(cf_init_particles(s.h, 3, canvas, 1.0f));
+    HOLDS(logged("k_init") == 1 && rt().log.back() == "sync");
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> cases = {
       {"grow_cells", grow_cells},
+      {"changes_wait", changes_wait},
   };
   const auto it = argc == 2 ? cases.find(argv[1]) : cases.end();
   if (it == cases.end()) die("usage: engine_host_check CASE");

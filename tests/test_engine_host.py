@@ -33,3 +33,7 @@ def check(tmp_path_factory):
 
 def test_failed_allocations_leave_the_sizes_true(check):
     check("grow_cells")
+
+
+def test_state_changes_wait_for_their_kernels(check):
+    check("changes_wait")
