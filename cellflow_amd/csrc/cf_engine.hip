@@ -1085,16 +1085,21 @@ struct Engine {
   }
 
   // The pinned staging buffer of loads and readbacks, at least `bytes` long (each use ends
-  // with a stream synchronisation, so no two overlap).
-  int pin(size_t bytes) {
-    if (bytes <= hpin_cap) return CF_OK;
-    HIPR(hipStreamSynchronize(st));
+  // with a stream synchronisation, so no two overlap).  False: no more memory can be pinned,
+  // and the copy goes without the buffer.
+  bool pin(size_t bytes) {
+    if (bytes <= hpin_cap) return true;
+    (void)hipStreamSynchronize(st);
     if (hpin) (void)hipHostFree(hpin);
     hpin = nullptr;
     hpin_cap = 0;
-    HIPR(hipHostMalloc((void**)&hpin, bytes, hipHostMallocDefault));
+    if (hipHostMalloc((void**)&hpin, bytes, hipHostMallocDefault) != hipSuccess) {
+      (void)hipGetLastError();
+      hpin = nullptr;
+      return false;
+    }
     hpin_cap = bytes;
-    return CF_OK;
+    return true;
   }
 
   // Device-to-host copy of `bytes` into the caller's memory through the pinned staging
@@ -1102,7 +1107,11 @@ struct Engine {
   // copied on by the host threads as it arrives, beside the DMA of the next ones.
   int to_host(void* dst, const void* src, size_t bytes) {
     if (bytes == 0) return CF_OK;
-    CFR(pin(bytes));
+    if (!pin(bytes)) {
+      HIPR(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, st));
+      HIPR(hipStreamSynchronize(st));
+      return CF_OK;
+    }
     const size_t slice = std::max(kSlice, (bytes + kSlices - 1) / kSlices);
     size_t k = 0;
     for (size_t at = 0; at < bytes; at += slice, ++k) {
@@ -1134,9 +1143,8 @@ struct Engine {
     // A simulation's first load goes straight from the caller's memory unless a readback has
     // pinned a buffer already: pinning one takes longer (0.1-0.25 ms for 1 MB, 5 ms for 44)
     // than one load gains, and a program may load once and never read.
-    const bool staged = n * rec <= hpin_cap || sims[s].loaded;
+    const bool staged = (n * rec <= hpin_cap || sims[s].loaded) && pin(n * rec);
     sims[s].loaded = true;
-    if (staged) CFR(pin(n * rec));
     const size_t slice = staged ? std::max(kSlice, (n * rec + kSlices - 1) / kSlices) / rec : n;
     std::atomic<long long> bad{(long long)n};
     for (size_t at = 0; at < n && bad.load() == (long long)n; at += slice) {

@@ -275,12 +275,36 @@ void changes_wait() {
   }
 }
 
+// Where the system pins little memory, loads and readbacks do without the staging buffer.
+void pins_little() {
+  Sim s(60000);  // 2.6 MB of records: two slices of the staged path
+  std::vector<cf_particle> in(s.n), out(s.n);
+  std::vector<int32_t> counts(s.n);
+  for (int round = 0; round < 4; ++round) {
+    rt().host_limit = round % 2 ? ~size_t(0) : size_t(1) << 16;
+    for (int i = 0; i < s.n; ++i) {
+      in[i].pos[0] = (float)(i + round);
+      in[i].ptype = (uint32_t)(i & 1);
+    }
+    OK(cf_set_particles(s.h, in.data(), s.n));
+    // nothing ran between, so what is read back is what the load left in the device buffer
+    OK(cf_get_particles(s.h, out.data(), s.n));
+    HOLDS(std::memcmp(in.data(), out.data(), in.size() * sizeof(cf_particle)) == 0);
+    OK(cf_get_neighbor_counts(s.h, counts.data(), s.n));
+    HOLDS(std::memcmp(in.data(), counts.data(), counts.size() * sizeof(int32_t)) == 0);
+    in[s.n - 1].ptype = 2;
+    HOLDS(cf_set_particles(s.h, in.data(), s.n) == CF_ERR_ARG);
+    HOLDS(hipGetLastError() == hipSuccess);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
   const std::map<std::string, std::function<void()>> cases = {
       {"grow_cells", grow_cells},
       {"changes_wait", changes_wait},
+      {"pins_little", pins_little},
   };
   const auto it = argc == 2 ? cases.find(argv[1]) : cases.end();
   if (it == cases.end()) die("usage: engine_host_check CASE");

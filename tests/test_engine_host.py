@@ -37,3 +37,7 @@ def test_failed_allocations_leave_the_sizes_true(check):
 
 def test_state_changes_wait_for_their_kernels(check):
     check("changes_wait")
+
+
+def test_copies_without_pinned_memory(check):
+    check("pins_little")
