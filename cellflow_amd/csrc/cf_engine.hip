@@ -1408,7 +1408,10 @@ struct Engine {
     if (nc > 0 && (hcol.size() != nc || std::memcmp(hcol.data(), cf, nc * sizeof(float)) != 0)) {
       HIPR(hipStreamSynchronize(st));  // `hcol` may still be read by a queued copy
       hcol.assign(cf, cf + nc);
-      HIPR(hipMemcpyAsync(vcol, hcol.data(), nc * sizeof(float), hipMemcpyHostToDevice, st));
+      const hipError_t e =
+          hipMemcpyAsync(vcol, hcol.data(), nc * sizeof(float), hipMemcpyHostToDevice, st);
+      if (e != hipSuccess) hcol.clear();  // they are not on the device
+      HIPR(e);
     }
     HIPR(launch_slot_of(b.id[cur], slot_of, b.sims, 0, sims[0].n, st));
     return CF_OK;

@@ -30,6 +30,7 @@ struct Runtime {
   // the countdowns reach a failure at 0; negative: never
   int fail_malloc = -1, fail_copy = -1;
   size_t host_limit = ~size_t(0);               // larger pinned allocations fail
+  uint32_t edges = 0;                           // the graph's size in the status words read back
   dim3 grid, block;
   size_t shm = 0;
   hipStream_t stream = nullptr;
@@ -156,6 +157,7 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind kind, 
   if (kind != hipMemcpyHostToDevice && !live(s, n)) die("copy of %zu bytes from %p", n, s);
   if (due(rt().fail_copy)) return result(hipErrorUnknown);
   std::memcpy(d, s, n);
+  if (kind == hipMemcpyDeviceToHost && n == 4 * sizeof(uint32_t)) ((uint32_t*)d)[1] = rt().edges;
   rt().log.push_back("copy");
   return hipSuccess;
 }
@@ -298,6 +300,33 @@ void pins_little() {
   }
 }
 
+// Colours are uploaded when they change, and again after an upload that failed.
+void colours() {
+  const cf_params p = params(0.1f, 2.0f);
+  cf_color c[2] = {{1, 0, 0}, {0, 1, 0}};
+  Sim s(2000);
+  OK(cf_simulate(s.h, &p, 1, nullptr));
+  rt().edges = 3;
+  OK(cf_build_edges(s.h, 0.05f, 4));
+  std::vector<float> out(12 * 3);
+  long long count = 0;
+  auto draw = [&] {
+    rt().log.clear();
+    return cf_get_line_vertices(s.h, c, 2, out.data(), (long long)out.size(), &count);
+  };
+  for (int k = 0; k < 2; ++k) {
+    OK(draw());
+    HOLDS(count == 6 && logged("copy") == 2);  // the colours up, the vertices down
+    OK(draw());
+    HOLDS(logged("copy") == 1);
+    c[0].g = 0.5f + k;
+    rt().fail_copy = 0;
+    HOLDS(draw() == CF_ERR_DEVICE);
+  }
+  OK(draw());
+  HOLDS(logged("copy") == 2);
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -305,6 +334,7 @@ int main(int argc, char** argv) {
       {"grow_cells", grow_cells},
       {"changes_wait", changes_wait},
       {"pins_little", pins_little},
+      {"colours", colours},
   };
   const auto it = argc == 2 ? cases.find(argv[1]) : cases.end();
   if (it == cases.end()) die("usage: engine_host_check CASE");

@@ -41,3 +41,7 @@ def test_state_changes_wait_for_their_kernels(check):
 
 def test_copies_without_pinned_memory(check):
     check("pins_little")
+
+
+def test_colours_after_a_failed_upload(check):
+    check("colours")
