@@ -271,8 +271,9 @@ struct Engine {
 
   Engine() { host_pool_hold(); }
   ~Engine() {
+    HostPool* ending = host_pool_leave();  // its threads end beside the frees
     release();
-    host_pool_drop();
+    host_pool_end(ending);
   }
   Engine(const Engine&) = delete;
   Engine& operator=(const Engine&) = delete;

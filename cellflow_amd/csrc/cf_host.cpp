@@ -36,9 +36,7 @@ int fail(int code, const char* fmt, ...) {
   return code;
 }
 
-namespace {
-
-struct Pool {
+struct HostPool {
   std::mutex mu;
   std::condition_variable wake, done;
   std::vector<std::thread> threads;
@@ -73,10 +71,13 @@ struct Pool {
   }
 };
 
-std::mutex g_pool_mu;  // guards the three below
+namespace {
+
+std::mutex g_pool_mu;  // guards the four below
 std::mutex g_run_mu;   // one job at a time
-Pool* g_pool = nullptr;
+HostPool* g_pool = nullptr;
 int g_pool_users = 0;
+size_t g_pool_seen = 0;  // ranges of the larger jobs before there was a pool
 std::atomic<pid_t> g_pool_pid{0};  // the process the threads live in
 
 }  // namespace
@@ -86,49 +87,56 @@ void host_pool_hold() {
   ++g_pool_users;
 }
 
-void host_pool_drop() {
+HostPool* host_pool_leave() {
   const pid_t owner = g_pool_pid.load();
-  if (owner != 0 && owner != getpid()) return;  // a forked child has none of the threads
-  Pool* gone = nullptr;
+  if (owner != 0 && owner != getpid()) return nullptr;  // a forked child has none of the threads
+  HostPool* gone = nullptr;
   {
     std::lock_guard<std::mutex> l(g_pool_mu);
     if (--g_pool_users == 0) {
       gone = g_pool;
       g_pool = nullptr;
+      g_pool_seen = 0;
       g_pool_pid = 0;
     }
   }
-  if (!gone) return;
+  if (!gone) return nullptr;
   {
     std::lock_guard<std::mutex> l(gone->mu);
     gone->stop = true;
   }
   gone->wake.notify_all();
+  return gone;
+}
+
+void host_pool_end(HostPool* gone) {
+  if (!gone) return;
   for (std::thread& t : gone->threads) t.join();
   delete gone;
 }
+
+void host_pool_drop() { host_pool_end(host_pool_leave()); }
 
 void host_parallel(size_t n, size_t grain, const std::function<void(size_t, size_t)>& fn) {
   grain = std::max<size_t>(grain, 1);
   const pid_t owner = g_pool_pid.load();
   std::unique_lock<std::mutex> run(g_run_mu, std::defer_lock);
-  if (n <= 3 * grain || (owner != 0 && owner != getpid()) || !run.try_lock()) {
+  if (n <= kHostAlone * grain || (owner != 0 && owner != getpid()) || !run.try_lock()) {
     if (n) fn(0, n);
     return;
   }
-  Pool* p = nullptr;
+  HostPool* p = nullptr;
   {
     std::unique_lock<std::mutex> l(g_pool_mu, std::try_to_lock);
     if (l && g_pool_users > 0) {
-      if (!g_pool) {
-        g_pool = new (std::nothrow) Pool;
-        if (g_pool) {
-          g_pool_pid = getpid();
-          try {
-            for (int k = 0; k < kHostHelpers; ++k)
-              g_pool->threads.emplace_back([q = g_pool] { q->work(); });
-          } catch (...) {  // as many as the system gives
-          }
+      if (!g_pool && (g_pool_seen += (n + grain - 1) / grain) >= kHostRepaid) {
+        g_pool = new (std::nothrow) HostPool;
+        if (g_pool) g_pool_pid = getpid();
+      }
+      if (g_pool && g_pool->threads.size() < (size_t)kHostHelpers) {
+        try {
+          g_pool->threads.emplace_back([q = g_pool] { q->work(); });
+        } catch (...) {  // as many as the system gives
         }
       }
       p = g_pool;

@@ -19,17 +19,33 @@ std::string& error_text();
 // CF_OK when every field of `t` holds an allowed value, else CF_ERR_ARG with the reason.
 int check_tuning(const cf_tuning* t);
 
-// A few helper threads for the host side of large loads and readbacks: one core copies about
-// 10 GB/s between pinned and pageable memory, a fifth of what the DMA beside it moves (100k
-// particles' records, 4.4 MB: 0.45 ms of copying against 0.09).  The process has at most one
-// pool of kHostHelpers threads; it starts with the first large copy while an engine lives
-// and ends with the last engine.
+// A few helper threads for the host side of large loads and readbacks, whose copies between
+// pinned and pageable memory take longer than the DMA beside them.  The process has at most one
+// pool of kHostHelpers threads while an engine lives; it ends with the last engine.
+//
+// Measured as whole readbacks of particle records, repeated, by one thread and by four (ranges
+// of 128 KiB): 0.40 MB 40 -> 47 us, 0.53 MB 46 -> 50, 0.79 MB 56 -> 59, 1.1 MB 80 -> 66,
+// 2.2 MB 131 -> 108, 4.4 MB 244 -> 161, 22 MB 1150 -> 653.  Hence kHostAlone: up to 1 MiB waking
+// the threads costs more than they take over.
+// Starting and ending them has to be repaid too.  They start once larger jobs add up to
+// kHostRepaid, one with each job, and end while the last engine frees its memory: all at once in
+// the first copy, and waited for after the frees, a program that opens an engine, loads, steps
+// once, reads and ends got nothing from them (9k particles, 0.40 MB: 756 us, 741 without any
+// threads, 633 now; 25k: 1007, 990, 874; 100k, 4.4 MB: 1577, 1653, 1490).
 constexpr int kHostHelpers = 3;
+constexpr size_t kHostAlone = 8;    // ranges that the caller does by itself
+constexpr size_t kHostRepaid = 24;  // ranges of larger jobs (3 MiB) before the first thread
+struct HostPool;
 void host_pool_hold();  // an engine begins to live
-void host_pool_drop();  // and ends: the last one joins the threads
+// ... and ends: the last one is given the pool, whose threads it has told to end, and waits
+// for them with host_pool_end (null: nothing to wait for) when its own work is done.
+HostPool* host_pool_leave();
+void host_pool_end(HostPool* gone);
+void host_pool_drop();  // both at once
 // fn(begin, end) over disjoint ranges of at most `grain` items that cover [0, n), by the
-// caller and the helpers; returns when all are done.  Up to three ranges, another thread's call in progress, a
-// forked child, or no engine: the caller does everything itself.  fn must not throw.
+// caller and the helpers; returns when all are done.  Up to kHostAlone ranges, another thread's
+// call in progress, a forked child, or no engine: the caller does everything itself.  fn must
+// not throw.
 void host_parallel(size_t n, size_t grain, const std::function<void(size_t, size_t)>& fn);
 
 }  // namespace cf
