@@ -1103,6 +1103,20 @@ struct Engine {
     return true;
   }
 
+  // Event k of the sliced readbacks.  An event belongs to the device that is current when it
+  // is made and is recorded on that device's streams only, and the calling thread's device may
+  // be another than the engine's.
+  int slice_event(size_t k) {
+    if (slice_ev[k]) return CF_OK;
+    int now = 0;
+    HIPR(hipGetDevice(&now));
+    if (now != device) HIPR(hipSetDevice(device));
+    const hipError_t e = hipEventCreateWithFlags(&slice_ev[k], hipEventDisableTiming);
+    if (now != device) (void)hipSetDevice(now);
+    HIPR(e);
+    return CF_OK;
+  }
+
   // Device-to-host copy of `bytes` into the caller's memory through the pinned staging
   // buffer; synchronous.  The DMAs of all slices are queued at once; each slice is then
   // copied on by the host threads as it arrives, beside the DMA of the next ones.
@@ -1119,7 +1133,7 @@ struct Engine {
       HIPR(hipMemcpyAsync(hpin + at, (const char*)src + at, std::min(slice, bytes - at),
                           hipMemcpyDeviceToHost, st));
       if (at + slice >= bytes) break;  // the stream's end serves as the last slice's event
-      if (!slice_ev[k]) HIPR(hipEventCreateWithFlags(&slice_ev[k], hipEventDisableTiming));
+      CFR(slice_event(k));
       HIPR(hipEventRecord(slice_ev[k], st));
     }
     k = 0;

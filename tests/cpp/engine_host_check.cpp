@@ -27,6 +27,7 @@ struct Runtime {
   std::map<const char*, size_t> mem;            // live allocations
   std::vector<std::string> log;
   hipError_t last = hipSuccess;
+  int device = 0;                               // the current one, of two
   // the countdowns reach a failure at 0; negative: never
   int fail_malloc = -1, fail_copy = -1;
   size_t host_limit = ~size_t(0);               // larger pinned allocations fail
@@ -115,14 +116,17 @@ hipError_t hipLaunchKernel(const void* f, dim3, dim3, void**, size_t, hipStream_
 }
 
 hipError_t hipGetDeviceCount(int* n) {
-  *n = 1;
+  *n = 2;
   return hipSuccess;
 }
 hipError_t hipGetDevice(int* d) {
-  *d = 0;
+  *d = rt().device;
   return hipSuccess;
 }
-hipError_t hipSetDevice(int) { return hipSuccess; }
+hipError_t hipSetDevice(int d) {
+  rt().device = d;
+  return hipSuccess;
+}
 hipError_t hipGetLastError(void) {
   const hipError_t e = rt().last;
   rt().last = hipSuccess;
@@ -162,24 +166,31 @@ hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, hipMemcpyKind kind, 
   return hipSuccess;
 }
 
+// a stream and an event are known by the device they were made on
 hipError_t hipStreamCreateWithFlags(hipStream_t* s, unsigned) {
-  static int handle;
-  *s = (hipStream_t)&handle;
+  *s = (hipStream_t) new int(rt().device);
   return hipSuccess;
 }
-hipError_t hipStreamDestroy(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamDestroy(hipStream_t s) {
+  delete (int*)s;
+  return hipSuccess;
+}
 hipError_t hipStreamSynchronize(hipStream_t) {
   rt().log.push_back("sync");
   return hipSuccess;
 }
 hipError_t hipEventCreateWithFlags(hipEvent_t* e, unsigned) {
-  static int handle;
-  *e = (hipEvent_t)&handle;
+  *e = (hipEvent_t) new int(rt().device);
   return hipSuccess;
 }
-hipError_t hipEventRecord(hipEvent_t, hipStream_t) { return hipSuccess; }
+hipError_t hipEventRecord(hipEvent_t e, hipStream_t s) {
+  return result(*(int*)e == *(int*)s ? hipSuccess : hipErrorInvalidHandle);
+}
 hipError_t hipEventSynchronize(hipEvent_t) { return hipSuccess; }
-hipError_t hipEventDestroy(hipEvent_t) { return hipSuccess; }
+hipError_t hipEventDestroy(hipEvent_t e) {
+  delete (int*)e;
+  return hipSuccess;
+}
 
 }  // extern "C"
 
@@ -327,6 +338,21 @@ void colours() {
   HOLDS(logged("copy") == 2);
 }
 
+// An engine of one device read back by a thread whose current device is another.
+void other_device() {
+  OK(hipSetDevice(1));
+  Sim s(60000);  // two slices
+  std::vector<cf_particle> in(s.n), out(s.n);
+  for (int i = 0; i < s.n; ++i) in[i].pos[0] = (float)i;
+  OK(cf_set_particles(s.h, in.data(), s.n));
+  OK(hipSetDevice(0));
+  for (int k = 0; k < 2; ++k) {
+    OK(cf_get_particles(s.h, out.data(), s.n));
+    HOLDS(std::memcmp(in.data(), out.data(), in.size() * sizeof(cf_particle)) == 0);
+    HOLDS(rt().device == 0);
+  }
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -335,6 +361,7 @@ int main(int argc, char** argv) {
       {"changes_wait", changes_wait},
       {"pins_little", pins_little},
       {"colours", colours},
+      {"other_device", other_device},
   };
   const auto it = argc == 2 ? cases.find(argv[1]) : cases.end();
   if (it == cases.end()) die("usage: engine_host_check CASE");

@@ -45,3 +45,7 @@ def test_copies_without_pinned_memory(check):
 
 def test_colours_after_a_failed_upload(check):
     check("colours")
+
+
+def test_readback_with_another_device_current(check):
+    check("other_device")
