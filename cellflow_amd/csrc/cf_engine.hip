@@ -1739,17 +1739,24 @@ struct Engine {
       return lay_adj(base, n, (nsteps + every - 1) / every, every, bins, T, rows, stride);
     };
     long every = std::min(*ckpt, std::max(nsteps, 1L));
-    if (every < nsteps) {
+    // (a layout lists every buffer on the host, so one that cannot fit is not made: a kept
+    // state alone takes its pos, vel and new velocities, and x64 and v64)
+    const size_t state_bytes = (size_t)P * (3 * sizeof(float4) + 2 * sizeof(double4));
+    if (every < nsteps && (size_t)nsteps <= kKeepBytes / state_bytes) {
       const size_t asked = lay(nullptr, every), all = lay(nullptr, nsteps);
       size_t avail = 0, total = 0;
-      if (all <= kKeepBytes && all <= kKeepTimes * asked && hipMemGetInfo(&avail, &total) == hipSuccess && all <= avail / 8)
-        every = nsteps;
+      if (hipMemGetInfo(&avail, &total) != hipSuccess) {
+        (void)hipGetLastError();
+        avail = 0;
+      }
+      if (all <= kKeepBytes && all <= kKeepTimes * asked && all <= avail / 8) every = nsteps;
     }
     size_t bytes = lay(nullptr, every);
     if (hipMalloc((void**)&adj.arena, bytes) != hipSuccess) {
       (void)hipGetLastError();
       adj.arena = nullptr;
-      if (every <= *ckpt) return fail(CF_ERR_DEVICE, "%zu bytes of gradient buffers: out of device memory", bytes);
+      if (every <= *ckpt)
+        return fail(CF_ERR_DEVICE, "%zu bytes of gradient buffers: out of device memory", bytes);
       every = *ckpt;
       bytes = lay(nullptr, every);
       CFR(dalloc(&adj.arena, bytes));

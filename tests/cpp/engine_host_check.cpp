@@ -7,6 +7,8 @@
 //   engine_host_check CASE   exits 0 when the case holds
 #include <hip/hip_runtime_api.h>
 
+#include <sys/resource.h>
+
 #include <cstdarg>
 #include <cstdio>
 #include <cstdlib>
@@ -30,6 +32,7 @@ struct Runtime {
   int device = 0;                               // the current one, of two
   // the countdowns reach a failure at 0; negative: never
   int fail_malloc = -1, fail_copy = -1;
+  bool fail_info = false;                       // hipMemGetInfo fails
   size_t host_limit = ~size_t(0);               // larger pinned allocations fail
   uint32_t edges = 0;                           // the graph's size in the status words read back
   dim3 grid, block;
@@ -134,6 +137,7 @@ hipError_t hipGetLastError(void) {
 }
 hipError_t hipGetSymbolAddress(void** p, const void*) { return allocate(p, 64); }
 hipError_t hipMemGetInfo(size_t* avail, size_t* total) {
+  if (rt().fail_info) return result(hipErrorInvalidValue);
   *avail = *total = size_t(256) << 30;
   return hipSuccess;
 }
@@ -353,6 +357,26 @@ void other_device() {
   }
 }
 
+// A gradient of more steps than could ever all be kept costs the host no memory to find out
+// (its checkpoints fit), and a runtime that cannot tell the free memory fails no call.
+void long_rollout() {
+  cf_params p = params(0.1f, 2.0f);
+  double target[4] = {1, 1, 1, 1}, loss = 0, table[4], ratio = 0;
+  const rlimit limit{size_t(8) << 30, size_t(8) << 30};
+  HOLDS(setrlimit(RLIMIT_AS, &limit) == 0);
+  for (const int steps : {1000000000, 100000000}) {
+    Sim s(64);
+    OK(cf_simulate(s.h, &p, 1, nullptr));
+    rt().fail_malloc = 0;  // before a step is run
+    HOLDS(cf_rollout_grad(s.h, &p, steps, 1000, 4, 0.1f, target, &loss, nullptr, table, &ratio) ==
+          CF_ERR_DEVICE);
+    HOLDS(rt().fail_malloc < 0);
+  }
+  Sim s(64);
+  rt().fail_info = true;
+  OK(cf_rollout_grad(s.h, &p, 20, 5, 4, 0.1f, target, &loss, nullptr, table, &ratio));
+}
+
 }  // namespace
 
 int main(int argc, char** argv) {
@@ -362,6 +386,7 @@ int main(int argc, char** argv) {
       {"pins_little", pins_little},
       {"colours", colours},
       {"other_device", other_device},
+      {"long_rollout", long_rollout},
   };
   const auto it = argc == 2 ? cases.find(argv[1]) : cases.end();
   if (it == cases.end()) die("usage: engine_host_check CASE");

@@ -49,3 +49,7 @@ def test_colours_after_a_failed_upload(check):
 
 def test_readback_with_another_device_current(check):
     check("other_device")
+
+
+def test_long_rollout_needs_no_host_memory(check):
+    check("long_rollout")
