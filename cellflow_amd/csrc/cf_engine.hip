@@ -826,7 +826,6 @@ struct Engine {
     ta.src_vel = b.tvel;
     ta.src_id = b.id[A];
     ta.key = b.key;
-    ta.hist = b.hist;
     ta.start_old = b.start[A];
     ta.start_new = b.start[B];
     ta.dst_pos = b.pos[B];

@@ -33,8 +33,9 @@ constexpr int kTileBlocks = 390;
 constexpr int kTileMin = 192;
 constexpr int kTileMax = 768;
 constexpr int kEdgeTile = 1024;        // owner ids per edge tile
-// The list force kernels (variants 3 and 4) keep each candidate as slot | image-shift code
-// << kCodeShift in LDS, so they take at most 2^kCodeShift slots.
+// The force kernels with candidate lists (variants 3 and 4, and variant 0 at 16 lanes) keep each
+// candidate as slot | image-shift code << kCodeShift in LDS, so they take at most 2^kCodeShift
+// slots.  Beyond, variants 3 and 4 are refused and variant 0 runs without lists.
 constexpr int kCodeShift = 26;
 constexpr uint32_t kFarBit = 0x80000000u;
 // Tile counters sit one per 128-byte line: a line takes every atomic of the tiles it holds,
@@ -242,7 +243,6 @@ struct TileSortArgs {
   const float4* __restrict__ src_vel;
   const uint32_t* __restrict__ src_id;
   const uint32_t* __restrict__ key;     // new cell (| kFarBit) by pre-step slot
-  uint32_t* hist;                       // per-cell counts (read, then cleared)
   const uint32_t* __restrict__ start_old;
   uint32_t* start_new;
   float4* dst_pos;

@@ -2504,7 +2504,8 @@ __device__ uint32_t lookback_wait(unsigned long long* flags, int g, int first, u
 }
 
 // Sums of `v` and `u` over the block, and the exclusive scan of `w` in thread order with
-// its total, behind one pair of barriers.  `red` holds 12 words.
+// its total, behind one pair of barriers.  `red` holds three words per wave of the block,
+// 3 * kSortThreads / kWave.
 __device__ __forceinline__ void block_sums_excl_u32(uint32_t v, uint32_t u, uint32_t w,
                                                     uint32_t* red, uint32_t& vsum,
                                                     uint32_t& usum, uint32_t& wpre,
@@ -2539,8 +2540,8 @@ __device__ __forceinline__ void block_sums_excl_u32(uint32_t v, uint32_t u, uint
 // An edge tile's owners' edges.  The block draws a ticket (its edge tile, in the order the
 // edge-tile blocks started), sums its owners' counts and finds the tile's place in the list
 // by a decoupled look-back over the tiles before it; then it writes the tile's edges
-// e = tid, tid + 256, ...: each finds its owner in LDS (the last thread whose first edge is
-// at or before e, then that thread's owners in order) and its rank k = e - the owner's
+// e = tid, tid + kSortThreads, ...: each finds its owner in LDS (the last thread whose first
+// edge is at or before e, then that thread's owners in order) and its rank k = e - the owner's
 // first edge, so a thread's staged-partner loads are all in flight together and the stores
 // are contiguous.  `toff`, `p0s` (kSortThreads words) and `ecs` (kEdgeTile words) are LDS
 // scratch.
@@ -2601,7 +2602,7 @@ __device__ void edge_tile(const TileSortArgs& a, uint32_t* red, uint32_t* toff, 
       own[b] = 0;
       ob[b] = 0u;
       if (e < total) {
-        int t = 0;  // toff[0] = 0 <= e; the steps reach at most index 255
+        int t = 0;  // toff[0] = 0 <= e; the steps reach at most index kSortThreads - 1
 #pragma unroll
         for (int st = kSortThreads / 2; st > 0; st >>= 1)
           if (toff[t + st] <= e) t += st;
