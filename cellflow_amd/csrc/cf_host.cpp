@@ -39,7 +39,8 @@ int fail(int code, const char* fmt, ...) {
 struct HostPool {
   std::mutex mu;
   std::condition_variable wake, done;
-  std::vector<std::thread> threads;
+  std::thread first;
+  std::vector<std::thread> rest;  // the first thread's until it ends
   const std::function<void(size_t, size_t)>* fn = nullptr;  // the job, null between jobs
   size_t n = 0, grain = 0;
   std::atomic<size_t> next{0};
@@ -50,6 +51,15 @@ struct HostPool {
   void take(const std::function<void(size_t, size_t)>& f, size_t count, size_t step) {
     for (size_t i = next.fetch_add(step); i < count; i = next.fetch_add(step))
       f(i, std::min(count, i + step));
+  }
+
+  // The first thread starts the others, so that the job it was started for waits for one.
+  void lead() {
+    try {
+      while ((int)rest.size() + 1 < kHostHelpers) rest.emplace_back([this] { work(); });
+    } catch (...) {  // as many as the system gives
+    }
+    work();
   }
 
   void work() {
@@ -73,11 +83,10 @@ struct HostPool {
 
 namespace {
 
-std::mutex g_pool_mu;  // guards the four below
+std::mutex g_pool_mu;  // guards the three below
 std::mutex g_run_mu;   // one job at a time
 HostPool* g_pool = nullptr;
 int g_pool_users = 0;
-size_t g_pool_seen = 0;  // ranges of the larger jobs before there was a pool
 std::atomic<pid_t> g_pool_pid{0};  // the process the threads live in
 
 }  // namespace
@@ -96,7 +105,6 @@ HostPool* host_pool_leave() {
     if (--g_pool_users == 0) {
       gone = g_pool;
       g_pool = nullptr;
-      g_pool_seen = 0;
       g_pool_pid = 0;
     }
   }
@@ -111,7 +119,8 @@ HostPool* host_pool_leave() {
 
 void host_pool_end(HostPool* gone) {
   if (!gone) return;
-  for (std::thread& t : gone->threads) t.join();
+  if (gone->first.joinable()) gone->first.join();
+  for (std::thread& t : gone->rest) t.join();
   delete gone;
 }
 
@@ -129,14 +138,14 @@ void host_parallel(size_t n, size_t grain, const std::function<void(size_t, size
   {
     std::unique_lock<std::mutex> l(g_pool_mu, std::try_to_lock);
     if (l && g_pool_users > 0) {
-      if (!g_pool && (g_pool_seen += (n + grain - 1) / grain) >= kHostRepaid) {
+      if (!g_pool) {
         g_pool = new (std::nothrow) HostPool;
-        if (g_pool) g_pool_pid = getpid();
-      }
-      if (g_pool && g_pool->threads.size() < (size_t)kHostHelpers) {
-        try {
-          g_pool->threads.emplace_back([q = g_pool] { q->work(); });
-        } catch (...) {  // as many as the system gives
+        if (g_pool) {
+          g_pool_pid = getpid();
+          try {
+            g_pool->first = std::thread([q = g_pool] { q->lead(); });
+          } catch (...) {  // none to be had: the callers do everything
+          }
         }
       }
       p = g_pool;

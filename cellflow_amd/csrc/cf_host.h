@@ -24,17 +24,18 @@ int check_tuning(const cf_tuning* t);
 // pool of kHostHelpers threads while an engine lives; it ends with the last engine.
 //
 // Measured as whole readbacks of particle records, repeated, by one thread and by four (ranges
-// of 128 KiB): 0.40 MB 40 -> 47 us, 0.53 MB 46 -> 50, 0.79 MB 56 -> 59, 1.1 MB 80 -> 66,
-// 2.2 MB 131 -> 108, 4.4 MB 244 -> 161, 22 MB 1150 -> 653.  Hence kHostAlone: up to 1 MiB waking
-// the threads costs more than they take over.
-// Starting and ending them has to be repaid too.  They start once larger jobs add up to
-// kHostRepaid, one with each job, and end while the last engine frees its memory: all at once in
-// the first copy, and waited for after the frees, a program that opens an engine, loads, steps
-// once, reads and ends got nothing from them (9k particles, 0.40 MB: 756 us, 741 without any
-// threads, 633 now; 25k: 1007, 990, 874; 100k, 4.4 MB: 1577, 1653, 1490).
+// of 128 KiB): 0.40 MB 42 -> 47 us, 0.53 MB 46 -> 50, 0.79 MB 56 -> 59, 1.1 MB 82 -> 67,
+// 2.2 MB 136 -> 108, 4.4 MB 245 -> 162, 22 MB 1150 -> 653; and of the copies alone into memory
+// that was never touched: 0.4 MB 60 -> 40, 1.0 MB 158 -> 93, 4.4 MB 962 -> 398.  Hence kHostAlone:
+// up to 768 KiB waking the threads costs a repeated copy more than they take over.
+// The threads begin with the first larger job, which starts one that starts the others, and end
+// while the last engine frees its memory.  Started by the job and joined after the frees, they
+// made a program that opens an engine, loads, steps once, reads and ends slower (1.1 MB of
+// records: 976 us, 876 without threads; now 994 against 1021 and 1007 on another machine; 0.40 MB:
+// 795, 769 without, 682 now).  Started only once jobs add up to 3 MiB, they came late for the
+// first pass over new buffers (14 MB of vertices and edges: 2960 -> 3150 us, 4700 without).
 constexpr int kHostHelpers = 3;
-constexpr size_t kHostAlone = 8;    // ranges that the caller does by itself
-constexpr size_t kHostRepaid = 24;  // ranges of larger jobs (3 MiB) before the first thread
+constexpr size_t kHostAlone = 6;  // ranges that the caller does by itself
 struct HostPool;
 void host_pool_hold();  // an engine begins to live
 // ... and ends: the last one is given the pool, whose threads it has told to end, and waits

@@ -1,10 +1,8 @@
-// When host_parallel's threads (cf_host.cpp) exist: never for small jobs, not before the larger
-// ones add up to kHostRepaid ranges, then one more with each up to kHostHelpers, until the last
-// holder is gone.  Exits 0 when all hold.
+// When host_parallel's threads (cf_host.cpp) exist: never for small jobs, kHostHelpers from the
+// first larger one on until the last holder is gone.  Exits 0 when all hold.
 #include <dirent.h>
 #include <unistd.h>
 
-#include <algorithm>
 #include <atomic>
 #include <cstdio>
 
@@ -42,17 +40,14 @@ int main() {
     cf::host_pool_hold();
     for (int k = 0; k < 1000; ++k)
       if (!job(small)) return 2;
-    for (size_t seen = cf::kHostAlone + 1; seen < cf::kHostRepaid; seen += cf::kHostAlone + 1)
-      if (!job(small + 1)) return 2;
     if (!extra(0)) return 3;
-    const int jobs = cycle == 0 ? 1 : 2 + cf::kHostHelpers;
-    for (int k = 1; k <= jobs; ++k) {
-      if (!job(k == 1 ? small + 1 : 100000)) return 4;
-      if (!extra(std::min(k, cf::kHostHelpers))) return 5;
+    for (int k = 0; k < (cycle == 0 ? 1 : 20); ++k) {
+      if (!job(k == 0 ? small + 1 : 100000)) return 4;
+      if (cycle < 2 && !extra(cf::kHostHelpers)) return 5;  // later: without a pause
     }
     cf::host_pool_hold();  // they belong to the process, not to one holder
     cf::host_pool_drop();
-    if (!extra(std::min(jobs, cf::kHostHelpers))) return 6;
+    if (cycle < 3 && !extra(cf::kHostHelpers)) return 6;
     if (cycle % 2) {
       cf::host_pool_drop();
     } else {  // a holder that begins while the last one's threads end has its own
@@ -60,7 +55,7 @@ int main() {
       cf::host_pool_hold();
       if (!ending || !job(100000)) return 7;
       cf::host_pool_end(ending);
-      if (!extra(1)) return 8;
+      if (!extra(cf::kHostHelpers)) return 8;
       if (cf::HostPool* last = cf::host_pool_leave()) cf::host_pool_end(last);
     }
     if (!extra(0)) return 9;

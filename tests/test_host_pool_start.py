@@ -10,7 +10,7 @@ import pytest
 ROOT = os.path.dirname(os.path.dirname(os.path.abspath(__file__)))
 
 
-def test_threads_start_one_by_one(tmp_path):
+def test_threads_start_with_the_first_large_job(tmp_path):
     if not shutil.which("g++"):
         pytest.skip("no g++")
     exe = str(tmp_path / "pool_start_check")
