@@ -33,7 +33,7 @@ int check_tuning(const cf_tuning* t);
 // made a program that opens an engine, loads, steps once, reads and ends slower (1.1 MB of
 // records: 976 us, 876 without threads; now 994 against 1021 and 1007 on another machine; 0.40 MB:
 // 795, 769 without, 682 now).  Started only once jobs add up to 3 MiB, they came late for the
-// first pass over new buffers (14 MB of vertices and edges: 2960 -> 3150 us, 4700 without).
+// first pass over new buffers (7.8 MB of vertices and edges: 2960 -> 3150 us, 4700 without).
 constexpr int kHostHelpers = 3;
 constexpr size_t kHostAlone = 6;  // ranges that the caller does by itself
 struct HostPool;
