@@ -5,6 +5,7 @@
 
 #include <atomic>
 #include <cstdio>
+#include <thread>
 
 #include "../../cellflow_amd/csrc/cf_host.h"
 
@@ -33,6 +34,8 @@ static bool job(size_t items) {
 }
 
 int main() {
+  std::thread([] {}).join();  // a sanitizer's own thread comes with the first
+  usleep(10000);
   began = threads();
   const size_t small = cf::kHostAlone * 100;
   for (int cycle = 0; cycle < 4; ++cycle) {
